@@ -549,11 +549,11 @@ __global__ __launch_bounds__(256) void view_pixel_areas(const float* view, int W
 //
 // Work split.  Near the shadow a pixel can project onto a large part of the
 // sky with tens of thousands of candidates; one lane would serialise them and
-// stall its wavefront.  star_map_light takes pixels with at most kLightStars
-// candidates (about 92% of the pixels of a lensed frame, 6% of the
-// candidates), one lane each, and queues the others for star_map_wave, where
-// one wavefront splits a pixel's candidates and reduces the taps in a fixed
-// order.
+// stall its wavefront.  star_scan finds the pixels with at most kLightStars
+// candidates and a star inside (5% of the pixels of a lensed 1080p frame;
+// star_few traces them, one lane each), and queues those with more (6%),
+// whose candidates star_map_chunk splits over wavefronts, the taps reduced in
+// a fixed order.
 //
 // Per tap the reference evaluates 100 * 10^(-0.4 (m - 2.5 log10 x)) with
 // x = frac * gaussian(d) and converts HSP -> RGB at brightness P * that.
@@ -625,27 +625,21 @@ __device__ void star_pixel_geom(const float* thphi, int W, int i, int j, float o
     P.sgn = orient < 0 ? -1 : 1;
 }
 
+// Lensing factor and redshift of the pixel whose corners P holds.
+__device__ __forceinline__ void star_lens(int W, size_t ij, int ind, int lr, const float* area, const float* view,
+                                          const Cam7& cam, StarPix& P) {
+    P.redshft = 1.f;
+    P.frac = 1.f;
+    if (lr) lensing_redshift(P.t, P.p, W, ind, cam, view, P.frac, P.redshft, area[ij]);
+    P.red = 4.f * log10f(P.redshft);   // device library FP32 (a few ulps)
+}
+
 __device__ bool star_pixel(const float* thphi, const uint8_t* bh, int W, int i, int j, float offset, int lr,
                            const float* area, const float* view, const Cam7& cam, StarPix& P) {
     const size_t ij = (size_t)i * W + j;
     if (bh[ij] != 0) return false;
-    P.colours = cam.colours;
-    const int ind = i * (W + 1) + j;
-    P.picheck = false;
-    corners(thphi, W, ind, P.t, P.p, P.picheck, offset);
-    const float* t = P.t;
-    const float* p = P.p;
-    P.mx[0] = fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]));
-    P.mx[1] = fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3]));
-    P.mn[0] = fminf(fminf(t[0], t[1]), fminf(t[2], t[3]));
-    P.mn[1] = fminf(fminf(p[0], p[1]), fminf(p[2], p[3]));
-    float orient = (t[1] - t[0]) * (p[1] + p[0]) + (t[2] - t[1]) * (p[2] + p[1]) + (t[3] - t[2]) * (p[3] + p[2]) +
-                   (t[0] - t[3]) * (p[0] + p[3]);
-    P.sgn = orient < 0 ? -1 : 1;
-    P.redshft = 1.f;
-    P.frac = 1.f;
-    if (lr) lensing_redshift(t, p, W, ind, cam, view, P.frac, P.redshft, area[ij]);
-    P.red = 4.f * log10f(P.redshft);   // device library FP32 (a few ulps)
+    star_pixel_geom(thphi, W, i, j, offset, cam, P);
+    star_lens(W, ij, i * (W + 1) + j, lr, area, view, cam, P);
     return true;
 }
 
@@ -655,11 +649,12 @@ __device__ __forceinline__ void node_range(const int32_t* tree, int node, int& b
 }
 
 // searchTree (MakeImageKernel.cu:27-96) with picheck = 0: visit(node) is
-// called for every listed node in the reference's list order.
+// called for every listed node in the reference's list order.  The node's
+// rectangle is held in scalars (0: theta, 1: phi), not in arrays indexed by
+// the level's axis, which would live in scratch memory.
 template <class F>
 __device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn, const float* mx, F&& visit) {
-    float nodeStart[2] = {0.f, 0.f};
-    float nodeSize[2] = {BT_FPI, BT_FPI2};
+    float start0 = 0.f, start1 = 0.f, size0 = BT_FPI, size1 = BT_FPI2;
     int node = 0;
     unsigned bitMask = 1u << treeLevel;
     int level = 0;
@@ -669,20 +664,25 @@ __device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn,
         for (lvl = level + 1; lvl <= treeLevel; lvl++) {
             int star_n = tree[node];
             if (node != 0 && ((node + 1) & node) != 0) star_n -= tree[node - 1];
-            int tp = lvl & 1;
-            float x_overlap = fmaxf(0.f, fminf(mx[0], nodeStart[0] + nodeSize[0]) - fmaxf(mn[0], nodeStart[0]));
-            float y_overlap = fmaxf(0.f, fminf(mx[1], nodeStart[1] + nodeSize[1]) - fmaxf(mn[1], nodeStart[1]));
-            float overlapArea = x_overlap * y_overlap;
-            bool size = overlapArea / (nodeSize[0] * nodeSize[1]) > 0.8f;
-            nodeSize[tp] = nodeSize[tp] * .5f;
+            const bool ph = (lvl & 1) != 0;
+            const float full0 = size0, full1 = size1;
+            if (ph) size1 = size1 * .5f;
+            else size0 = size0 * .5f;
             if (star_n == 0) {
                 node = node * 2 + 1;
                 break;
             }
-            float check = nodeStart[tp] + nodeSize[tp];
-            bool lu = mn[tp] < check;
-            bool rd = mx[tp] >= check;
-            if (lvl == treeLevel || (rd && lu && size)) {
+            float check = ph ? start1 + size1 : start0 + size0;
+            bool lu = (ph ? mn[1] : mn[0]) < check;
+            bool rd = (ph ? mx[1] : mx[0]) >= check;
+            bool list = lvl == treeLevel;
+            if (!list && rd && lu) {   // the quad covers most of the node
+                float x_overlap = fmaxf(0.f, fminf(mx[0], start0 + full0) - fmaxf(mn[0], start0));
+                float y_overlap = fmaxf(0.f, fminf(mx[1], start1 + full1) - fmaxf(mn[1], start1));
+                float overlapArea = x_overlap * y_overlap;
+                list = overlapArea / (full0 * full1) > 0.8f;
+            }
+            if (list) {
                 if (rd) visit(node * 2 + 2);
                 if (lu) visit(node * 2 + 1);
                 node = node * 2 + 1;
@@ -697,14 +697,18 @@ __device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn,
         if (level >= 0) {
             int diff = lvl - level;
             for (int q = 0; q < diff; q++) {
-                int tp = (lvl - q) & 1;
-                if (!(node & 1)) nodeStart[tp] -= nodeSize[tp];
-                nodeSize[tp] = nodeSize[tp] * 2.f;
+                if ((lvl - q) & 1) {
+                    if (!(node & 1)) start1 -= size1;
+                    size1 = size1 * 2.f;
+                } else {
+                    if (!(node & 1)) start0 -= size0;
+                    size0 = size0 * 2.f;
+                }
                 node = (node - 1) / 2;
             }
             node++;
-            int tp = level & 1;
-            nodeStart[tp] += nodeSize[tp];
+            if (level & 1) start1 += size1;
+            else start0 += size0;
         }
     }
 }
@@ -750,6 +754,19 @@ __device__ __forceinline__ void row_span(const StarPix& P, int r, int p0, int p1
     q1 = min(p1, bin_of(hi, kBinDP, kBinP) + 1);
 }
 
+// The candidates [b, e) of bin row r (none beyond row r1).
+__device__ __forceinline__ void row_bounds(const StarPix& P, const SceneK& s, int r, int r1, int p0, int p1, int& b,
+                                           int& e) {
+    b = e = 0;
+    if (r > r1) return;
+    int q0, q1;
+    row_span(P, r, p0, p1, q0, q1);
+    if (q0 <= q1) {
+        b = s.bin_start[r * kBinP + q0];
+        e = s.bin_start[r * kBinP + q1 + 1];
+    }
+}
+
 // f(begin, end) for every candidate range of a pixel; ranges index
 // ranges_pos/ranges_mag (tree order for picheck pixels, bin order otherwise).
 template <class F>
@@ -763,10 +780,14 @@ __device__ void for_ranges(const StarPix& P, const SceneK& s, F&& f) {
     } else {
         const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
         const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
-        for (int r = r0; r <= r1; r++) {
-            int q0, q1;
-            row_span(P, r, p0, p1, q0, q1);
-            if (q0 <= q1) f(s.bin_start[r * kBinP + q0], s.bin_start[r * kBinP + q1 + 1]);
+        // four rows' bounds load together
+        for (int r = r0; r <= r1; r += 4) {
+            int b[4], e[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) row_bounds(P, s, r + k, r1, p0, p1, b[k], e[k]);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (b[k] < e[k]) f(b[k], e[k]);
         }
     }
 }
@@ -806,6 +827,21 @@ __device__ __forceinline__ bool star_pixel_odd(const StarPix& P, const SceneK& s
     return !(s.mag_tame && P.frac >= 1e-30f && P.frac <= 1e30f && P.red >= -80.f && P.red <= 80.f);
 }
 
+// The reference's own expression for one tap (kernel.cuh:390,
+// MakeImageKernel.cu:310-318).  Out of line: its FP64 log and pow inlined in
+// every tap make the odd kernels larger than the instruction cache, and they
+// then wait for their own code (the odd chunks of a 320x180 frame took 250 us).
+struct Rgb {
+    float r, g, b;
+};
+__device__ __attribute__((noinline)) Rgb star_tap_slow(float part, float x, float hh, float ss, float pp) {
+    const float appMag = part - 2.5f * f_log10(x);
+    const float brightness = 100 * f_exp10(-.4f * appMag);
+    Rgb o;
+    hsp_to_rgb(hh, ss, pp * brightness, o.r, o.g, o.b);
+    return o;
+}
+
 // The light of one star inside the pixel (MakeImageKernel.cu:293-322).
 // Per tap the reference evaluates 100 * 10^(-0.4 (part - 2.5 log10 x)) with
 // x = frac * gaussian(d); for finite x > 0 and finite E = 10^(-0.4 part)
@@ -828,6 +864,12 @@ __device__ __forceinline__ void star_splat(const StarPix& P, const float* mag, i
     const float r1 = col[3], g1 = col[4], b1 = col[5];
     const float E = ODD ? f_exp10(-.4f * part) : exp10_f32(-.4f * part);
     const float maxDistSq = (STEP + .5f) * (STEP + .5f);
+    // A lensing factor that is no positive finite number makes every tap's x
+    // the same infinity, zero or (log of a negative) NaN: one slow evaluation
+    // serves them all.
+    const bool flat = ODD && !(P.frac > 0.f && P.frac <= 3.4e38f);
+    Rgb all{0.f, 0.f, 0.f};
+    if (flat) all = star_tap_slow(part, P.frac, col[0], col[1], col[2]);
 #pragma unroll
     for (int u = 0; u < FW; u++)
 #pragma unroll
@@ -844,9 +886,10 @@ __device__ __forceinline__ void star_splat(const StarPix& P, const float* mag, i
                 gg = g1 * bright;
                 bb = b1 * bright;
             } else {
-                float appMag = part - 2.5f * f_log10(x);
-                float brightness = 100 * f_exp10(-.4f * appMag);
-                hsp_to_rgb(col[0], col[1], col[2] * brightness, rr, gg, bb);
+                const Rgb o = flat ? all : star_tap_slow(part, x, col[0], col[1], col[2]);
+                rr = o.r;
+                gg = o.g;
+                bb = o.b;
             }
             rr *= 255.f;
             gg *= 255.f;
@@ -867,8 +910,8 @@ __device__ __forceinline__ void star_accumulate(const StarPix& P, const float* p
 
 // Pixels with more than kLightStars candidates are queued with their
 // candidate count and cut into chunks of kChunk candidates, one wavefront
-// per chunk; their chunk indices are taken by an atomic when the pixel is
-// queued (contiguous per pixel).  A pixel's chunk partials are summed in
+// per chunk; their chunk indices are taken by an atomic in star_assign
+// (contiguous per pixel).  A pixel's chunk partials are summed in
 // chunk order, so the result does not depend on which waves ran which
 // chunks.  Every queued star is then
 // one of a few candidates of one lane, whatever the pixel it lands in: the
@@ -877,10 +920,9 @@ __device__ __forceinline__ void star_accumulate(const StarPix& P, const float* p
 constexpr int kChunk = 256;
 
 // A queued count with this bit set is a pixel whose candidates come from
-// the star tree (a quad across phi = 2 pi).  The tree is walked once for
-// such a pixel (star_tree_ranges) and its listed node ranges are stored, so
-// that every chunk of the pixel walks the stored ranges as a binned pixel
-// walks its bin rows.
+// the star tree (a quad across phi = 2 pi).  star_wide walks the tree for
+// such a pixel and stores its listed node ranges, so that every chunk of the
+// pixel walks the stored ranges as a binned pixel walks its bin rows.
 constexpr uint32_t kTreePixel = 0x80000000u;
 // A queued count with this bit set is an odd pixel (star_pixel_odd): its
 // chunks are traced by the ODD instance of star_map_chunk.
@@ -896,7 +938,7 @@ constexpr uint32_t kNoOwner = 0xffffffffu;
 
 struct StarQueue {
     uint32_t* pix;         // queued pixel indices
-    uint32_t* cnt;         // their candidate counts (| kTreePixel)
+    uint32_t* cnt;         // their candidate counts (| kTreePixel | kOddPixel); 0: no chunk work
     uint32_t* nnode;       // tree pixels: listed node count
     uint32_t* rbase;       // tree pixels: first stored range
     int2* ranges;          // stored node ranges (begin, end) of tree pixels
@@ -904,17 +946,26 @@ struct StarQueue {
     uint32_t* cstart;      // first chunk of each queued pixel
     uint32_t* owner;       // queued pixel of each chunk (or kNoOwner)
     float* lens;           // per queued pixel: frac, redshift, 4 log10(redshift)
+    uint32_t* wide;        // queue entries that star_wide counts: binned ones from the front, tree ones from the back
     uint32_t* odd;         // pixels for star_map_odd
-    unsigned* ctr;         // [0] queued pixels, [1] chunk indices taken, [2] odd pixels, [3] stored ranges
+    unsigned* ctr;         // the counters below, each on a line of its own
     float* partial;        // per chunk: FW*FW*3 partial taps
     unsigned cap;          // chunk capacity of `partial`
-    uint8_t* lit;          // per pixel: 1 when its taps are written this frame (0: all its taps are zero)
+    uint8_t* lit;          // per pixel: kDark, or who writes its taps this frame
 };
+// StarQueue::ctr, in words: queued pixels, chunk indices taken, odd pixels,
+// stored ranges, wide entries, tree entries.
+constexpr int kCtrQueued = 0, kCtrChunks = 32, kCtrOdd = 64, kCtrRanges = 96, kCtrWide = 128, kCtrTree = 160;
+constexpr int kStarCtrWords = 192;
+// Pixel classes: no star inside (all taps zero, none stored), taps written by
+// star_few / star_map_odd, taps written from the chunks.
+constexpr uint8_t kDark = 0, kFew = 1, kQueued = 2;
 
 // All candidates of a pixel in order, into acc (the reference's loop),
-// kLightStars at a time: the window's candidate indices are collected into
-// this thread's LDS slots `cand`, then traced, so that the kernel holds one
-// copy of the splat whichever of the tree or the bins lists the candidates.
+// kLightStars at a time: those of the window that lie inside are collected
+// into this thread's LDS slots `cand`, then traced, so that a wave runs the
+// splat as often as its fullest pixel has stars inside, and the kernel holds
+// one copy of it whichever of the tree or the bins lists the candidates.
 template <int STEP, bool ODD>
 __device__ __forceinline__ void star_seq(const StarPix& P, const SceneK& s, int count, int* cand,
                                          float (&acc)[(2 * STEP + 1) * (2 * STEP + 1)][3]) {
@@ -926,7 +977,10 @@ __device__ __forceinline__ void star_seq(const StarPix& P, const SceneK& s, int 
             const int len = e - b;
             if (g + len > w && g < w + kLightStars) {
                 const int q0 = b + max(0, w - g), q1 = b + min(len, w + kLightStars - g);
-                for (int q = q0; q < q1; q++) cand[nq++] = q;
+                for (int q = q0; q < q1; q++) {
+                    float st, sp;
+                    if (star_test(P, pos, q, st, sp)) cand[nq++] = q;
+                }
             }
             g += len;
         });
@@ -946,95 +1000,309 @@ __device__ __forceinline__ void store_taps(float* taps, size_t NP, size_t ij,
     }
 }
 
-template <int STEP>
-__global__ __launch_bounds__(256) void star_map_light(const float* thphi, const uint8_t* bh, SceneK s, Cam7 cam,
-                                                      int W, int H, float offset, int lr, const float* area,
-                                                      const float* view, float* taps, StarQueue Q) {
-    constexpr int FW = 2 * STEP + 1;
-    __shared__ int s_cand[256][kLightStars];
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = blockIdx.y * blockDim.y + threadIdx.y;
-    // every lane stays to the end: the queue append below scans over the wave
-    const bool valid = i < H && j < W;
-    const size_t NP = (size_t)W * H;
-    const size_t ij = valid ? (size_t)i * W + j : 0;
-    float acc[FW * FW][3];
-#pragma unroll
-    for (int u = 0; u < FW * FW; u++) acc[u][0] = acc[u][1] = acc[u][2] = 0.f;
-    StarPix P;
-    int count = 0, nodes = 0;
-    bool odd = false;
-    if (valid && star_pixel(thphi, bh, W, i, j, offset, lr, area, view, cam, P)) {
-        for_ranges(P, s, [&](int b, int e) {
-            count += e - b;
-            nodes++;
-        });
-        odd = count > 0 && star_pixel_odd(P, s);
-    }
-    // pixels of many candidates go to the chunks; odd pixels of few to
-    // star_map_odd
-    const bool queue = count > kLightStars;
-    bool to_odd = odd && !queue;
-    bool self = valid && !queue && !odd;   // this lane writes the pixel's taps
-    bool seq = self && count > 0;          // ... after tracing its candidates
-    // wave-aggregated append of (pixel, count) and of the pixel's chunks
+// Bin rows a lane of star_scan walks itself; taller quads go to star_wide.
+constexpr int kScanRows = 4;
+// Tiles of 16 x 16 pixels side by side per workgroup of star_scan, at most.
+// One in small frames (at 320 x 180 four leave three quarters of the SIMDs
+// without a wave: 37 us against 16), kScanTiles from a million pixels on.
+constexpr int kScanTiles = 4;
+
+// Sorts the pixels by how much star work they hold: none (most of a frame),
+// few candidates with a star inside (kFew), or more than kLightStars
+// candidates (kQueued, cut into chunks).  Geometry and inside tests only: the
+// lensing's FP64 trigonometry and the splats, which a few percent of the
+// pixels need, run on full waves in the kernels below instead of on a few
+// lanes of every wave here.  The 2 x kScanRows bin bounds of a pixel load
+// together.  Quads taller than kScanRows bin rows and quads across
+// phi = 2 pi take a queue entry and are counted by star_wide.  The queue
+// entries of the workgroup are staged in LDS and appended with one atomic
+// per list: a shared counter takes an atomic only every few nanoseconds.
+// (One lane doing all of it, lensing and splats included, took 307 us of a
+// 1080p frame and 990 us of a 4K one beside the sky pass.)
+__global__ __launch_bounds__(256) void star_scan(const float* thphi, const uint8_t* bh, SceneK s, Cam7 cam, int W,
+                                                 int H, float offset, StarQueue Q, int tiles) {
+    __shared__ uint32_t s_pix[256 * kScanTiles], s_cnt[256 * kScanTiles];
+    __shared__ uint16_t s_wide[256 * kScanTiles], s_tree[256 * kScanTiles];
+    __shared__ unsigned s_n[3], s_base[3];
+    const unsigned tid = threadIdx.y * 16 + threadIdx.x;
+    if (tid < 3) s_n[tid] = 0;
+    __syncthreads();
+    const int i = blockIdx.y * 16 + threadIdx.y;
     const unsigned lane = __lane_id();
-    const unsigned long long m = __ballot(queue);
-    if (m) {
-        const int leader = __ffsll((long long)m) - 1;
-        const unsigned nchunk = queue ? ((unsigned)count + kChunk - 1) / kChunk : 0u;
-        const unsigned nrng = queue && P.picheck ? (unsigned)nodes : 0u;
-        unsigned inc = nchunk, rinc = nrng;
+    for (int tile = 0; tile < tiles; tile++) {
+        const int j = (blockIdx.x * tiles + tile) * 16 + threadIdx.x;
+        const bool valid = i < H && j < W;
+        const size_t ij = valid ? (size_t)i * W + j : 0;
+        uint8_t cls = kDark;
+        bool wide = false, tree = false;
+        int count = 0;
+        if (valid && bh[ij] == 0) {
+            StarPix P;
+            star_pixel_geom(thphi, W, i, j, offset, cam, P);
+            const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
+            const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
+            tree = P.picheck;
+            wide = !tree && r1 - r0 >= kScanRows;
+            if (!tree && !wide) {
+                int b[kScanRows], e[kScanRows];
+#pragma unroll
+                for (int k = 0; k < kScanRows; k++) row_bounds(P, s, r0 + k, r1, p0, p1, b[k], e[k]);
+#pragma unroll
+                for (int k = 0; k < kScanRows; k++) count += e[k] - b[k];
+                if (count > kLightStars) {
+                    cls = kQueued;
+                } else if (count > 0) {
+#pragma unroll
+                    for (int k = 0; k < kScanRows; k++)
+                        for (int q = b[k]; q < e[k]; q++) {
+                            float st, sp;
+                            if (star_test(P, s.bin_pos, q, st, sp)) cls = kFew;
+                        }
+                }
+            }
+        }
+        const bool take = cls == kQueued || wide || tree;
+        const unsigned long long m = __ballot(take);
+        if (m) {
+            unsigned pos = 0;
+            if (lane == 0) pos = atomicAdd(&s_n[0], (unsigned)__popcll(m));
+            pos = __shfl(pos, 0) + (unsigned)__popcll(m & ((1ull << lane) - 1));
+            if (take) {
+                s_pix[pos] = (uint32_t)ij;
+                s_cnt[pos] = wide || tree ? 0u : (uint32_t)count;
+                if (wide) s_wide[atomicAdd(&s_n[1], 1u)] = (uint16_t)pos;
+                if (tree) s_tree[atomicAdd(&s_n[2], 1u)] = (uint16_t)pos;
+            }
+        }
+        if (valid) Q.lit[ij] = cls;
+    }
+    __syncthreads();
+    if (tid < 3 && s_n[tid])
+        s_base[tid] = atomicAdd(&Q.ctr[tid == 0 ? kCtrQueued : tid == 1 ? kCtrWide : kCtrTree], s_n[tid]);
+    __syncthreads();
+    const unsigned n = s_n[0], qb = s_base[0];
+    for (unsigned k = tid; k < n; k += 256) {
+        Q.pix[qb + k] = s_pix[k];
+        Q.cnt[qb + k] = s_cnt[k];
+    }
+    for (unsigned k = tid; k < s_n[1]; k += 256) Q.wide[s_base[1] + k] = qb + s_wide[k];
+    const size_t last = (size_t)W * H + 63;
+    for (unsigned k = tid; k < s_n[2]; k += 256) Q.wide[last - (s_base[2] + k)] = qb + s_tree[k];
+}
+
+// Listed tree nodes of a pixel that star_wide keeps in LDS.
+constexpr int kTreeNodes = 192;
+
+// Counts the candidates of the queue entries star_scan left open: a pixel of
+// more than kLightStars keeps its entry; one of fewer is kFew if a star is
+// inside, else kDark.  One wave per workgroup.  The first `ntree` workgroups
+// take the quads across phi = 2 pi, one lane each, and store their listed
+// node ranges.  A walk of the star tree is a chain of a few hundred
+// dependent steps: it reads the tree from LDS and keeps the listed nodes
+// there, so that it runs once (two walks over memory took 150 us of every
+// frame, however small).  The other workgroups take a tall quad at a time,
+// one bin row per lane (a strongly lensed pixel spans up to all 256).
+__global__ __launch_bounds__(64) void star_wide(const float* thphi, SceneK s, Cam7 cam, int W, int H, float offset,
+                                                StarQueue Q, unsigned ntree) {
+    __shared__ int32_t s_tree[2048];
+    __shared__ uint16_t s_node[kTreeNodes][64];
+    const unsigned lane = threadIdx.x;
+    StarPix P;
+    if (blockIdx.x < ntree) {
+        const unsigned n = Q.ctr[kCtrTree];
+        if (blockIdx.x * 64 >= n) return;
+        const int nodes = (1 << (s.tree_level + 1)) - 1;   // tree_level <= 10
+        for (int k = (int)lane; k < nodes; k += 64) s_tree[k] = s.tree[k];
+        __syncthreads();
+        const size_t last = (size_t)W * H + 63;
+        for (unsigned e0 = blockIdx.x * 64; e0 < n; e0 += ntree * 64) {
+            const bool live = e0 + lane < n;
+            unsigned k = 0, nrng = 0;
+            uint32_t ij = 0;
+            int count = 0;
+            if (live) {
+                k = Q.wide[last - (e0 + lane)];
+                ij = Q.pix[k];
+                star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
+                search_tree(s_tree, s.tree_level, P.mn, P.mx, [&](int node) {
+                    int b, e;
+                    node_range(s_tree, node, b, e);
+                    count += e - b;
+                    if (nrng < (unsigned)kTreeNodes) s_node[nrng][lane] = (uint16_t)node;
+                    nrng++;
+                });
+            }
+            // f(begin, end) for the listed nodes in list order
+            auto listed = [&](auto&& f) {
+                if (nrng <= (unsigned)kTreeNodes) {
+                    for (unsigned x = 0; x < nrng; x++) {
+                        int b, e;
+                        node_range(s_tree, s_node[x][lane], b, e);
+                        f(b, e);
+                    }
+                } else {
+                    search_tree(s_tree, s.tree_level, P.mn, P.mx, [&](int node) {
+                        int b, e;
+                        node_range(s_tree, node, b, e);
+                        f(b, e);
+                    });
+                }
+            };
+            const bool few = live && count <= kLightStars;
+            if (few && count > 0) {
+                bool inside = false;
+                listed([&](int b, int e) {
+                    for (int q = b; q < e; q++) {
+                        float st, sp;
+                        if (star_test(P, s.star_pos, q, st, sp)) inside = true;
+                    }
+                });
+                if (inside) Q.lit[ij] = kFew;
+            }
+            // room for the ranges, one reservation per wave
+            const unsigned want = live && !few ? nrng : 0u;
+            unsigned inc = want;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned o = __shfl_up(inc, off);
+                if ((int)lane >= off) inc += o;
+            }
+            const unsigned tot = __shfl(inc, 63);
+            unsigned base = 0;
+            if (lane == 0 && tot) base = atomicAdd(&Q.ctr[kCtrRanges], tot);
+            const unsigned long long r0 = (unsigned long long)__shfl(base, 0) + inc - want;
+            if (want) {
+                if (r0 + want <= Q.rcap) {
+                    unsigned r = (unsigned)r0;
+                    listed([&](int b, int e) { Q.ranges[r++] = make_int2(b, e); });
+                    Q.rbase[k] = (uint32_t)r0;
+                    Q.nnode[k] = want;
+                    Q.cnt[k] = (uint32_t)count | kTreePixel;
+                    Q.lit[ij] = kQueued;
+                } else {
+                    Q.lit[ij] = kFew;   // no room: traced by one lane
+                }
+            }
+        }
+        return;
+    }
+    const unsigned n = Q.ctr[kCtrWide];
+    for (unsigned w = blockIdx.x - ntree; w < n; w += gridDim.x - ntree) {
+        const unsigned k = Q.wide[w];
+        const uint32_t ij = Q.pix[k];
+        star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
+        const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
+        const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
+        int count = 0;
+        for (int r = r0 + (int)lane; r <= r1; r += 64) {
+            int b, e;
+            row_bounds(P, s, r, r1, p0, p1, b, e);
+            count += e - b;
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) count += __shfl_xor(count, off);
+        if (count > kLightStars) {
+            if (lane == 0) {
+                Q.cnt[k] = (uint32_t)count;
+                Q.lit[ij] = kQueued;
+            }
+        } else if (count > 0) {
+            bool inside = false;
+            for (int r = r0 + (int)lane; r <= r1; r += 64) {
+                int b, e;
+                row_bounds(P, s, r, r1, p0, p1, b, e);
+                for (int q = b; q < e; q++) {
+                    float st, sp;
+                    if (star_test(P, s.bin_pos, q, st, sp)) inside = true;
+                }
+            }
+            if (__ballot(inside) && lane == 0) Q.lit[ij] = kFew;
+        }
+    }
+}
+
+// One lane per queued pixel: its lensing, and its chunk indices.
+__global__ __launch_bounds__(256) void star_assign(const float* thphi, SceneK s, Cam7 cam, int W, int H, float offset,
+                                                   int lr, const float* area, const float* view, StarQueue Q) {
+    const unsigned n = Q.ctr[kCtrQueued];
+    const unsigned lane = threadIdx.x & 63;
+    for (unsigned e0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; e0 < n; e0 += gridDim.x * blockDim.x) {
+        const unsigned k = e0 + lane;
+        const uint32_t qc = k < n ? Q.cnt[k] : 0u;
+        const unsigned nchunk = queued_chunks(qc);
+        unsigned inc = nchunk;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
-            unsigned o = __shfl_up(inc, off), ro = __shfl_up(rinc, off);
-            if ((int)lane >= off) {
-                inc += o;
-                rinc += ro;
-            }
+            const unsigned o = __shfl_up(inc, off);
+            if ((int)lane >= off) inc += o;
         }
-        const unsigned tot = __shfl(inc, 63), rtot = __shfl(rinc, 63);
-        unsigned base = 0, cbase = 0, rbase = 0;
-        if (lane == (unsigned)leader) {
-            base = atomicAdd(&Q.ctr[0], (unsigned)__popcll(m));
-            cbase = atomicAdd(&Q.ctr[1], tot);
-            if (rtot) rbase = atomicAdd(&Q.ctr[3], rtot);
-        }
-        base = __shfl(base, leader);
-        cbase = __shfl(cbase, leader);
-        rbase = __shfl(rbase, leader);
-        if (queue) {
-            const unsigned k = base + (unsigned)__popcll(m & ((1ull << lane) - 1));
-            const unsigned long long c0 = (unsigned long long)cbase + inc - nchunk;
-            const unsigned long long r0 = (unsigned long long)rbase + rinc - nrng;
-            Q.pix[k] = (uint32_t)ij;
-            Q.nnode[k] = (uint32_t)nodes;
-            Q.lens[3 * k] = P.frac;
-            Q.lens[3 * k + 1] = P.redshft;
-            Q.lens[3 * k + 2] = P.red;
-            Q.cstart[k] = (uint32_t)c0;
-            Q.rbase[k] = (uint32_t)r0;
-            if (c0 + nchunk <= Q.cap && r0 + nrng <= Q.rcap) {
-                Q.cnt[k] = (uint32_t)count | (P.picheck ? kTreePixel : 0u) | (odd ? kOddPixel : 0u);
-                for (unsigned c = 0; c < nchunk; c++) Q.owner[c0 + c] = k;
-            } else {
-                // its chunks or tree ranges do not fit: no chunk work, this
-                // lane (or star_map_odd) traces it
-                Q.cnt[k] = 0;
-                for (unsigned long long c = c0; c < Q.cap && c < c0 + nchunk; c++) Q.owner[c] = kNoOwner;
-                if (odd)
-                    to_odd = true;
-                else
-                    seq = self = true;
-            }
+        const unsigned tot = __shfl(inc, 63);
+        unsigned base = 0;
+        if (lane == 0 && tot) base = atomicAdd(&Q.ctr[kCtrChunks], tot);
+        base = __shfl(base, 0);
+        if (nchunk == 0) continue;
+        const uint32_t ij = Q.pix[k];
+        const int i = (int)(ij / (uint32_t)W), j = (int)(ij % (uint32_t)W);
+        StarPix P;
+        star_pixel_geom(thphi, W, i, j, offset, cam, P);
+        star_lens(W, ij, i * (W + 1) + j, lr, area, view, cam, P);
+        Q.lens[3 * k] = P.frac;
+        Q.lens[3 * k + 1] = P.redshft;
+        Q.lens[3 * k + 2] = P.red;
+        const unsigned long long c0 = (unsigned long long)base + inc - nchunk;
+        Q.cstart[k] = (uint32_t)c0;
+        if (c0 + nchunk <= Q.cap) {
+            if (star_pixel_odd(P, s)) Q.cnt[k] = qc | kOddPixel;
+            for (unsigned c = 0; c < nchunk; c++) Q.owner[c0 + c] = k;
+        } else {
+            // its chunks do not fit: no chunk work, one lane traces it
+            Q.cnt[k] = 0;
+            Q.lit[ij] = kFew;
+            for (unsigned long long c = c0; c < Q.cap && c < c0 + nchunk; c++) Q.owner[c] = kNoOwner;
         }
     }
-    wave_append(Q.odd, &Q.ctr[2], to_odd, (uint32_t)ij);
-    if (seq) star_seq<STEP, false>(P, s, count, s_cand[threadIdx.y * blockDim.x + threadIdx.x], acc);
-    // a pixel without candidates has all-zero taps: they are not stored, and
-    // star_sum skips them (the reference zeroes every tap of every pixel)
-    if (valid) Q.lit[ij] = (queue || to_odd || seq) ? 1 : 0;
-    if (seq) store_taps<STEP>(taps, NP, ij, acc);
+}
+
+// Pixels per workgroup of star_few, at most: a span of the frame is chosen so
+// that there are about a thousand workgroups (few_span), each gathering
+// enough kFew pixels to fill its waves where the frame is large.
+constexpr int kFewSpan = 8192;
+
+// The kFew pixels of a span of the frame, gathered in LDS so that full waves
+// trace them, one pixel per lane: all its candidates in order.
+template <int STEP>
+__global__ __launch_bounds__(256) void star_few(const float* thphi, const uint8_t* bh, SceneK s, Cam7 cam, int W,
+                                                int H, float offset, int lr, const float* area, const float* view,
+                                                float* taps, StarQueue Q, int span) {
+    constexpr int FW = 2 * STEP + 1;
+    __shared__ int s_cand[256][kLightStars];
+    __shared__ uint16_t s_list[kFewSpan];
+    __shared__ unsigned s_n;
+    const size_t NP = (size_t)W * H;
+    const size_t p0 = (size_t)blockIdx.x * span;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (int k = 0; k < span; k += 256) {
+        const size_t p = p0 + k + threadIdx.x;
+        if (p < NP && Q.lit[p] == kFew) s_list[atomicAdd(&s_n, 1u)] = (uint16_t)(k + threadIdx.x);
+    }
+    __syncthreads();
+    const unsigned n = s_n;
+    for (unsigned t = threadIdx.x; t < n; t += 256) {
+        const size_t ij = p0 + s_list[t];
+        StarPix P;
+        star_pixel(thphi, bh, W, (int)(ij / (size_t)W), (int)(ij % (size_t)W), offset, lr, area, view, cam, P);
+        const bool odd = star_pixel_odd(P, s);
+        wave_append(Q.odd, &Q.ctr[kCtrOdd], odd, (uint32_t)ij);
+        if (odd) continue;
+        float acc[FW * FW][3];
+#pragma unroll
+        for (int u = 0; u < FW * FW; u++) acc[u][0] = acc[u][1] = acc[u][2] = 0.f;
+        int count = 0;
+        for_ranges(P, s, [&](int b, int e) { count += e - b; });
+        star_seq<STEP, false>(P, s, count, s_cand[threadIdx.x], acc);
+        store_taps<STEP>(taps, NP, ij, acc);
+    }
 }
 
 // One lane per odd pixel (star_pixel_odd) of few candidates: all its
@@ -1045,7 +1313,7 @@ __global__ __launch_bounds__(256) void star_map_odd(const float* thphi, const ui
                                                     const float* view, float* taps, StarQueue Q) {
     constexpr int FW = 2 * STEP + 1;
     __shared__ int s_cand[256][kLightStars];
-    const unsigned n = Q.ctr[2];
+    const unsigned n = Q.ctr[kCtrOdd];
     const size_t NP = (size_t)W * H;
     for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
         const uint32_t ij = Q.odd[k];
@@ -1063,26 +1331,74 @@ __global__ __launch_bounds__(256) void star_map_odd(const float* thphi, const ui
     }
 }
 
-// One lane per queued tree pixel: walks the star tree once more and stores
-// the listed node ranges, in list order, at the place star_map_light took
-// for them.
-__global__ __launch_bounds__(256) void star_tree_ranges(const float* thphi, int W, float offset, SceneK s,
-                                                        Cam7 cam, StarQueue Q) {
-    const unsigned n = Q.ctr[0];
-    for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        if (!(Q.cnt[k] & kTreePixel)) continue;
-        const uint32_t ij = Q.pix[k];
-        StarPix P;
-        star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
-        unsigned r = Q.rbase[k];
-        for_ranges(P, s, [&](int b, int e) { Q.ranges[r++] = make_int2(b, e); });
+// One step of store_tap_sums on the wave's first n values, pairing each lane
+// with lane ^ OFF: h = ceil(n / 2) values stay, the lanes whose bit OFF is
+// clear keep the first h, the others the rest.
+template <int OFF, int N>
+__device__ __forceinline__ void fold_taps(float* v, unsigned lane) {
+    constexpr int h = (N + 1) / 2;
+#pragma unroll
+    for (int k = 0; k < h; k++) {
+        const float a = v[k], b = h + k < N ? v[h + k] : 0.f;
+        if (OFF == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+            v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else if (OFF == 16) {
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+            v[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        } else {
+            const bool up = (lane & OFF) != 0;
+            v[k] = (up ? b : a) + __shfl_xor(up ? a : b, OFF);
+        }
     }
 }
 
+// out[t] = the sum over the wave's lanes of value t of acc, in the order of
+// the xor butterfly 32, 16, 8, 4, 2, 1.  Each step halves the values a lane
+// holds instead of summing all of them on every lane: 29 exchanges for the
+// 27 tap values of step 1 instead of 162, with the same pairs added (an
+// addition's order within a pair does not matter), so the same sums bit for
+// bit.  The two widest steps are the swap instructions of the lane halves
+// and of the 16-lane rows, which move both directions of an exchange at
+// once.  `any` false: every value is zero.
+template <int NT>
+__device__ __forceinline__ void store_tap_sums(float (&acc)[NT / 3][3], bool any, float* out, unsigned lane) {
+    constexpr int n1 = (NT + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2, n4 = (n3 + 1) / 2, n5 = (n4 + 1) / 2,
+                  n6 = (n5 + 1) / 2;
+    if (!any) {
+        for (unsigned t = lane; t < (unsigned)NT; t += 64) out[t] = 0.f;
+        return;
+    }
+    float v[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) v[t] = acc[t / 3][t % 3];
+    fold_taps<32, NT>(v, lane);
+    fold_taps<16, n1>(v, lane);
+    fold_taps<8, n2>(v, lane);
+    fold_taps<4, n3>(v, lane);
+    fold_taps<2, n4>(v, lane);
+    fold_taps<1, n5>(v, lane);
+    // the values this lane is left with: `real` of them from t0 on
+    int t0 = 0, real = NT, n = NT;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const int h = (n + 1) / 2;
+        if (lane & off) {
+            t0 += h;
+            real -= h;
+        } else {
+            real = min(real, h);
+        }
+        n = h;
+    }
+#pragma unroll
+    for (int k = 0; k < n6; k++)
+        if (k < real) out[t0 + k] = v[k];
+}
+
 // One wavefront per chunk (grid-stride): lane l takes the chunk's
-// candidates l, l + 64, ...; the taps are reduced over the wave by a fixed
-// xor butterfly into the chunk's partial, summed per pixel by
-// star_chunk_reduce.  For a binned pixel
+// candidates l, l + 64, ...; the taps are reduced over the wave in a fixed
+// order into the chunk's partial, summed per pixel by star_chunk_reduce.  For a binned pixel
 // the wave walks the footprint's bin rows 64 at a time: each lane loads one
 // row's range, a wave scan gives the rows' first candidate numbers (kept in
 // LDS), and each lane finds the row of each of its candidates.
@@ -1092,11 +1408,10 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
                                                       const float* view, float* taps, StarQueue Q) {
     constexpr int FW = 2 * STEP + 1;
     constexpr int NT = FW * FW * 3;
-    constexpr int PER = (NT + 63) / 64;   // tap values per lane
     const unsigned lane = threadIdx.x & 63;
     const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const unsigned nwaves = (gridDim.x * blockDim.x) >> 6;
-    const unsigned nch = min(Q.ctr[1], Q.cap);
+    const unsigned nch = min(Q.ctr[kCtrChunks], Q.cap);
     const unsigned CH = kChunk;
     __shared__ int s_beg[4][64];
     __shared__ unsigned s_pre[4][65];
@@ -1123,6 +1438,7 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
         float acc[FW * FW][3];
 #pragma unroll
         for (int u = 0; u < FW * FW; u++) acc[u][0] = acc[u][1] = acc[u][2] = 0.f;
+        bool any = false;
         const bool tree = (qc & kTreePixel) != 0;
         const uint32_t rbase = tree ? Q.rbase[lo] : 0u;
         {
@@ -1136,6 +1452,7 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
             const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
             const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
             const int nrange = tree ? (int)Q.nnode[lo] : r1 - r0 + 1;
+            // `any`: a star was found inside.
             // wave-uniform state: current block, its candidate window
             // [gb, a1), the candidates before it, staged stars
             int kb = 0;
@@ -1158,12 +1475,7 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
                                 e = R.y;
                             } else {
                                 const int r = r0 + k;
-                                int q0, q1;
-                                row_span(P, r, p0, p1, q0, q1);
-                                if (q0 <= q1) {
-                                    b = s.bin_start[r * kBinP + q0];
-                                    e = s.bin_start[r * kBinP + q1 + 1];
-                                }
+                                row_bounds(P, s, r, r1, p0, p1, b, e);
                             }
                         }
                         unsigned len = (unsigned)(e - b), inc = len;
@@ -1223,6 +1535,7 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
                     __builtin_amdgcn_wave_barrier();
                 }
                 if (nin == 0) break;
+                any = true;
                 const unsigned take = nin < 64 ? nin : 64u;
                 if (lane < take)
                     star_splat<STEP, ODD>(P, mag, s_iq[wslot][lane], s_ist[wslot][lane], s_isp[wslot][lane],
@@ -1246,26 +1559,9 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
                 if (done && nin == 0) break;
             }
         }
-        // tap value t (tap t / 3, colour t % 3) goes to lane t % 64, slot t / 64
-        float mine[PER];
-#pragma unroll
-        for (int k = 0; k < PER; k++) mine[k] = 0.f;
-#pragma unroll
-        for (int u = 0; u < FW * FW; u++)
-#pragma unroll
-            for (int cc = 0; cc < 3; cc++) {
-                float v = acc[u][cc];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-                if (lane == (unsigned)((3 * u + cc) & 63)) mine[(3 * u + cc) >> 6] = v;
-            }
-        // contiguous per chunk (one coalesced store); the per-tap planes
+        // the sums over the lanes, contiguous per chunk; the per-tap planes
         // are written by star_chunk_reduce
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const unsigned t = (unsigned)k * 64 + lane;
-            if (t < (unsigned)NT) Q.partial[(size_t)c * NT + t] = mine[k];
-        }
+        store_tap_sums<NT>(acc, any, Q.partial + (size_t)c * NT, lane);
     }
 }
 
@@ -1274,7 +1570,7 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
 template <int STEP>
 __global__ __launch_bounds__(256) void star_chunk_reduce(int W, int H, float* taps, StarQueue Q) {
     constexpr int NT = (2 * STEP + 1) * (2 * STEP + 1) * 3;
-    const unsigned n = Q.ctr[0];
+    const unsigned n = Q.ctr[kCtrQueued];
     const size_t NP = (size_t)W * H;
     const size_t total = (size_t)n * NT;
     for (size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x; x < total; x += (size_t)gridDim.x * blockDim.x) {
@@ -1283,7 +1579,18 @@ __global__ __launch_bounds__(256) void star_chunk_reduce(int W, int H, float* ta
         if (nchunk == 0) continue;   // traced by its own lane
         const unsigned c0 = Q.cstart[k];
         float v = 0.f;
-        for (unsigned ch = 0; ch < nchunk; ch++) v += Q.partial[(size_t)(c0 + ch) * NT + t];
+        // eight loads in flight; the sum stays in chunk order (a pixel of
+        // hundreds of chunks would otherwise wait for one load at a time)
+        const float* part = Q.partial + (size_t)c0 * NT + t;
+        unsigned ch = 0;
+        for (; ch + 8 <= nchunk; ch += 8) {
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = part[(size_t)(ch + u) * NT];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v += x[u];
+        }
+        for (; ch < nchunk; ch++) v += part[(size_t)ch * NT];
         taps[(size_t)t * NP + Q.pix[k]] = v;
     }
 }
@@ -1327,7 +1634,7 @@ __global__ __launch_bounds__(256) void star_sum(const float* taps, const uint8_t
     for (int u = start; u <= stop; u++)
         for (int v = 0; v <= 2 * STEP; v++) {
             size_t src = (size_t)(i + u - STEP) * W + ((j + v - STEP + W) % W);
-            if (!lit[src]) continue;   // its taps are zero (and not stored)
+            if (lit[src] == kDark) continue;   // its taps are zero (and not stored)
             int tap = FW * FW - (FW * u + v + 1);
             br += factor * taps[(size_t)(tap * 3 + 0) * NP + src];
             bg += factor * taps[(size_t)(tap * 3 + 1) * NP + src];
@@ -2065,6 +2372,27 @@ __global__ void zero_u32_r(unsigned* p, int n) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
 }
 
+// The pixels that one lane each traces: those of few candidates, then the
+// odd ones among them.
+int few_span(size_t NP) {
+    int span = 256;
+    while (span < kFewSpan && (size_t)span * 1024 < NP) span *= 2;
+    return span;
+}
+
+template <int STEP>
+void star_rest(Context* c, hipStream_t st, const float* thphi, const uint8_t* bh, const SceneK& s,
+               const Cam7& cam, int W, int H, const bt_render_flags& f, const float* area, const float* view,
+               float* taps, const StarQueue& Q) {
+    KTimer t(c, "star_odd", st);
+    const size_t NP = (size_t)W * H;
+    const int span = few_span(NP);
+    star_few<STEP><<<(unsigned)((NP + span - 1) / span), 256, 0, st>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, area,
+                                                                       view, taps, Q, span);
+    star_map_odd<STEP><<<(unsigned)c->num_cus, 256, 0, st>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, area, view, taps,
+                                                             Q);
+}
+
 dim3 grid2d(int W, int H) { return dim3((unsigned)((W + 15) / 16), (unsigned)((H + 15) / 16)); }
 
 }  // namespace
@@ -2249,8 +2577,9 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         StarQueue Q;
         if ((rc = c->buffer("r_star_lens", sizeof(float) * 3 * (NP + 64), &p))) return rc;
         Q.lens = (float*)p;
-        if ((rc = c->buffer("r_star_odd", sizeof(uint32_t) * (NP + 64), &p))) return rc;
+        if ((rc = c->buffer("r_star_odd", sizeof(uint32_t) * 2 * (NP + 64), &p))) return rc;
         Q.odd = (uint32_t*)p;
+        Q.wide = Q.odd + NP + 64;
         if ((rc = c->buffer("r_star_q", sizeof(uint32_t) * 6 * (NP + 64), &p))) return rc;
         Q.pix = (uint32_t*)p;
         Q.cnt = Q.pix + NP + 64;
@@ -2262,18 +2591,21 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         Q.rcap = (unsigned)(NP / 4 + 65536);
         if ((rc = c->buffer("r_star_ranges", sizeof(int2) * (size_t)Q.rcap, &p))) return rc;
         Q.ranges = (int2*)p;
-        if ((rc = c->buffer("r_star_qn", 64, &p))) return rc;
+        if ((rc = c->buffer("r_star_qn", sizeof(unsigned) * kStarCtrWords, &p))) return rc;
         Q.ctr = (unsigned*)p;
         if ((rc = c->buffer("r_star_lit", NP, &p))) return rc;
         Q.lit = (uint8_t*)p;
         const int NT = fw * fw * 3;
         // chunk indices beyond cap are never used: a pixel whose chunks do
-        // not fit is traced by its own lane in star_map_light
+        // not fit is traced by one lane in star_few
         Q.cap = (unsigned)(NP + 64);
         if ((rc = c->buffer("r_star_part", sizeof(float) * NT * (size_t)Q.cap, &p))) return rc;
         Q.partial = (float*)p;
-        zero_u32_r<<<1, 64, 0, c->stream>>>(Q.ctr, 4);
+        zero_u32_r<<<1, 256, 0, c->stream>>>(Q.ctr, kStarCtrWords);
         const unsigned nwave = (unsigned)c->num_cus * 16, nred = (unsigned)c->num_cus * 4;
+        const unsigned ntree = (unsigned)c->num_cus * 2;
+        const int tiles = NP >= (size_t(1) << 20) ? kScanTiles : 1;
+        const dim3 gscan((unsigned)((W + 16 * tiles - 1) / (16 * tiles)), (unsigned)((H + 15) / 16));
         if (tf) {
             // with both passes on, the trails go first on the auxiliary stream:
             // the main stream waits there (after the odd chunks) before the
@@ -2292,18 +2624,13 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
     {                                                                                                       \
         {                                                                                                   \
             KTimer t(c, "star_light");                                                                      \
-            star_map_light<S><<<grid2d(W, H), blk, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr,  \
-                                                                  area, v.view, taps, Q);                   \
-        }                                                                                                   \
-        {                                                                                                   \
-            KTimer t0(c, "star_odd");                                                                       \
-            star_map_odd<S><<<nred, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, area,     \
-                                                         v.view, taps, Q);                                  \
+            star_scan<<<gscan, blk, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, Q, tiles);               \
         }                                                                                                   \
         KTimer t(c, "star_heavy");                                                                          \
         {                                                                                                   \
             KTimer t1(c, "star_tree");                                                                      \
-            star_tree_ranges<<<nred, 256, 0, c->stream>>>(thphi, W, f.offset, s, cam, Q);                   \
+            star_wide<<<nred * 2 + ntree, 64, 0, c->stream>>> (thphi, s, cam, W, H, f.offset, Q, ntree);    \
+            star_assign<<<nred, 256, 0, c->stream>>>(thphi, s, cam, W, H, f.offset, f.lr, area, v.view, Q); \
         }                                                                                                   \
         if (overlap) {                                                                                      \
             /* the odd pixels' chunks (few, long, latency-bound) on the auxiliary stream, between */       \
@@ -2311,6 +2638,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             BT_HIP(hipEventRecord(c->ev_hand, c->stream));                                                  \
             sky_light(c->aux);                                                                              \
             BT_HIP(hipStreamWaitEvent(c->aux, c->ev_hand, 0));                                              \
+            star_rest<S>(c, c->aux, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);               \
             star_map_chunk<S, true><<<nred, 256, 0, c->aux>>>(thphi, bh, s, cam, W, H, f.offset, f.lr,      \
                                                               area, v.view, taps, Q);                       \
             BT_HIP(hipEventRecord(c->ev_back, c->aux));                                                     \
@@ -2320,9 +2648,11 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             KTimer t2(c, "star_chunk");                                                                     \
             star_map_chunk<S, false><<<nwave, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr,  \
                                                                    area, v.view, taps, Q);                  \
-            if (!overlap)                                                                                   \
+            if (!overlap) {                                                                                 \
+                star_rest<S>(c, c->stream, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);        \
                 star_map_chunk<S, true><<<nred, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset,     \
                                                                      f.lr, area, v.view, taps, Q);          \
+            }                                                                                               \
         }                                                                                                   \
         if (overlap) BT_HIP(hipStreamWaitEvent(c->stream, c->ev_back, 0));                                  \
         KTimer t3(c, "star_reduce");                                                                        \
