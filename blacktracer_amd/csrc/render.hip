@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void pix_interp(GridV g, int gridlvl, const fl
     if (i > H || j > W) return;
     size_t c = (size_t)i * (W + 1) + j;
     float theta = view[2 * c] + ver;
-    float phi = fmodf(view[2 * c + 1] + hor + BT_FPI2, BT_FPI2);
+    float phi = fmod_2pi(view[2 * c + 1] + hor + BT_FPI2);
     int gs = 0;
     F2 r = interpolate_pix(g, theta, phi, gridlvl, gs);
     thphi[2 * c] = r.x;
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void pix_interp_blend(GridV ga, GridV gb, int 
     if (i > H || j > W) return;
     size_t c = (size_t)i * (W + 1) + j;
     float theta = view[2 * c] + ver;
-    float phi = fmodf(view[2 * c + 1] + hor + BT_FPI2, BT_FPI2);
+    float phi = fmod_2pi(view[2 * c + 1] + hor + BT_FPI2);
     const float2 b0 = border[0], b1 = border[1];
     const float cx = .5f * b0.x + .5f * b0.y, cy = .5f * b1.x + .5f * b1.y;
     const float stretchRad = fmaxf(b0.y - b0.x, b1.x - b1.y) * 0.75f;
@@ -428,7 +428,7 @@ __device__ __forceinline__ bool corners(const float* thphi, int W, int ind, floa
     p[0] = c0.y; p[1] = c1.y; p[2] = c2.y; p[3] = c3.y;
     for (int q = 0; q < 4; q++) {
         if (p[q] < 0 || t[q] < 0) return false;
-        p[q] = fmodf(p[q] + offset, BT_FPI2);
+        p[q] = fmod_2pi(p[q] + offset);
     }
     picheck = pi_check(p, .2f);
     return true;
@@ -506,7 +506,7 @@ __device__ void lensing_redshift(const float* t, const float* p, int W, int ind,
                                  const float* view, float& frac, float& redshft, float solidAngle) {
     const int M1 = W + 1;
     if (solidAngle == 0.f)
-        solidAngle = calc_area3(t[0], t[1], t[2], p[0], p[1], p[2]) + calc_area3(t[0], t[2], t[3], p[0], p[2], p[3]);
+        solidAngle = quad_area_cold(t[0], t[1], t[2], t[3], p[0], p[1], p[2], p[3]);
     const float2* v = reinterpret_cast<const float2*>(view);
     float2 v0 = v[ind], v1 = v[ind + 1], v2 = v[ind + M1 + 1], v3 = v[ind + M1];
     float ver4[4] = {v0.x, v1.x, v2.x, v3.x};
@@ -727,23 +727,34 @@ __device__ __forceinline__ int bin_of(float v, float d, int n) { return min(max(
 // |A| could reach a bin) bounds nothing.  On a strongly lensed pixel (a thin
 // arc of the Einstein ring) this tests a small fraction of its bounding
 // box's stars.
-__device__ __forceinline__ void row_span(const StarPix& P, int r, int p0, int p1, int& q0, int& q1) {
+struct EdgeLines {
+    float g[4];      // dphi/dtheta of edge k's line
+    unsigned side;   // bit k: it bounds phi from below; bit 4 + k: from above
+    __device__ __forceinline__ void set(const StarPix& P) {
+        const float sg = (float)P.sgn;
+        side = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int kb = (k + 1) & 3;
+            const float A = sg * (P.t[k] - P.t[kb]);
+            const float B = sg * (P.p[k] - P.p[kb]);
+            g[k] = B / A;
+            if (fabsf(B) <= 1000.f * fabsf(A)) side |= A > 0.f ? 1u << k : 16u << k;   // not A == 0, NaN
+        }
+    }
+};
+
+__device__ __forceinline__ void row_span(const float* t, const float* p, float mn1, float mx1, const EdgeLines& L,
+                                         int r, int p0, int p1, int& q0, int& q1) {
     const float ta = ((float)r - 1e-3f) * kBinDT, tb = ((float)r + 1.001f) * kBinDT;
-    float lo = P.mn[1], hi = P.mx[1];
-    const float sg = (float)P.sgn;
+    float lo = mn1, hi = mx1;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int kb = (k + 1) & 3;
-        const float A = sg * (P.t[k] - P.t[kb]);
-        const float B = sg * (P.p[k] - P.p[kb]);
-        if (!(fabsf(B) <= 1000.f * fabsf(A))) continue;   // also A == 0, NaN
-        const float g = B / A;
-        const float la = P.p[kb] + g * (ta - P.t[kb]);
-        const float lb = P.p[kb] + g * (tb - P.t[kb]);
-        if (A > 0.f)
-            lo = fmaxf(lo, fminf(la, lb));
-        else
-            hi = fminf(hi, fmaxf(la, lb));
+        const float la = p[kb] + L.g[k] * (ta - t[kb]);
+        const float lb = p[kb] + L.g[k] * (tb - t[kb]);
+        if (L.side & (1u << k)) lo = fmaxf(lo, fminf(la, lb));
+        if (L.side & (16u << k)) hi = fminf(hi, fmaxf(la, lb));
     }
     if (!(lo <= hi)) {
         q0 = 1;
@@ -755,12 +766,12 @@ __device__ __forceinline__ void row_span(const StarPix& P, int r, int p0, int p1
 }
 
 // The candidates [b, e) of bin row r (none beyond row r1).
-__device__ __forceinline__ void row_bounds(const StarPix& P, const SceneK& s, int r, int r1, int p0, int p1, int& b,
-                                           int& e) {
+__device__ __forceinline__ void row_bounds(const StarPix& P, const EdgeLines& L, const SceneK& s, int r, int r1, int p0,
+                                           int p1, int& b, int& e) {
     b = e = 0;
     if (r > r1) return;
     int q0, q1;
-    row_span(P, r, p0, p1, q0, q1);
+    row_span(P.t, P.p, P.mn[1], P.mx[1], L, r, p0, p1, q0, q1);
     if (q0 <= q1) {
         b = s.bin_start[r * kBinP + q0];
         e = s.bin_start[r * kBinP + q1 + 1];
@@ -780,11 +791,13 @@ __device__ void for_ranges(const StarPix& P, const SceneK& s, F&& f) {
     } else {
         const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
         const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
+        EdgeLines L;
+        L.set(P);
         // four rows' bounds load together
         for (int r = r0; r <= r1; r += 4) {
             int b[4], e[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) row_bounds(P, s, r + k, r1, p0, p1, b[k], e[k]);
+            for (int k = 0; k < 4; k++) row_bounds(P, L, s, r + k, r1, p0, p1, b[k], e[k]);
 #pragma unroll
             for (int k = 0; k < 4; k++)
                 if (b[k] < e[k]) f(b[k], e[k]);
@@ -948,15 +961,17 @@ struct StarQueue {
     float* lens;           // per queued pixel: frac, redshift, 4 log10(redshift)
     uint32_t* wide;        // queue entries that star_wide counts: binned ones from the front, tree ones from the back
     uint32_t* odd;         // pixels for star_map_odd
+    uint32_t* oddc;        // chunks of odd pixels
     unsigned* ctr;         // the counters below, each on a line of its own
     float* partial;        // per chunk: FW*FW*3 partial taps
     unsigned cap;          // chunk capacity of `partial`
     uint8_t* lit;          // per pixel: kDark, or who writes its taps this frame
 };
 // StarQueue::ctr, in words: queued pixels, chunk indices taken, odd pixels,
-// stored ranges, wide entries, tree entries.
-constexpr int kCtrQueued = 0, kCtrChunks = 32, kCtrOdd = 64, kCtrRanges = 96, kCtrWide = 128, kCtrTree = 160;
-constexpr int kStarCtrWords = 192;
+// stored ranges, wide entries, tree entries, odd chunks.
+constexpr int kCtrQueued = 0, kCtrChunks = 32, kCtrOdd = 64, kCtrRanges = 96, kCtrWide = 128, kCtrTree = 160,
+              kCtrOddChunks = 192;
+constexpr int kStarCtrWords = 224;
 // Pixel classes: no star inside (all taps zero, none stored), taps written by
 // star_few / star_map_odd, taps written from the chunks.
 constexpr uint8_t kDark = 0, kFew = 1, kQueued = 2;
@@ -1044,9 +1059,11 @@ __global__ __launch_bounds__(256) void star_scan(const float* thphi, const uint8
             tree = P.picheck;
             wide = !tree && r1 - r0 >= kScanRows;
             if (!tree && !wide) {
+                EdgeLines L;
+                L.set(P);
                 int b[kScanRows], e[kScanRows];
 #pragma unroll
-                for (int k = 0; k < kScanRows; k++) row_bounds(P, s, r0 + k, r1, p0, p1, b[k], e[k]);
+                for (int k = 0; k < kScanRows; k++) row_bounds(P, L, s, r0 + k, r1, p0, p1, b[k], e[k]);
 #pragma unroll
                 for (int k = 0; k < kScanRows; k++) count += e[k] - b[k];
                 if (count > kLightStars) {
@@ -1090,13 +1107,16 @@ __global__ __launch_bounds__(256) void star_scan(const float* thphi, const uint8
     for (unsigned k = tid; k < s_n[2]; k += 256) Q.wide[last - (s_base[2] + k)] = qb + s_tree[k];
 }
 
-// Listed tree nodes of a pixel that star_wide keeps in LDS.
-constexpr int kTreeNodes = 192;
+// Quads across phi = 2 pi per wave of star_wide, and their listed tree nodes
+// kept in LDS.  Lanes of one wave part at every node of their walks, so a
+// wave of 64 walks takes twice as long as one of 8, and a frame has only a
+// few thousand such quads: not enough for 64 a wave to fill the SIMDs.
+constexpr int kTreeLanes = 8, kTreeNodes = 512;
 
 // Counts the candidates of the queue entries star_scan left open: a pixel of
 // more than kLightStars keeps its entry; one of fewer is kFew if a star is
 // inside, else kDark.  One wave per workgroup.  The first `ntree` workgroups
-// take the quads across phi = 2 pi, one lane each, and store their listed
+// take the quads across phi = 2 pi, a few lanes each with a quad, and store their listed
 // node ranges.  A walk of the star tree is a chain of a few hundred
 // dependent steps: it reads the tree from LDS and keeps the listed nodes
 // there, so that it runs once (two walks over memory took 150 us of every
@@ -1105,18 +1125,18 @@ constexpr int kTreeNodes = 192;
 __global__ __launch_bounds__(64) void star_wide(const float* thphi, SceneK s, Cam7 cam, int W, int H, float offset,
                                                 StarQueue Q, unsigned ntree) {
     __shared__ int32_t s_tree[2048];
-    __shared__ uint16_t s_node[kTreeNodes][64];
+    __shared__ uint16_t s_node[kTreeNodes][kTreeLanes];
     const unsigned lane = threadIdx.x;
     StarPix P;
     if (blockIdx.x < ntree) {
         const unsigned n = Q.ctr[kCtrTree];
-        if (blockIdx.x * 64 >= n) return;
+        if (blockIdx.x * kTreeLanes >= n) return;
         const int nodes = (1 << (s.tree_level + 1)) - 1;   // tree_level <= 10
         for (int k = (int)lane; k < nodes; k += 64) s_tree[k] = s.tree[k];
         __syncthreads();
         const size_t last = (size_t)W * H + 63;
-        for (unsigned e0 = blockIdx.x * 64; e0 < n; e0 += ntree * 64) {
-            const bool live = e0 + lane < n;
+        for (unsigned e0 = blockIdx.x * kTreeLanes; e0 < n; e0 += ntree * kTreeLanes) {
+            const bool live = lane < kTreeLanes && e0 + lane < n;
             unsigned k = 0, nrng = 0;
             uint32_t ij = 0;
             int count = 0;
@@ -1193,10 +1213,12 @@ __global__ __launch_bounds__(64) void star_wide(const float* thphi, SceneK s, Ca
         star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
         const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
         const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
+        EdgeLines L;
+        L.set(P);
         int count = 0;
         for (int r = r0 + (int)lane; r <= r1; r += 64) {
             int b, e;
-            row_bounds(P, s, r, r1, p0, p1, b, e);
+            row_bounds(P, L, s, r, r1, p0, p1, b, e);
             count += e - b;
         }
 #pragma unroll
@@ -1210,7 +1232,7 @@ __global__ __launch_bounds__(64) void star_wide(const float* thphi, SceneK s, Ca
             bool inside = false;
             for (int r = r0 + (int)lane; r <= r1; r += 64) {
                 int b, e;
-                row_bounds(P, s, r, r1, p0, p1, b, e);
+                row_bounds(P, L, s, r, r1, p0, p1, b, e);
                 for (int q = b; q < e; q++) {
                     float st, sp;
                     if (star_test(P, s.bin_pos, q, st, sp)) inside = true;
@@ -1252,8 +1274,16 @@ __global__ __launch_bounds__(256) void star_assign(const float* thphi, SceneK s,
         const unsigned long long c0 = (unsigned long long)base + inc - nchunk;
         Q.cstart[k] = (uint32_t)c0;
         if (c0 + nchunk <= Q.cap) {
-            if (star_pixel_odd(P, s)) Q.cnt[k] = qc | kOddPixel;
-            for (unsigned c = 0; c < nchunk; c++) Q.owner[c0 + c] = k;
+            const bool odd = star_pixel_odd(P, s);
+            unsigned o = 0;
+            if (odd) {
+                Q.cnt[k] = qc | kOddPixel;
+                o = atomicAdd(&Q.ctr[kCtrOddChunks], nchunk);
+            }
+            for (unsigned c = 0; c < nchunk; c++) {
+                Q.owner[c0 + c] = k;
+                if (odd) Q.oddc[o + c] = (uint32_t)c0 + c;
+            }
         } else {
             // its chunks do not fit: no chunk work, one lane traces it
             Q.cnt[k] = 0;
@@ -1353,7 +1383,7 @@ __device__ __forceinline__ void fold_taps(float* v, unsigned lane) {
     }
 }
 
-// out[t] = the sum over the wave's lanes of value t of acc, in the order of
+// out[t * stride] = the sum over the wave's lanes of value t of acc, in the order of
 // the xor butterfly 32, 16, 8, 4, 2, 1.  Each step halves the values a lane
 // holds instead of summing all of them on every lane: 29 exchanges for the
 // 27 tap values of step 1 instead of 162, with the same pairs added (an
@@ -1362,11 +1392,12 @@ __device__ __forceinline__ void fold_taps(float* v, unsigned lane) {
 // and of the 16-lane rows, which move both directions of an exchange at
 // once.  `any` false: every value is zero.
 template <int NT>
-__device__ __forceinline__ void store_tap_sums(float (&acc)[NT / 3][3], bool any, float* out, unsigned lane) {
+__device__ __forceinline__ void store_tap_sums(float (&acc)[NT / 3][3], bool any, float* out, size_t stride,
+                                               unsigned lane) {
     constexpr int n1 = (NT + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2, n4 = (n3 + 1) / 2, n5 = (n4 + 1) / 2,
                   n6 = (n5 + 1) / 2;
     if (!any) {
-        for (unsigned t = lane; t < (unsigned)NT; t += 64) out[t] = 0.f;
+        for (unsigned t = lane; t < (unsigned)NT; t += 64) out[t * stride] = 0.f;
         return;
     }
     float v[NT];
@@ -1393,7 +1424,78 @@ __device__ __forceinline__ void store_tap_sums(float (&acc)[NT / 3][3], bool any
     }
 #pragma unroll
     for (int k = 0; k < n6; k++)
-        if (k < real) out[t0 + k] = v[k];
+        if (k < real) out[(t0 + k) * stride] = v[k];
+}
+
+// What star_map_chunk needs of a chunk and its pixel, made by star_heads with
+// one lane per chunk (a wave making it for its own chunk spent a fifth of
+// its instructions on it) and kept in the chunk's partial until the chunk's
+// sums replace it: kHeadWords words, at most the 27 floats of the smallest
+// partial.
+struct ChunkHead {
+    float t[4], p[4];      // the quad's corners
+    EdgeLines edge;        // its edges' lines (side: see kHead* for more bits)
+    float frac, redshft, red;
+    unsigned rows, cols;   // first and last bin row / column (low, high half)
+    unsigned g0, g1;       // its candidates [g0, g1) of the pixel's; g1 == 0: nothing to do
+    unsigned ij, rbase, nrange;
+};
+constexpr int kHeadWords = sizeof(ChunkHead) / 4;
+static_assert(kHeadWords <= 27, "a chunk's head fits its partial");
+constexpr unsigned kHeadFlip = 0x100u, kHeadTree = 0x200u, kHeadOne = 0x400u, kHeadOdd = 0x800u;
+
+template <int NT>
+__global__ __launch_bounds__(256) void star_heads(const float* thphi, Cam7 cam, int W, float offset, StarQueue Q) {
+    const unsigned nch = min(Q.ctr[kCtrChunks], Q.cap);
+    for (unsigned c = blockIdx.x * blockDim.x + threadIdx.x; c < nch; c += gridDim.x * blockDim.x) {
+        ChunkHead h;
+        const uint32_t k = Q.owner[c];
+        const uint32_t qc = k == kNoOwner ? 0u : Q.cnt[k];
+        h.g0 = h.g1 = 0;
+        if (qc) {
+            h.ij = Q.pix[k];
+            h.g0 = (c - Q.cstart[k]) * (unsigned)kChunk;
+            h.g1 = min(h.g0 + kChunk, queued_count(qc));
+            StarPix P;
+            star_pixel_geom(thphi, W, (int)(h.ij / (uint32_t)W), (int)(h.ij % (uint32_t)W), offset, cam, P);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                h.t[q] = P.t[q];
+                h.p[q] = P.p[q];
+            }
+            h.edge.set(P);
+            const bool tree = (qc & kTreePixel) != 0;
+            h.edge.side |= (P.sgn < 0 ? kHeadFlip : 0u) | (tree ? kHeadTree : 0u) |
+                           (queued_chunks(qc) == 1 ? kHeadOne : 0u) | (qc & kOddPixel ? kHeadOdd : 0u);
+            h.frac = Q.lens[3 * k];
+            h.redshft = Q.lens[3 * k + 1];
+            h.red = Q.lens[3 * k + 2];
+            const unsigned r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
+            h.rows = r0 | r1 << 16;
+            h.cols = (unsigned)bin_of(P.mn[1], kBinDP, kBinP) | (unsigned)bin_of(P.mx[1], kBinDP, kBinP) << 16;
+            h.rbase = tree ? Q.rbase[k] : 0u;
+            h.nrange = tree ? Q.nnode[k] : r1 - r0 + 1;
+        }
+        const unsigned* w = reinterpret_cast<const unsigned*>(&h);
+        unsigned* o = reinterpret_cast<unsigned*>(Q.partial + (size_t)c * NT);
+        if (h.g1)
+#pragma unroll
+            for (int q = 0; q < kHeadWords; q++) o[q] = w[q];
+        else
+            o[offsetof(ChunkHead, g1) / 4] = 0;
+    }
+}
+
+// Inclusive sum over the wave's lanes: DPP row shifts, then the rows' last
+// lanes broadcast to the rows after them.
+__device__ __forceinline__ unsigned wave_scan(unsigned v) {
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast15 into rows 1, 3
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast31 into rows 2, 3
+    return v;
 }
 
 // One wavefront per chunk (grid-stride): lane l takes the chunk's
@@ -1409,38 +1511,50 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
     constexpr int FW = 2 * STEP + 1;
     constexpr int NT = FW * FW * 3;
     const unsigned lane = threadIdx.x & 63;
-    const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     const unsigned nwaves = (gridDim.x * blockDim.x) >> 6;
-    const unsigned nch = min(Q.ctr[kCtrChunks], Q.cap);
-    const unsigned CH = kChunk;
+    const unsigned nch = ODD ? Q.ctr[kCtrOddChunks] : min(Q.ctr[kCtrChunks], Q.cap);
     __shared__ int s_beg[4][64];
     __shared__ unsigned s_pre[4][65];
     // stars found inside, staged until 64 can be splatted by a full wave
     __shared__ int s_iq[4][128];
     __shared__ float s_ist[4][128], s_isp[4][128];
     const unsigned wslot = threadIdx.x >> 6;
-    for (unsigned c = wave; c < nch; c += nwaves) {
-        const unsigned lo = Q.owner[c];
-        if (lo == kNoOwner) continue;
-        const uint32_t qc = Q.cnt[lo];
-        if (((qc & kOddPixel) != 0) != ODD) continue;   // the other instance's chunk
-        const uint32_t ij = Q.pix[lo];
-        const unsigned g0 = (c - Q.cstart[lo]) * CH;
-        const unsigned g1 = min(g0 + CH, queued_count(qc));
-        const int i = (int)(ij / (uint32_t)W), j = (int)(ij % (uint32_t)W);
+    for (unsigned x = wave; x < nch; x += nwaves) {
+        const unsigned c = ODD ? Q.oddc[x] : x;
+        // the head, one word per lane, spread to scalars
+        ChunkHead h;
+        {
+            float* part = Q.partial + (size_t)c * NT;
+            const int w = lane < (unsigned)kHeadWords ? __float_as_int(part[lane]) : 0;
+            int* o = reinterpret_cast<int*>(&h);
+#pragma unroll
+            for (int q = 0; q < kHeadWords; q++) o[q] = __builtin_amdgcn_readlane(w, q);
+        }
+        if (h.g1 == 0 || (!ODD && (h.edge.side & kHeadOdd))) continue;   // odd: the other instance's chunk
+        const uint32_t ij = h.ij;
+        const unsigned g0 = h.g0, g1 = h.g1;
+        const bool tree = (h.edge.side & kHeadTree) != 0;
         StarPix P;
-        star_pixel_geom(thphi, W, i, j, offset, cam, P);
-        P.frac = Q.lens[3 * lo];
-        P.redshft = Q.lens[3 * lo + 1];
-        P.red = Q.lens[3 * lo + 2];
-        const float* pos = P.picheck ? s.star_pos : s.bin_pos;
-        const float* mag = P.picheck ? s.star_mag : s.bin_mag;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            P.t[q] = h.t[q];
+            P.p[q] = h.p[q];
+        }
+        P.colours = cam.colours;
+        P.mn[1] = fminf(fminf(P.p[0], P.p[1]), fminf(P.p[2], P.p[3]));
+        P.mx[1] = fmaxf(fmaxf(P.p[0], P.p[1]), fmaxf(P.p[2], P.p[3]));
+        P.frac = h.frac;
+        P.redshft = h.redshft;
+        P.red = h.red;
+        P.sgn = h.edge.side & kHeadFlip ? -1 : 1;
+        P.picheck = tree;   // a quad across phi = 2 pi
+        const float* pos = tree ? s.star_pos : s.bin_pos;
+        const float* mag = tree ? s.star_mag : s.bin_mag;
         float acc[FW * FW][3];
 #pragma unroll
         for (int u = 0; u < FW * FW; u++) acc[u][0] = acc[u][1] = acc[u][2] = 0.f;
         bool any = false;
-        const bool tree = (qc & kTreePixel) != 0;
-        const uint32_t rbase = tree ? Q.rbase[lo] : 0u;
         {
             // The pixel's candidate ranges, 64 at a time: the stored tree
             // node ranges, or the bin rows r0..r1 cut to their phi spans.
@@ -1449,9 +1563,9 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
             // splat runs on full waves however few candidates pass.  One
             // loop alternates filling (up to 64 staged) and splatting, so
             // that the splat has one call site.
-            const int r0 = bin_of(P.mn[0], kBinDT, kBinT), r1 = bin_of(P.mx[0], kBinDT, kBinT);
-            const int p0 = bin_of(P.mn[1], kBinDP, kBinP), p1 = bin_of(P.mx[1], kBinDP, kBinP);
-            const int nrange = tree ? (int)Q.nnode[lo] : r1 - r0 + 1;
+            const int r0 = (int)(h.rows & 0xffffu), r1 = (int)(h.rows >> 16);
+            const int p0 = (int)(h.cols & 0xffffu), p1 = (int)(h.cols >> 16);
+            const int nrange = (int)h.nrange;
             // `any`: a star was found inside.
             // wave-uniform state: current block, its candidate window
             // [gb, a1), the candidates before it, staged stars
@@ -1470,25 +1584,20 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
                         int b = 0, e = 0;
                         if (k < nrange) {
                             if (tree) {
-                                const int2 R = Q.ranges[rbase + (unsigned)k];
+                                const int2 R = Q.ranges[h.rbase + (unsigned)k];
                                 b = R.x;
                                 e = R.y;
                             } else {
                                 const int r = r0 + k;
-                                row_bounds(P, s, r, r1, p0, p1, b, e);
+                                row_bounds(P, h.edge, s, r, r1, p0, p1, b, e);
                             }
                         }
-                        unsigned len = (unsigned)(e - b), inc = len;
-#pragma unroll
-                        for (int off = 1; off < 64; off <<= 1) {
-                            unsigned o = __shfl_up(inc, off);
-                            if ((int)lane >= off) inc += o;
-                        }
+                        const unsigned inc = wave_scan((unsigned)(e - b));
                         __builtin_amdgcn_wave_barrier();
                         s_beg[wslot][lane] = b;
                         s_pre[wslot][lane + 1] = inc;
                         if (lane == 0) s_pre[wslot][0] = 0;
-                        tot = __shfl(inc, 63);
+                        tot = (unsigned)__builtin_amdgcn_readlane((int)inc, 63);
                         __builtin_amdgcn_wave_barrier();
                         gb = max(base, g0);
                         a1 = min(base + tot, g1);
@@ -1559,14 +1668,18 @@ __global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const 
                 if (done && nin == 0) break;
             }
         }
-        // the sums over the lanes, contiguous per chunk; the per-tap planes
-        // are written by star_chunk_reduce
-        store_tap_sums<NT>(acc, any, Q.partial + (size_t)c * NT, lane);
+        // the sums over the lanes: straight into the tap planes for a pixel of
+        // one chunk, else contiguous per chunk for star_chunk_reduce
+        const bool one = (h.edge.side & kHeadOne) != 0;
+        store_tap_sums<NT>(acc, any, one ? taps + ij : Q.partial + (size_t)c * NT, one ? (size_t)W * H : (size_t)1,
+                           lane);
     }
 }
 
-// One thread per (queued pixel, tap value): the pixel's chunk partials
-// summed in chunk order.
+// The queued pixels of several chunks: their partials summed in chunk order,
+// one thread per (pixel, tap value), eight partials in flight at a time (a
+// pixel may have hundreds).  A pixel of one chunk is its partial, which
+// star_map_chunk stores itself.
 template <int STEP>
 __global__ __launch_bounds__(256) void star_chunk_reduce(int W, int H, float* taps, StarQueue Q) {
     constexpr int NT = (2 * STEP + 1) * (2 * STEP + 1) * 3;
@@ -1576,19 +1689,16 @@ __global__ __launch_bounds__(256) void star_chunk_reduce(int W, int H, float* ta
     for (size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x; x < total; x += (size_t)gridDim.x * blockDim.x) {
         const unsigned k = (unsigned)(x / NT), t = (unsigned)(x % NT);
         const unsigned nchunk = queued_chunks(Q.cnt[k]);
-        if (nchunk == 0) continue;   // traced by its own lane
-        const unsigned c0 = Q.cstart[k];
+        if (nchunk <= 1) continue;   // 0: traced by one lane
+        const float* part = Q.partial + (size_t)Q.cstart[k] * NT + t;
         float v = 0.f;
-        // eight loads in flight; the sum stays in chunk order (a pixel of
-        // hundreds of chunks would otherwise wait for one load at a time)
-        const float* part = Q.partial + (size_t)c0 * NT + t;
         unsigned ch = 0;
         for (; ch + 8 <= nchunk; ch += 8) {
-            float x[8];
+            float y[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) x[u] = part[(size_t)(ch + u) * NT];
+            for (int u = 0; u < 8; u++) y[u] = part[(size_t)(ch + u) * NT];
 #pragma unroll
-            for (int u = 0; u < 8; u++) v += x[u];
+            for (int u = 0; u < 8; u++) v += y[u];
         }
         for (; ch < nchunk; ch++) v += part[(size_t)ch * NT];
         taps[(size_t)t * NP + Q.pix[k]] = v;
@@ -2028,41 +2138,60 @@ __global__ __launch_bounds__(256) void make_pix_all(const float* light, int64_t 
     if (ij < NP) make_pix(light[3 * ij], light[3 * ij + 1], light[3 * ij + 2], img, (size_t)ij);
 }
 
-// distortEnvironmentMap (MakeImageKernel.cu:631-751)
 // ---- distortEnvironmentMap (MakeImageKernel.cu:631-751) ----
-// Pixels whose celestial footprint spans at most kHeavyCols sky columns
-// (about 90% of them) are done one per lane by env_map; those with up to
-// kLaneCols queue for env_map_lane (one per lane, compacted, so that a wave's
-// lanes have similar work) and the rest for env_map_heavy, one wavefront
-// per pixel, so that a pixel on the Einstein ring with thousands of columns
-// does not stall its neighbours' wave.
+// A pixel sums one summed-table difference per sky column of its footprint,
+// in column order.  env_map does pixels of at most kInlineCols columns (70%
+// of a lensed 1080p frame), one lane each; env_map_group those of up to
+// kGroupCols, eight lanes each; env_map_heavy the rest, one wavefront each.
 
-constexpr int kHeavyCols = 32;
+constexpr int kInlineCols = 8;
+constexpr int kGroupCols = 256;
 
 struct EnvPix {
     float t[4], p[4];
+    float slope[4];   // of edge q, theta over phi
     int ind, pixMin, pixNum;
-    float pixSize, thMax, thMin;
+    float thMax, thMin;
 };
+
+// The sky: summed table, its size, the size of a texel and the inverse of
+// that in FP64.
+struct SkyK {
+    const float4* table;
+    int rows, cols;
+    float pixSize;
+    double inv;
+};
+
+// Texel index of an angle: cvt_i32(x / pixSize).  The FP64 product with the
+// rounded inverse is within 2^-52 of the quotient, and a quotient of two
+// 24-bit numbers is no 25-bit one and at least 2^-49 from any, so it rounds
+// to the same float as the division (a third of its instructions).
+__device__ __forceinline__ int texel(const SkyK& K, float x) { return cvt_i32((float)((double)x * K.inv)); }
 
 // Corners and column range of pixel (i, j); false for pixel index 0 (the
 // reference's `ind > 0`, MakeImageKernel.cu:647), which stays black.
-__device__ __forceinline__ bool env_setup(const float* thphi, int W, int i, int j, float offset, int rows,
+__device__ __forceinline__ bool env_setup(const float* thphi, int W, int i, int j, float offset, const SkyK& K,
                                           EnvPix& E) {
     bool picheck = false;
     E.ind = i * (W + 1) + j;
     corners(thphi, W, E.ind, E.t, E.p, picheck, offset);
     if (E.ind <= 0) return false;
-    E.pixSize = BT_FPI / (float)rows;
     float phMax = fmaxf(fmaxf(E.p[0], E.p[1]), fmaxf(E.p[2], E.p[3]));
     float phMin = fminf(fminf(E.p[0], E.p[1]), fminf(E.p[2], E.p[3]));
-    int pixMax = cvt_i32(phMax / E.pixSize);
-    E.pixMin = cvt_i32(phMin / E.pixSize);
+    int pixMax = texel(K, phMax);
+    E.pixMin = texel(K, phMin);
     E.pixNum = pixMax - E.pixMin + 1;
-    if (E.pixNum > 1 && pixMax * E.pixSize > phMax) E.pixNum -= 1;
+    if (E.pixNum > 1 && pixMax * K.pixSize > phMax) E.pixNum -= 1;
     E.thMax = fmaxf(fmaxf(E.t[0], E.t[1]), fmaxf(E.t[2], E.t[3]));
     E.thMin = fminf(fminf(E.t[0], E.t[1]), fminf(E.t[2], E.t[3]));
     return true;
+}
+
+__device__ __forceinline__ void env_slopes(EnvPix& E) {
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        E.slope[q] = (E.t[(q + 1) % 4] - E.t[q]) / (E.p[(q + 1) % 4] - E.p[q]);
 }
 
 // The quad's theta span on the column boundary at phi = cp, folded into the
@@ -2071,27 +2200,32 @@ __device__ __forceinline__ void env_boundary(const EnvPix& E, float cp, float& m
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         float ap = E.p[q], bp = E.p[(q + 1) % 4];
-        float at = E.t[q], bt = E.t[(q + 1) % 4];
-        if ((cp - ap) * (cp - bp) <= 0) {
-            float ct = at + (bt - at) / (bp - ap) * (cp - ap);
-            mn = ct < mn ? ct : mn;
-            mx = ct > mx ? ct : mx;
-        }
+        float ct = E.t[q] + E.slope[q] * (cp - ap);
+        const bool on = (cp - ap) * (cp - bp) <= 0;
+        mn = on && ct < mn ? ct : mn;
+        mx = on && ct > mx ? ct : mx;
     }
 }
 
-// Summed-table difference of column `col` over the running span.
-__device__ __forceinline__ float4 env_column(const float4* table, int rows, int cols, float pixSize, int col,
-                                             float mn, float mx) {
-    int rmax = min(max(cvt_i32(mx / pixSize), 0), rows - 1);
-    float4 mxc = table[(size_t)rmax * cols + col];
-    int index2 = (cvt_i32(mn / pixSize) - 1) * cols + col;
-    float4 mnc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (index2 > 0) {
-        if (index2 >= rows * cols) index2 = (rows - 1) * cols + col;
-        mnc = table[index2];
-    }
+// Table indices of the two ends of column `col` over the running span; lo < 0: no lower end.
+__device__ __forceinline__ void env_ends(const SkyK& K, int col, float mn, float mx, int& hi, int& lo) {
+    hi = min(max(texel(K, mx), 0), K.rows - 1) * K.cols + col;
+    const int index2 = (texel(K, mn) - 1) * K.cols + col;
+    lo = index2 <= 0 ? -1 : index2 >= K.rows * K.cols ? (K.rows - 1) * K.cols + col : index2;
+}
+
+__device__ __forceinline__ float4 env_diff(float4 mxc, float4 mnc) {
     return make_float4(mxc.x - mnc.x, mxc.y - mnc.y, mxc.z - mnc.z, mxc.w - mnc.w);
+}
+
+// Summed-table difference of column `col` over the running span.
+__device__ __forceinline__ float4 env_column(const SkyK& K, int col, float mn, float mx) {
+    int hi, lo;
+    env_ends(K, col, mn, mx, hi, lo);
+    const float4 mxc = K.table[hi];
+    float4 mnc = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (lo >= 0) mnc = K.table[lo];
+    return env_diff(mxc, mnc);
 }
 
 // Mean colour -> gamma -> HSP -> lensing/redshift -> BGRA (MakeImageKernel.cu:733-750).
@@ -2120,37 +2254,57 @@ __device__ __forceinline__ uchar4 env_finish(const EnvPix& E, float cx, float cy
 }
 
 // Column sums of a pixel in the reference's order (one lane).
-__device__ __forceinline__ float4 env_seq(const EnvPix& E, const float4* table, int rows, int cols) {
+__device__ __forceinline__ float4 env_seq(EnvPix& E, const SkyK& K) {
+    const int cols = K.cols;
     float cx = 0.f, cy = 0.f, cz = 0.f, cw = 0.f;
     if (E.pixNum == 1) {
-        int rmax = min(max(cvt_i32(E.thMax / E.pixSize), 0), rows - 1);
-        int rmin = cvt_i32(E.thMin / E.pixSize) - 1;
+        int rmax = min(max(texel(K, E.thMax), 0), K.rows - 1);
+        int rmin = texel(K, E.thMin) - 1;
         int col = min(max(E.pixMin, 0), cols - 1);
-        float4 mxc = table[(size_t)rmax * cols + col];
+        float4 mxc = K.table[(size_t)rmax * cols + col];
         float4 mnc = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (rmin >= 0) mnc = table[(size_t)min(rmin, rows - 1) * cols + col];
+        if (rmin >= 0) mnc = K.table[(size_t)min(rmin, K.rows - 1) * cols + col];
         cx = mxc.x - mnc.x;
         cy = mxc.y - mnc.y;
         cz = mxc.z - mnc.z;
         cw = mxc.w - mnc.w;
     } else if (E.pixNum < cols) {
+        env_slopes(E);
         float mx = -100, mn = cols + 1;
-        for (int sidx = 0; sidx <= E.pixNum; sidx++) {
-            env_boundary(E, (E.pixMin + sidx) * E.pixSize, mn, mx);
-            if (sidx > 0) {
-                float4 d = env_column(table, rows, cols, E.pixSize, (E.pixMin + sidx) % cols, mn, mx);
-                cx += d.x;
-                cy += d.y;
-                cz += d.z;
-                cw += d.w;
+        env_boundary(E, E.pixMin * K.pixSize, mn, mx);
+        int col = E.pixMin % cols;
+        // four columns at a time: their loads are in flight together, their
+        // terms are added in column order
+        for (int s0 = 1; s0 <= E.pixNum; s0 += 4) {
+            float4 a[4], b[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                a[u] = b[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (s0 + u <= E.pixNum) {
+                    env_boundary(E, (E.pixMin + s0 + u) * K.pixSize, mn, mx);
+                    col = col + 1 == cols ? 0 : col + 1;
+                    int hi, lo;
+                    env_ends(K, col, mn, mx, hi, lo);
+                    a[u] = K.table[hi];
+                    if (lo >= 0) b[u] = K.table[lo];
+                }
             }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (s0 + u <= E.pixNum) {
+                    const float4 d = env_diff(a[u], b[u]);
+                    cx += d.x;
+                    cy += d.y;
+                    cz += d.z;
+                    cw += d.w;
+                }
         }
     } else {
-        int thMaxPix = min(max(cvt_i32(E.thMax / E.pixSize), 0), rows - 1) * cols;
-        int thMinPix = min(max(cvt_i32(E.thMin / E.pixSize), 0), rows - 1) * cols;
+        int thMaxPix = min(max(texel(K, E.thMax), 0), K.rows - 1) * cols;
+        int thMinPix = min(max(texel(K, E.thMin), 0), K.rows - 1) * cols;
         for (int q = 0; q < E.pixNum; q++) {
-            float4 mxc = table[thMaxPix + (E.pixMin + q) % cols];
-            float4 mnc = table[thMinPix + (E.pixMin + q) % cols];
+            float4 mxc = K.table[thMaxPix + (E.pixMin + q) % cols];
+            float4 mnc = K.table[thMinPix + (E.pixMin + q) % cols];
             cx += mxc.x - mnc.x;
             cy += mxc.y - mnc.y;
             cz += mxc.z - mnc.z;
@@ -2160,44 +2314,135 @@ __device__ __forceinline__ float4 env_seq(const EnvPix& E, const float4* table, 
     return make_float4(cx, cy, cz, cw);
 }
 
-constexpr int kLaneCols = 256;
+// env counters, each on a line of its own: entries of the group and the heavy queue
+constexpr int kCtrGroup = 0, kCtrHeavy = 32, kEnvCtrWords = 64;
 
-__global__ __launch_bounds__(256) void env_map(const float* thphi, const uint8_t* bh, SceneK s, Cam7 cam, int W,
+__global__ __launch_bounds__(256) void env_map(const float* thphi, const uint8_t* bh, SkyK K, Cam7 cam, int W,
                                                int H, float offset, int lr, const float* area,
-                                               const float* view, uint8_t* img, uint32_t* qlane, uint32_t* qwave,
+                                               const float* view, uint8_t* img, uint32_t* qgroup, uint32_t* qwave,
                                                unsigned* nq) {
+    __shared__ uint32_t s_q[2][256];
+    __shared__ unsigned s_n[2], s_base[2];
+    const unsigned tid = threadIdx.y * 16 + threadIdx.x;
+    if (tid < 2) s_n[tid] = 0;
+    __syncthreads();
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     int i = blockIdx.y * blockDim.y + threadIdx.y;
-    if (i >= H || j >= W) return;
-    const size_t ij = (size_t)i * W + j;
-    const float4* table = reinterpret_cast<const float4*>(s.table);
-    uchar4 o = make_uchar4(0, 0, 0, 255);
+    const bool valid = i < H && j < W;
+    const size_t ij = valid ? (size_t)i * W + j : 0;
     EnvPix E;
-    const bool live = bh[ij] == 0 && env_setup(thphi, W, i, j, offset, s.rows, E);
-    const int tier = !live || E.pixNum <= kHeavyCols ? 0 : E.pixNum <= kLaneCols ? 1 : 2;
-    wave_append(qlane, &nq[0], tier == 1, (uint32_t)ij);
-    wave_append(qwave, &nq[1], tier == 2, (uint32_t)ij);
-    if (tier != 0) return;   // env_map_lane / env_map_heavy write this pixel
+    const bool live = valid && bh[ij] == 0 && env_setup(thphi, W, i, j, offset, K, E);
+    const int tier = !live || E.pixNum <= kInlineCols ? 0 : E.pixNum <= kGroupCols ? 1 : 2;
+    if (tier) s_q[tier - 1][atomicAdd(&s_n[tier - 1], 1u)] = (uint32_t)ij;
+    __syncthreads();
+    // one append per workgroup and queue
+    if (tid < 2 && s_n[tid]) s_base[tid] = atomicAdd(&nq[tid ? kCtrHeavy : kCtrGroup], s_n[tid]);
+    __syncthreads();
+    if (tid < s_n[0]) qgroup[s_base[0] + tid] = s_q[0][tid];
+    if (tid < s_n[1]) qwave[s_base[1] + tid] = s_q[1][tid];
+    if (!valid || tier != 0) return;   // env_map_group / env_map_heavy write this pixel
+    uchar4 o = make_uchar4(0, 0, 0, 255);
     if (live) {
-        float4 c4 = env_seq(E, table, s.rows, s.cols);
+        float4 c4 = env_seq(E, K);
         o = env_finish(E, c4.x, c4.y, c4.z, c4.w, W, lr, cam, view, area[ij]);
     }
     reinterpret_cast<uchar4*>(img)[ij] = o;
 }
 
-// One queued pixel per lane, in the reference's column order.
-__global__ __launch_bounds__(256) void env_map_lane(const float* thphi, SceneK s, Cam7 cam, int W, float offset,
-                                                    int lr, const float* area, const float* view, uint8_t* img,
-                                                    const uint32_t* q, const unsigned* nq) {
+// Sixteen lanes per queued pixel: a lane takes every sixteenth column
+// boundary, the running span (an exact min/max) is scanned over the lanes,
+// the sixteen columns' loads are in flight together, and their terms, staged
+// in LDS, are added in column order, one colour component per lane.  A wave
+// takes 64 pixels (fewer where the queue does not fill the launch) and
+// finishes their means together.  (One lane per pixel, column after column,
+// took 180 us of every frame, however small.)
+constexpr int kGroupLanes = 16, kGroupPix = 64 / kGroupLanes;   // a 16-lane DPP row per pixel
+
+// One step of the inclusive min/max scan over a 16-lane row: CTRL is the DPP
+// row shift; lanes shifted in from outside the row keep their own values.
+template <int CTRL>
+__device__ __forceinline__ void row_scan(float& mn, float& mx) {
+    const float a = __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(mn), __float_as_int(mn), CTRL, 0xf, 0xf, false));
+    const float b = __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(mx), __float_as_int(mx), CTRL, 0xf, 0xf, false));
+    mn = fminf(mn, a);
+    mx = fmaxf(mx, b);
+}
+
+__global__ __launch_bounds__(256) void env_map_group(const float* thphi, SkyK K, Cam7 cam, int W, float offset,
+                                                     int lr, const float* area, const float* view, uint8_t* img,
+                                                     const uint32_t* queue, const unsigned* nq) {
+    __shared__ float4 s_d[4][64];     // per wave: the terms of kGroupPix pixels x kGroupLanes columns
+    __shared__ float s_c[4][64][4];   // per wave: the sums of its pixels
     const unsigned n = *nq;
-    const float4* table = reinterpret_cast<const float4*>(s.table);
-    for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-        const uint32_t ij = q[e];
-        EnvPix E;
-        env_setup(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, s.rows, E);
-        float4 c4 = env_seq(E, table, s.rows, s.cols);
-        reinterpret_cast<uchar4*>(img)[ij] = env_finish(E, c4.x, c4.y, c4.z, c4.w, W, lr, cam, view, area[ij]);
+    const unsigned lane = threadIdx.x & 63, wslot = threadIdx.x >> 6;
+    const unsigned sub = lane % kGroupLanes, grp = lane / kGroupLanes;
+    const unsigned nwaves = gridDim.x * 4;
+    const unsigned rounds = min(64u / kGroupPix, max(1u, n / (kGroupPix * nwaves)));
+    const unsigned per = rounds * kGroupPix;   // pixels a wave takes at a time
+    const int cols = K.cols;
+    for (unsigned e0 = (blockIdx.x * 4 + wslot) * per; e0 < n; e0 += nwaves * per) {
+        for (unsigned r = 0; r < rounds; r++) {
+            const unsigned e = e0 + r * kGroupPix + grp;
+            int num = -1;   // last boundary; -1: nothing to do here
+            EnvPix E;
+            if (e < n) {
+                const uint32_t ij = queue[e];
+                env_setup(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, K, E);
+                env_slopes(E);
+                if (E.pixNum < cols) num = E.pixNum;
+            }
+            float sum = 0.f, cmn = cols + 1, cmx = -100;   // (cmn, cmx): the span after the columns so far
+            int col = num >= 0 ? (E.pixMin + (int)sub) % cols : 0;
+            for (int s0 = 0; __ballot(s0 <= num); s0 += kGroupLanes) {
+                const int sidx = s0 + (int)sub;
+                float mn = cols + 1, mx = -100;
+                if (sidx <= num) env_boundary(E, (E.pixMin + sidx) * K.pixSize, mn, mx);
+                row_scan<0x111>(mn, mx);
+                row_scan<0x112>(mn, mx);
+                row_scan<0x114>(mn, mx);
+                row_scan<0x118>(mn, mx);
+                mn = fminf(mn, cmn);
+                mx = fmaxf(mx, cmx);
+                cmn = __shfl(mn, kGroupLanes - 1, kGroupLanes);
+                cmx = __shfl(mx, kGroupLanes - 1, kGroupLanes);
+                float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (sidx > 0 && sidx <= num) d = env_column(K, col, mn, mx);
+                col += kGroupLanes;
+                while (col >= cols) col -= cols;
+                __builtin_amdgcn_wave_barrier();
+                s_d[wslot][lane] = d;
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (sub < 4) {
+                    const float* x = reinterpret_cast<const float*>(&s_d[wslot][grp * kGroupLanes]) + sub;
+                    float v[kGroupLanes];
+#pragma unroll
+                    for (int u = 0; u < kGroupLanes; u++) v[u] = x[4 * u];
+#pragma unroll
+                    for (int u = 0; u < kGroupLanes; u++) sum += v[u];   // a term outside the footprint is zero
+                }
+            }
+            if (sub < 4) s_c[wslot][r * kGroupPix + grp][sub] = sum;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < per && e0 + lane < n) {
+            const uint32_t ij = queue[e0 + lane];
+            EnvPix E;
+            env_setup(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, K, E);
+            const float* c = s_c[wslot][lane];
+            float4 c4 = make_float4(c[0], c[1], c[2], c[3]);
+            if (E.pixNum >= cols) c4 = env_seq(E, K);   // a sky of fewer columns than the footprint's
+            reinterpret_cast<uchar4*>(img)[ij] = env_finish(E, c4.x, c4.y, c4.z, c4.w, W, lr, cam, view, area[ij]);
+        }
+        __builtin_amdgcn_wave_barrier();
     }
+}
+
+__device__ __forceinline__ float read_lane(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 __device__ __forceinline__ float wave_xor_sum(float v) {
@@ -2206,77 +2451,114 @@ __device__ __forceinline__ float wave_xor_sum(float v) {
     return v;
 }
 
-// One wavefront per queued pixel (grid-stride over the queue).  Lanes take
-// contiguous chunks of the column boundaries; the running theta span is an
-// exact min/max, so a lane starts its chunk from the min/max of all earlier
-// boundaries (a wave scan) and sees the spans the sequential loop sees.
-// Column terms are summed per lane and reduced in a fixed order.
-__global__ __launch_bounds__(256) void env_map_heavy(const float* thphi, SceneK s, Cam7 cam, int W,
+// One wavefront per queued pixel.  The sum's order: the column boundaries are
+// cut into 64 contiguous chunks, each chunk's terms are added in order, and
+// the 64 sums by an xor butterfly.  The terms are made 64 neighbouring
+// columns at a time, one per lane (the running theta span is an exact
+// min/max, scanned over the lanes), so that the table is read in whole
+// lines, and staged in LDS, kHeavyWindow of them; then the lanes add the
+// terms of their chunks.  (A lane walking its own chunk through memory read
+// every line about twice and made every boundary twice: 277 us of a 1080p
+// frame's sky pass.)  A wave finishes the means of its pixels together, one
+// per lane.
+constexpr int kHeavyWindow = 512;
+
+__global__ __launch_bounds__(128) void env_map_heavy(const float* thphi, SkyK K, Cam7 cam, int W,
                                                      float offset, int lr, const float* area, const float* view,
                                                      uint8_t* img, const uint32_t* heavy, const unsigned* nheavy) {
-    const unsigned lane = threadIdx.x & 63;
+    __shared__ float4 s_c[2][64];
+    __shared__ float4 s_d[2][kHeavyWindow];
+    const unsigned lane = threadIdx.x & 63, wslot = threadIdx.x >> 6;
     const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const unsigned nwaves = (gridDim.x * blockDim.x) >> 6;
     const unsigned n = *nheavy;
-    const int rows = s.rows, cols = s.cols;
-    const float4* table = reinterpret_cast<const float4*>(s.table);
-    for (unsigned e = wave; e < n; e += nwaves) {
-        const uint32_t ij = heavy[e];
-        const int i = (int)(ij / (uint32_t)W), j = (int)(ij % (uint32_t)W);
-        EnvPix E;
-        env_setup(thphi, W, i, j, offset, rows, E);
-        float cx = 0.f, cy = 0.f, cz = 0.f, cw = 0.f;
-        if (E.pixNum < cols) {
-            const int nb = E.pixNum + 1;   // boundaries 0..pixNum
-            const int per = (nb + 63) / 64;
-            const int lo = min((int)lane * per, nb), hi = min(lo + per, nb);
-            float mx = -100, mn = cols + 1;
-            for (int b = lo; b < hi; b++) env_boundary(E, (E.pixMin + b) * E.pixSize, mn, mx);
-            // exclusive scan of (mn, mx) over lanes
-            float pmn = mn, pmx = mx;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                float omn = __shfl_up(pmn, off), omx = __shfl_up(pmx, off);
-                if ((int)lane >= off) {
-                    pmn = fminf(pmn, omn);
-                    pmx = fmaxf(pmx, omx);
+    const int rows = K.rows, cols = K.cols;
+    // pixel wave + k nwaves is the wave's k-th
+    for (unsigned e0 = wave; e0 < n; e0 += 64 * nwaves) {
+        unsigned cnt = 0;
+        for (; cnt < 64 && e0 + cnt * nwaves < n; cnt++) {
+            const uint32_t ij = heavy[e0 + cnt * nwaves];
+            EnvPix E;
+            env_setup(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, K, E);
+            float cx = 0.f, cy = 0.f, cz = 0.f, cw = 0.f;
+            if (E.pixNum < cols) {
+                env_slopes(E);
+                const int nb = E.pixNum + 1;   // boundaries 0..pixNum
+                const int per = (nb + 63) / 64;
+                int next = min((int)lane * per, nb);   // the chunk's next term
+                const int end = min(next + per, nb);
+                float cmn = cols + 1, cmx = -100;      // the span after the boundaries so far
+                int col = (E.pixMin + (int)lane) % cols;
+                for (int w0 = 0; w0 < nb; w0 += kHeavyWindow) {
+#pragma unroll 4
+                    for (int b0 = 0; b0 < kHeavyWindow; b0 += 64) {
+                        if (w0 + b0 >= nb) break;
+                        const int b = w0 + b0 + (int)lane;
+                        float mn = cols + 1, mx = -100;
+                        if (b < nb) env_boundary(E, (E.pixMin + b) * K.pixSize, mn, mx);
+                        // inclusive scan over the rows of 16, then over the rows
+                        row_scan<0x111>(mn, mx);
+                        row_scan<0x112>(mn, mx);
+                        row_scan<0x114>(mn, mx);
+                        row_scan<0x118>(mn, mx);
+                        const float n0 = read_lane(mn, 15), n1 = read_lane(mn, 31), n2 = read_lane(mn, 47),
+                                    n3 = read_lane(mn, 63);
+                        const float x0 = read_lane(mx, 15), x1 = read_lane(mx, 31), x2 = read_lane(mx, 47),
+                                    x3 = read_lane(mx, 63);
+                        const float n01 = fminf(n0, n1), x01 = fmaxf(x0, x1);
+                        const float n02 = fminf(n01, n2), x02 = fmaxf(x01, x2);
+                        const unsigned row = lane >> 4;
+                        mn = fminf(fminf(mn, cmn), row == 0 ? mn : row == 1 ? n0 : row == 2 ? n01 : n02);
+                        mx = fmaxf(fmaxf(mx, cmx), row == 0 ? mx : row == 1 ? x0 : row == 2 ? x01 : x02);
+                        cmn = fminf(cmn, fminf(n02, n3));
+                        cmx = fmaxf(cmx, fmaxf(x02, x3));
+                        float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
+                        if (b > 0 && b < nb) d = env_column(K, col, mn, mx);
+                        col += 64;
+                        while (col >= cols) col -= cols;
+                        s_d[wslot][b0 + lane] = d;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    const int stop = min(end, w0 + kHeavyWindow);
+                    for (; next < stop; next++) {
+                        const float4 d = s_d[wslot][next - w0];   // term 0 is zero
+                        cx += d.x;
+                        cy += d.y;
+                        cz += d.z;
+                        cw += d.w;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                }
+            } else {
+                int thMaxPix = min(max(texel(K, E.thMax), 0), rows - 1) * cols;
+                int thMinPix = min(max(texel(K, E.thMin), 0), rows - 1) * cols;
+                for (int q = lane; q < E.pixNum; q += 64) {
+                    float4 mxc = K.table[thMaxPix + (E.pixMin + q) % cols];
+                    float4 mnc = K.table[thMinPix + (E.pixMin + q) % cols];
+                    cx += mxc.x - mnc.x;
+                    cy += mxc.y - mnc.y;
+                    cz += mxc.z - mnc.z;
+                    cw += mxc.w - mnc.w;
                 }
             }
-            float emn = __shfl_up(pmn, 1), emx = __shfl_up(pmx, 1);
-            if (lane == 0) {
-                emn = cols + 1;
-                emx = -100;
-            }
-            mn = emn;
-            mx = emx;
-            for (int b = lo; b < hi; b++) {
-                env_boundary(E, (E.pixMin + b) * E.pixSize, mn, mx);
-                if (b > 0) {
-                    float4 d = env_column(table, rows, cols, E.pixSize, (E.pixMin + b) % cols, mn, mx);
-                    cx += d.x;
-                    cy += d.y;
-                    cz += d.z;
-                    cw += d.w;
-                }
-            }
-        } else {
-            int thMaxPix = min(max(cvt_i32(E.thMax / E.pixSize), 0), rows - 1) * cols;
-            int thMinPix = min(max(cvt_i32(E.thMin / E.pixSize), 0), rows - 1) * cols;
-            for (int q = lane; q < E.pixNum; q += 64) {
-                float4 mxc = table[thMaxPix + (E.pixMin + q) % cols];
-                float4 mnc = table[thMinPix + (E.pixMin + q) % cols];
-                cx += mxc.x - mnc.x;
-                cy += mxc.y - mnc.y;
-                cz += mxc.z - mnc.z;
-                cw += mxc.w - mnc.w;
-            }
+            cx = wave_xor_sum(cx);
+            cy = wave_xor_sum(cy);
+            cz = wave_xor_sum(cz);
+            cw = wave_xor_sum(cw);
+            if (lane == 0) s_c[wslot][cnt] = make_float4(cx, cy, cz, cw);
         }
-        cx = wave_xor_sum(cx);
-        cy = wave_xor_sum(cy);
-        cz = wave_xor_sum(cz);
-        cw = wave_xor_sum(cw);
-        if (lane == 0)
-            reinterpret_cast<uchar4*>(img)[ij] = env_finish(E, cx, cy, cz, cw, W, lr, cam, view, area[ij]);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < cnt) {
+            const uint32_t ij = heavy[e0 + lane * nwaves];
+            EnvPix E;
+            env_setup(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, K, E);
+            const float4 c4 = s_c[wslot][lane];
+            reinterpret_cast<uchar4*>(img)[ij] = env_finish(E, c4.x, c4.y, c4.z, c4.w, W, lr, cam, view, area[ij]);
+        }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -2535,29 +2817,31 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
     // each has latency-bound kernels (the lensed pixels' queues) that leave
     // the other room.  Joined before the composite.
     const bool overlap = f.star && f.map;
-    uint32_t *qlane = nullptr, *qwave = nullptr;
+    uint32_t *qgroup = nullptr, *qwave = nullptr;
     unsigned* nq = nullptr;
+    const float texel_size = BT_FPI / (float)s.rows;
+    const SkyK sky{reinterpret_cast<const float4*>(s.table), s.rows, s.cols, texel_size, 1.0 / (double)texel_size};
     if (f.map) {
         if ((rc = c->buffer("r_env_q", sizeof(uint32_t) * 2 * (NP + 64), &p))) return rc;
-        qlane = (uint32_t*)p;
+        qgroup = (uint32_t*)p;
         qwave = (uint32_t*)p + NP + 64;
-        if ((rc = c->buffer("r_env_qn", 64, &p))) return rc;
+        if ((rc = c->buffer("r_env_qn", sizeof(unsigned) * kEnvCtrWords, &p))) return rc;
         nq = (unsigned*)p;
     }
-    // distortEnvironmentMap: pixels with few sky columns inline and one lane
-    // each; then the wide ones, one wave each
+    // distortEnvironmentMap: pixels with few sky columns inline, those with
+    // more eight lanes each; then the wide ones, one wave each
     auto sky_light = [&](hipStream_t es) {
-        zero_u32_r<<<1, 64, 0, es>>>(nq, 2);
+        zero_u32_r<<<1, 64, 0, es>>>(nq, kEnvCtrWords);
         KTimer t(c, "env_map", es);
-        env_map<<<grid2d(W, H), blk, 0, es>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, area, v.view, img_map, qlane,
+        env_map<<<grid2d(W, H), blk, 0, es>>>(thphi, bh, sky, cam, W, H, f.offset, f.lr, area, v.view, img_map, qgroup,
                                               qwave, nq);
-        env_map_lane<<<(unsigned)c->num_cus * 8, 256, 0, es>>>(thphi, s, cam, W, f.offset, f.lr, area, v.view,
-                                                              img_map, qlane, nq);
+        env_map_group<<<(unsigned)c->num_cus * 4, 256, 0, es>>>(thphi, sky, cam, W, f.offset, f.lr, area, v.view,
+                                                               img_map, qgroup, nq + kCtrGroup);
     };
     auto sky_heavy = [&](hipStream_t es) {
         KTimer t(c, "env_heavy", es);
-        env_map_heavy<<<(unsigned)c->num_cus * 8, 256, 0, es>>>(thphi, s, cam, W, f.offset, f.lr, area, v.view,
-                                                               img_map, qwave, nq + 1);
+        env_map_heavy<<<(unsigned)c->num_cus * 8, 128, 0, es>>>(thphi, sky, cam, W, f.offset, f.lr, area, v.view,
+                                                               img_map, qwave, nq + kCtrHeavy);
     };
     auto join = [&]() -> hipError_t {
         const hipError_t e = hipEventRecord(c->ev_join, c->aux);
@@ -2577,9 +2861,10 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         StarQueue Q;
         if ((rc = c->buffer("r_star_lens", sizeof(float) * 3 * (NP + 64), &p))) return rc;
         Q.lens = (float*)p;
-        if ((rc = c->buffer("r_star_odd", sizeof(uint32_t) * 2 * (NP + 64), &p))) return rc;
+        if ((rc = c->buffer("r_star_odd", sizeof(uint32_t) * 3 * (NP + 64), &p))) return rc;
         Q.odd = (uint32_t*)p;
         Q.wide = Q.odd + NP + 64;
+        Q.oddc = Q.wide + NP + 64;
         if ((rc = c->buffer("r_star_q", sizeof(uint32_t) * 6 * (NP + 64), &p))) return rc;
         Q.pix = (uint32_t*)p;
         Q.cnt = Q.pix + NP + 64;
@@ -2603,7 +2888,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         Q.partial = (float*)p;
         zero_u32_r<<<1, 256, 0, c->stream>>>(Q.ctr, kStarCtrWords);
         const unsigned nwave = (unsigned)c->num_cus * 16, nred = (unsigned)c->num_cus * 4;
-        const unsigned ntree = (unsigned)c->num_cus * 2;
+        const unsigned ntree = (unsigned)c->num_cus * 4;
         const int tiles = NP >= (size_t(1) << 20) ? kScanTiles : 1;
         const dim3 gscan((unsigned)((W + 16 * tiles - 1) / (16 * tiles)), (unsigned)((H + 15) / 16));
         if (tf) {
@@ -2631,6 +2916,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             KTimer t1(c, "star_tree");                                                                      \
             star_wide<<<nred * 2 + ntree, 64, 0, c->stream>>> (thphi, s, cam, W, H, f.offset, Q, ntree);    \
             star_assign<<<nred, 256, 0, c->stream>>>(thphi, s, cam, W, H, f.offset, f.lr, area, v.view, Q); \
+            star_heads<(2 * S + 1) * (2 * S + 1) * 3><<<nred, 256, 0, c->stream>>>(thphi, cam, W, f.offset, Q); \
         }                                                                                                   \
         if (overlap) {                                                                                      \
             /* the odd pixels' chunks (few, long, latency-bound) on the auxiliary stream, between */       \

@@ -22,13 +22,22 @@ struct F2 {
     float x, y;
 };
 
-// float -> int as CUDA's cvt.rzi.s32.f32: truncate, saturate, NaN -> 0
-// (LLVM's fptosi is poison for NaN and out-of-range inputs).
+// float -> int as CUDA's cvt.rzi.s32.f32: truncate, saturate, NaN -> 0,
+// which is the conversion instruction's own behaviour (LLVM's fptosi is
+// poison for NaN and out-of-range inputs, so the cast alone will not do).
 __device__ __forceinline__ int cvt_i32(float x) {
-    if (!(x == x)) return 0;
-    if (x >= 2147483648.0f) return 2147483647;
-    if (x <= -2147483648.0f) return -2147483647 - 1;
-    return (int)x;
+    int r;
+    __asm__("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
+// fmodf(x, 2 pi) without the general reduction where it is one exact
+// subtraction at most (the remainder of x in [2 pi, 4 pi) is x - 2 pi, which
+// is exact).
+__device__ __forceinline__ float fmod_2pi(float x) {
+    if (x >= 0.f && x < BT_FPI2) return x;
+    if (x >= BT_FPI2 && x < 2.f * BT_FPI2) return x - BT_FPI2;
+    return fmodf(x, BT_FPI2);
 }
 
 __device__ __forceinline__ float f_sin(float x) { return (float)sin((double)x); }
@@ -65,17 +74,8 @@ __device__ inline float calc_area4(const float* t, const float* p) {
     return 2.f * (f_atan(triprod1 / dotpr1) + f_atan(triprod2 / dotpr2));
 }
 
-// kernel.cuh:612-649
-__device__ inline float calc_area3(float t0, float t1, float t2, float p0, float p1, float p2) {
-    const float t[3] = {t0, t1, t2}, p[3] = {p0, p1, p2};
-    float xi[3], yi[3], zi[3];
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-        float sint = f_sin(t[q]);
-        xi[q] = sint * f_cos(p[q]);
-        yi[q] = sint * f_sin(p[q]);
-        zi[q] = f_cos(t[q]);
-    }
+// kernel.cuh:612-649 from the corners' unit vectors
+__device__ __forceinline__ float area3_of(const float* xi, const float* yi, const float* zi) {
     float dot01 = xi[0] * xi[1] + yi[0] * yi[1] + zi[0] * zi[1];
     float dot02 = xi[0] * xi[2] + yi[0] * yi[2] + zi[0] * zi[2];
     float dot12 = xi[2] * xi[1] + yi[2] * yi[1] + zi[2] * zi[1];
@@ -98,6 +98,42 @@ __device__ inline float calc_area3(float t0, float t1, float t2, float p0, float
     float triprod1 = fabsf(x[0] * (y[1] * z[2] - y[2] * z[1]) - y[0] * (x[1] * z[2] - x[2] * z[1]) +
                            z[0] * (x[1] * y[2] - x[2] * y[1]));
     return 2.f * (f_atan(triprod1 / dotpr1));
+}
+
+struct HotTrig {
+    static __device__ __forceinline__ float s(float x) { return f_sin(x); }
+    static __device__ __forceinline__ float c(float x) { return f_cos(x); }
+};
+
+// kernel.cuh:612-649
+template <class Trig = HotTrig>
+__device__ __forceinline__ float calc_area3(float t0, float t1, float t2, float p0, float p1, float p2) {
+    const float t[3] = {t0, t1, t2}, p[3] = {p0, p1, p2};
+    float xi[3], yi[3], zi[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        float sint = Trig::s(t[q]);
+        xi[q] = sint * Trig::c(p[q]);
+        yi[q] = sint * Trig::s(p[q]);
+        zi[q] = Trig::c(t[q]);
+    }
+    return area3_of(xi, yi, zi);
+}
+
+// The solid angle of a quad as its two triangles (kernel.cuh:681-684), for
+// the rare pixel whose smoothed solid angle is zero.  Out of line, with the
+// trigonometric functions out of line in it: inlined, their twelve FP64
+// chains took 168 registers of every kernel that might need this, three
+// waves per SIMD where six to eight fit.
+__device__ __attribute__((noinline)) float sin_cold(float x) { return f_sin(x); }
+__device__ __attribute__((noinline)) float cos_cold(float x) { return f_cos(x); }
+struct ColdTrig {
+    static __device__ __forceinline__ float s(float x) { return sin_cold(x); }
+    static __device__ __forceinline__ float c(float x) { return cos_cold(x); }
+};
+__device__ __attribute__((noinline)) float quad_area_cold(float t0, float t1, float t2, float t3, float p0, float p1,
+                                                          float p2, float p3) {
+    return calc_area3<ColdTrig>(t0, t1, t2, p0, p1, p2) + calc_area3<ColdTrig>(t0, t2, t3, p0, p2, p3);
 }
 
 // kernel.cuh:274-295
@@ -133,14 +169,14 @@ __device__ __forceinline__ void pi_check_tot(F2* tp, float factor, int size) {
 
 // kernel.cuh:694-703
 __device__ __forceinline__ void wrap_to_pi(float& thetaW, float& phiW) {
-    thetaW = fmodf(thetaW, BT_FPI2);
+    thetaW = fmod_2pi(thetaW);
     while (thetaW < 0.f) thetaW += BT_FPI2;
     if (thetaW > BT_FPI) {
         thetaW -= 2.f * (thetaW - BT_FPI);
         phiW += BT_FPI;
     }
     while (phiW < 0.f) phiW += BT_FPI2;
-    phiW = fmodf(phiW, BT_FPI2);
+    phiW = fmod_2pi(phiW);
 }
 
 // kernel.cuh:790-815 (tension = bias = 0)
@@ -291,21 +327,27 @@ __device__ inline void hsp_to_rgb(float H, float S, float P, float& R, float& G,
     }
 }
 
-// kernel.cuh:348-365; cam = {speed, alpha, w, wbar, br, btheta, bphi}
+// kernel.cuh:348-365; cam = {speed, alpha, w, wbar, br, btheta, bphi}.  For a
+// camera on its orbit (br = btheta = 0, |speed| < 1, so that 1 - speed y > 0)
+// the x and z terms of phiFido are zeros added to the y term, which changes
+// nothing that follows: only the y direction's two sines are evaluated.
 __device__ inline float redshift(float theta, float phi, const float* cam) {
-    float xCam = f_sin(theta) * f_cos(phi);
-    float zCam = f_cos(theta);
+    const bool orbit = cam[4] == 0.f && cam[5] == 0.f && fabsf(cam[0]) < 1.f;
     float yCam = f_sin(theta) * f_sin(phi);
     float part = (1.f - cam[0] * yCam);
     float betaPart = sqrtf(1.f - cam[0] * cam[0]) / part;
-    float xFido = -sqrtf(1.f - cam[0] * cam[0]) * xCam / part;
-    float zFido = -sqrtf(1.f - cam[0] * cam[0]) * zCam / part;
     float yFido = (-yCam + cam[0]) / part;
-    float k = sqrtf(1.f - cam[5] * cam[5]);
-    float phiFido = -xFido * cam[4] / k + cam[6] * yFido + cam[6] * cam[5] / k * zFido;
+    float phiFido = cam[6] * yFido;
+    if (!orbit) {
+        float xCam = f_sin(theta) * f_cos(phi);
+        float zCam = f_cos(theta);
+        float xFido = -sqrtf(1.f - cam[0] * cam[0]) * xCam / part;
+        float zFido = -sqrtf(1.f - cam[0] * cam[0]) * zCam / part;
+        float k = sqrtf(1.f - cam[5] * cam[5]);
+        phiFido = -xFido * cam[4] / k + cam[6] * yFido + cam[6] * cam[5] / k * zFido;
+    }
     float eF = 1.f / (cam[1] + cam[2] * cam[3] * phiFido);
     float b = eF * cam[3] * phiFido;
-    (void)zFido;
     return 1.f / (betaPart * (1.f - b * cam[2]) / cam[1]);
 }
 
@@ -324,58 +366,48 @@ __device__ __forceinline__ bool star_in_polygon(const float* t, const float* p, 
            cross_ok(t[2], t[3], p[2], p[3], st, sp, sgn) && cross_ok(t[3], t[0], p[3], p[0], st, sp, sgn);
 }
 
-// kernel.cuh:112-200
+// kernel.cuh:112-200.  Each round halves the quad in both directions and
+// keeps the quarter the star lies in.  The new corners are selected, not
+// branched to: the lanes of a wave fall into all four quarters, and running
+// the four moves one after the other under masks took half of the round.
 __device__ inline void interpolate_star(float t0, float t1, float t2, float t3, float p0, float p1,
                                         float p2, float p3, float& start, float& starp, int sgn) {
-    float error = 0.00001f;
+    const float error = 0.00001f;
     float midT = (t0 + t1 + t2 + t3) * .25f;
     float midP = (p0 + p1 + p2 + p3) * .25f;
     float starInPixY = 0.5f;
     float starInPixX = 0.5f;
     float perc = 0.5f;
+    const bool flip = sgn < 0;
 #pragma unroll 1
     for (int q = 0; q < 10; q++) {
         if ((fabsf(start - midT) < error) && (fabsf(starp - midP) < error)) break;
-        float half01T = (t0 + t1) * .5f;
-        float half23T = (t2 + t3) * .5f;
-        float half12T = (t2 + t1) * .5f;
-        float half03T = (t0 + t3) * .5f;
-        float half01P = (p0 + p1) * .5f;
-        float half23P = (p2 + p3) * .5f;
-        float half12P = (p2 + p1) * .5f;
-        float half03P = (p0 + p3) * .5f;
-        float line01to23T = half23T - half01T;
-        float line03to12T = half12T - half03T;
-        float line01to23P = half23P - half01P;
-        float line03to12P = half12P - half03P;
-        float line01toStarT = start - half01T;
-        float line03toStarT = start - half03T;
-        float line01toStarP = starp - half01P;
-        float line03toStarP = starp - half03P;
-        int a = (((line03to12T * line03toStarP) - (line03toStarT * line03to12P)) > 0.f) ? 1 : -1;
-        int b = (((line01to23T * line01toStarP) - (line01toStarT * line01to23P)) > 0.f) ? 1 : -1;
+        const float half01T = (t0 + t1) * .5f, half23T = (t2 + t3) * .5f;
+        const float half12T = (t2 + t1) * .5f, half03T = (t0 + t3) * .5f;
+        const float half01P = (p0 + p1) * .5f, half23P = (p2 + p3) * .5f;
+        const float half12P = (p2 + p1) * .5f, half03P = (p0 + p3) * .5f;
+        const float line01to23T = half23T - half01T, line03to12T = half12T - half03T;
+        const float line01to23P = half23P - half01P, line03to12P = half12P - half03P;
+        const float line01toStarT = start - half01T, line03toStarT = start - half03T;
+        const float line01toStarP = starp - half01P, line03toStarP = starp - half03P;
+        // the sides of the two middle lines, seen with the quad's orientation
+        const bool A = ((line03to12T * line03toStarP) - (line03toStarT * line03to12P) > 0.f) != flip;
+        const bool B = ((line01to23T * line01toStarP) - (line01toStarT * line01to23P) > 0.f) != flip;
         perc *= 0.5f;
-        if (sgn * a > 0) {
-            if (sgn * b > 0) {
-                t2 = half12T; t0 = half01T; t3 = midT;
-                p2 = half12P; p0 = half01P; p3 = midP;
-                starInPixX -= perc; starInPixY -= perc;
-            } else {
-                t2 = midT; t1 = half01T; t3 = half03T;
-                p2 = midP; p1 = half01P; p3 = half03P;
-                starInPixX -= perc; starInPixY += perc;
-            }
-        } else {
-            if (sgn * b > 0) {
-                t1 = half12T; t3 = half23T; t0 = midT;
-                p1 = half12P; p3 = half23P; p0 = midP;
-                starInPixX += perc; starInPixY -= perc;
-            } else {
-                t0 = half03T; t1 = midT; t2 = half23T;
-                p0 = half03P; p1 = midP; p2 = half23P;
-                starInPixX += perc; starInPixY += perc;
-            }
-        }
+        starInPixX += A ? -perc : perc;
+        starInPixY += B ? -perc : perc;
+        const float a0 = B ? half01T : t0, a1 = B ? t1 : half01T, a2 = B ? half12T : midT, a3 = B ? midT : half03T;
+        const float c0 = B ? midT : half03T, c1 = B ? half12T : midT, c2 = B ? t2 : half23T, c3 = B ? half23T : t3;
+        t0 = A ? a0 : c0;
+        t1 = A ? a1 : c1;
+        t2 = A ? a2 : c2;
+        t3 = A ? a3 : c3;
+        const float b0 = B ? half01P : p0, b1 = B ? p1 : half01P, b2 = B ? half12P : midP, b3 = B ? midP : half03P;
+        const float d0 = B ? midP : half03P, d1 = B ? half12P : midP, d2 = B ? p2 : half23P, d3 = B ? half23P : p3;
+        p0 = A ? b0 : d0;
+        p1 = A ? b1 : d1;
+        p2 = A ? b2 : d2;
+        p3 = A ? b3 : d3;
         midT = (t0 + t1 + t2 + t3) * .25f;
         midP = (p0 + p1 + p2 + p3) * .25f;
     }
@@ -383,12 +415,21 @@ __device__ inline void interpolate_star(float t0, float t1, float t2, float t3, 
     starp = starInPixX;
 }
 
+// x / d for a constant d of inverse r, rounded as the division: the quotient
+// estimate, its remainder and one correction.  (Checked against the division
+// over every significand for the two constants below.)
+__device__ __forceinline__ float div_by(float x, float d, float r) {
+    const float q = x * r;
+    return fmaf(fmaf(-q, d, x), r, q);
+}
+
 // kernel.cuh:335-338.  FP32 expf (within 1 ulp): the star taps' sums are
 // compared with a relative tolerance, and this is evaluated 9-49 times per
 // star.
 __device__ __forceinline__ float gaussian(float dist) {
-    float sigma = 1.f / 2.5f;
-    return expf(-.5f * dist / (sigma * sigma)) * 1.f / (sigma * BT_SQRT2PI);
+    constexpr float sigma = 1.f / 2.5f;
+    constexpr float var = sigma * sigma, norm = sigma * BT_SQRT2PI;
+    return div_by(expf(div_by(-.5f * dist, var, 1.f / var)), norm, 1.f / norm);
 }
 
 }  // namespace rdr
