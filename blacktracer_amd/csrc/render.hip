@@ -69,98 +69,110 @@ __device__ F2 interpolate_linear(float percDown, float percRight, const F2* c) {
 
 // The reference's findPoint may recurse once into interpolateHermite
 // (count 0 -> 1) and never deeper; the two levels are written out here.
-__device__ F2 interpolate_hermite_l1(const GridV& g, int i, int j, int gap, float percDown,
+__device__ __attribute__((noinline)) F2 interpolate_hermite_l1(const GridV& g, int i, int j, int gap, float percDown,
                                      float percRight, F2* c);
 
-// kernel.cuh:817-889 for recursion depth `count`.
-template <int COUNT>
-__device__ F2 find_point(const GridV& g, int i, int j, int offver, int offhor, int gap) {
-    const int GM = g.GM, GN = g.GN;
-    F2 gridpt = g.at(i, j);
-    if (gridpt.x == -2 && gridpt.y == -2) {
-        int j2 = (j + offhor * gap + GM) % GM;
-        int i2 = i + offver * gap;
-        F2 ij2 = g.at(i2, j2);
-        if (ij2.x == -1 && ij2.y == -1) return F2{-1, -1};
-        if (ij2.x != -2 && ij2.y != -2) {
-            int j0 = (j - offhor * gap + GM) % GM;
-            int i0 = (i - offver * gap);
-            F2 ij0 = g.at(i0, j0);
-            if (ij0.x < 0) return F2{-1, -1};
-            int jprev = (j - 3 * offhor * gap + GM) % GM;
-            int jnext = (j + 3 * offhor * gap + GM) % GM;
-            int iprev = i - offver * 3 * gap;
-            int inext = i + offver * 3 * gap;
-            if (offver != 0) {
-                if (i2 == 0) {
-                    jnext = (j0 + GM / 2) % GM;
-                    inext = i0;
-                } else if (i0 == GN - 1) {
-                    jprev = (j0 + GM / 2) % GM;
-                    iprev = i2;
-                } else if (i2 == GN - 1) {
-                    inext = i0;
-                    jnext = (j0 + GM / 2) % GM;
-                }
-            }
-            F2 ijprev = g.at(iprev, jprev);
-            F2 ijnext = g.at(inext, jnext);
-            if (ijprev.x > -2 && ijnext.x > -2) {
-                F2 pt[4] = {ijprev, ij0, ij2, ijnext};
-                if (pt[0].x != -1 && pt[3].x != -1) {
-                    pi_check_tot(pt, 0.2f, 4);
-                    return hermite(0.5f, pt[0], pt[1], pt[2], pt[3]);
-                }
-            }
-            F2 pt[2] = {ij2, ij0};
-            pi_check_tot(pt, 0.2f, 2);
-            return F2{.5f * (pt[0].x + pt[1].x), .5f * (pt[0].y + pt[1].y)};
-        }
-        if (COUNT > 0) return F2{-1.f, -1.f};
-        int j0 = (j + gap) % GM;
-        int j1 = (j - gap + GM) % GM;
-        if (i - gap < 0) return F2{-1, -1};
-        F2 cc[12];
-        cc[0] = g.at(i + gap, j0);
-        cc[1] = g.at(i - gap, j0);
-        cc[2] = g.at(i - gap, j1);
-        cc[3] = g.at(i + gap, j1);
-        for (int q = 0; q < 4; q++)
-            if (cc[q].x == -1 || cc[q].x == -2) return F2{-1, -1};
-        return interpolate_hermite_l1(g, i - gap, j1, 2 * gap, .5f, .5f, cc);
-    }
-    return gridpt;
+// x % GM of a column index x < 4 GM (a negative x stays, as with %).
+__device__ __forceinline__ int wrap_col(int x, int GM) {
+    while (x >= GM) x -= GM;
+    return x;
 }
 
-// kernel.cuh:891-938 for recursion depth COUNT.
+// kernel.cuh:817-889 for recursion depth `count`, for a point (i, j) that the
+// grid does not hold.  Out of line: most points are held, and the eight
+// copies of this in every interpolation were larger than the instruction
+// cache.
 template <int COUNT>
-__device__ F2 interpolate_hermite(const GridV& g, int i, int j, int gap, float percDown,
-                                  float percRight, F2* c) {
+__device__ __attribute__((noinline)) F2 find_missing(GridV g, int i, int j, int offver, int offhor, int gap) {
+    const int GM = g.GM, GN = g.GN;
+    int j2 = wrap_col(j + offhor * gap + GM, GM);
+    int i2 = i + offver * gap;
+    F2 ij2 = g.at(i2, j2);
+    if (ij2.x == -1 && ij2.y == -1) return F2{-1, -1};
+    if (ij2.x != -2 && ij2.y != -2) {
+        int j0 = wrap_col(j - offhor * gap + GM, GM);
+        int i0 = (i - offver * gap);
+        F2 ij0 = g.at(i0, j0);
+        if (ij0.x < 0) return F2{-1, -1};
+        int jprev = wrap_col(j - 3 * offhor * gap + GM, GM);
+        int jnext = wrap_col(j + 3 * offhor * gap + GM, GM);
+        int iprev = i - offver * 3 * gap;
+        int inext = i + offver * 3 * gap;
+        if (offver != 0) {
+            if (i2 == 0) {
+                jnext = wrap_col(j0 + GM / 2, GM);
+                inext = i0;
+            } else if (i0 == GN - 1) {
+                jprev = wrap_col(j0 + GM / 2, GM);
+                iprev = i2;
+            } else if (i2 == GN - 1) {
+                inext = i0;
+                jnext = wrap_col(j0 + GM / 2, GM);
+            }
+        }
+        F2 ijprev = g.at(iprev, jprev);
+        F2 ijnext = g.at(inext, jnext);
+        if (ijprev.x > -2 && ijnext.x > -2) {
+            F2 pt[4] = {ijprev, ij0, ij2, ijnext};
+            if (pt[0].x != -1 && pt[3].x != -1) {
+                pi_check_tot(pt, 0.2f, 4);
+                return hermite(0.5f, pt[0], pt[1], pt[2], pt[3]);
+            }
+        }
+        F2 pt[2] = {ij2, ij0};
+        pi_check_tot(pt, 0.2f, 2);
+        return F2{.5f * (pt[0].x + pt[1].x), .5f * (pt[0].y + pt[1].y)};
+    }
+    if (COUNT > 0) return F2{-1.f, -1.f};
+    int j0 = wrap_col(j + gap, GM);
+    int j1 = wrap_col(j - gap + GM, GM);
+    if (i - gap < 0) return F2{-1, -1};
+    F2 cc[12];
+    cc[0] = g.at(i + gap, j0);
+    cc[1] = g.at(i - gap, j0);
+    cc[2] = g.at(i - gap, j1);
+    cc[3] = g.at(i + gap, j1);
+    for (int q = 0; q < 4; q++)
+        if (cc[q].x == -1 || cc[q].x == -2) return F2{-1, -1};
+    return interpolate_hermite_l1(g, i - gap, j1, 2 * gap, .5f, .5f, cc);
+}
+
+// kernel.cuh:891-938 for recursion depth COUNT.  The eight outer points load
+// together; the missing ones are then looked for.
+template <int COUNT>
+__device__ __forceinline__ F2 interpolate_hermite(const GridV& g, int i, int j, int gap, float percDown,
+                                                  float percRight, F2* c) {
     const int GM = g.GM, GN = g.GN;
     int k = i + gap;
-    int l = (j + gap) % GM;
+    int l = wrap_col(j + gap, GM);
     int imin1 = i - gap;
     int kplus1 = k + gap;
-    int jmin1 = (j - gap + GM) % GM;
-    int lplus1 = (l + gap) % GM;
+    int jmin1 = wrap_col(j - gap + GM, GM);
+    int lplus1 = wrap_col(l + gap, GM);
     int jx = j, jy = j, lx = l, ly = l;
     if (i == 0) {
-        jx = (j + GM / 2) % GM;
-        lx = (jx + gap) % GM;
+        jx = wrap_col(j + GM / 2, GM);
+        lx = wrap_col(jx + gap, GM);
         imin1 = k;
     } else if (k == GN - 1) {
-        jy = (j + GM / 2) % GM;
-        ly = (jy + gap) % GM;
+        jy = wrap_col(j + GM / 2, GM);
+        ly = wrap_col(jy + gap, GM);
         kplus1 = i;
     }
-    c[4] = find_point<COUNT>(g, i, jmin1, 0, -1, gap);
-    c[5] = find_point<COUNT>(g, i, lplus1, 0, 1, gap);
-    c[6] = find_point<COUNT>(g, k, jmin1, 0, -1, gap);
-    c[7] = find_point<COUNT>(g, k, lplus1, 0, 1, gap);
-    c[8] = find_point<COUNT>(g, imin1, jx, -1, 0, gap);
-    c[9] = find_point<COUNT>(g, imin1, lx, -1, 0, gap);
-    c[10] = find_point<COUNT>(g, kplus1, jy, 1, 0, gap);
-    c[11] = find_point<COUNT>(g, kplus1, ly, 1, 0, gap);
+    const int pi[8] = {i, i, k, k, imin1, imin1, kplus1, kplus1};
+    const int pj[8] = {jmin1, lplus1, jmin1, lplus1, jx, lx, jy, ly};
+    bool missing = false;
+#pragma unroll
+    for (int q = 0; q < 8; q++) c[4 + q] = g.at(pi[q], pj[q]);
+#pragma unroll
+    for (int q = 0; q < 8; q++) missing = missing || (c[4 + q].x == -2 && c[4 + q].y == -2);
+    if (missing) {
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            if (c[4 + q].x == -2 && c[4 + q].y == -2)
+                c[4 + q] = find_missing<COUNT>(g, pi[q], pj[q], q < 4 ? 0 : q < 6 ? -1 : 1,
+                                               q >= 4 ? 0 : q % 2 ? 1 : -1, gap);
+    }
     for (int q = 4; q < 12; q++)
         if (c[q].x == -1) return interpolate_linear(percDown, percRight, c);
     pi_check_tot(c, 0.2f, 12);
@@ -171,8 +183,8 @@ __device__ F2 interpolate_hermite(const GridV& g, int i, int j, int gap, float p
     return hermite(percDown, upup, up, down, downdown);
 }
 
-__device__ F2 interpolate_hermite_l1(const GridV& g, int i, int j, int gap, float percDown,
-                                     float percRight, F2* c) {
+__device__ __attribute__((noinline)) F2 interpolate_hermite_l1(const GridV& g, int i, int j, int gap, float percDown,
+                                                               float percRight, F2* c) {
     return interpolate_hermite<1>(g, i, j, gap, percDown, percRight, c);
 }
 
@@ -200,7 +212,7 @@ __device__ F2 interpolate_pix(const GridV& g, float theta, float phi, int gridlv
     int l = b + gap;
     float factor = BT_FPI2 / (1.f * GM);
     float thetaUp = factor * a, phiLeft = factor * b, thetaDown = factor * k, phiRight = factor * l;
-    l = l % GM;
+    l = wrap_col(l, GM);
     F2 c[12];
     c[0] = g.at(a, b);
     c[1] = g.at(a, l);
@@ -434,7 +446,43 @@ __device__ __forceinline__ bool corners(const float* thphi, int W, int ind, floa
     return true;
 }
 
-__global__ __launch_bounds__(256) void bh_area(const float* thphi, int W, int H, uint8_t* bh, float* area) {
+// Unit vectors of the (16 + 1) x (16 + 1) corners of a 16 x 16 tile of
+// quads, in LDS: four quads share a corner, and its FP64 sines and cosines
+// are most of the work on a solid angle.
+struct TileVec {
+    float x[17 * 17], y[17 * 17], z[17 * 17];
+    __device__ __forceinline__ void set(int c, float t, float p) {
+        const float sint = f_sin(t);
+        x[c] = sint * f_cos(p);
+        y[c] = sint * f_sin(p);
+        z[c] = f_cos(t);
+    }
+    __device__ __forceinline__ void get(const int* c, float* xi, float* yi, float* zi, int n) const {
+        for (int q = 0; q < n; q++) {
+            xi[q] = x[c[q]];
+            yi[q] = y[c[q]];
+            zi[q] = z[c[q]];
+        }
+    }
+};
+
+// Shadow flag and celestial solid angle (findBlackPixels + findArea).  The
+// pixel across phi = 2 pi, whose corners pi_check moves, makes its own
+// vectors.  Also clears the counters of the star and sky queues of the frame.
+__global__ __launch_bounds__(256) void bh_area(const float* thphi, int W, int H, uint8_t* bh, float* area,
+                                               unsigned* ctr, int nctr) {
+    __shared__ TileVec V;
+    const int tid = threadIdx.y * 16 + threadIdx.x;
+    if (blockIdx.x == 0 && blockIdx.y == 0)
+        for (int k = tid; k < nctr; k += 256) ctr[k] = 0u;
+    const float2* tp = reinterpret_cast<const float2*>(thphi);
+    for (int c = tid; c < 17 * 17; c += 256) {
+        const int ci = blockIdx.y * 16 + c / 17, cj = blockIdx.x * 16 + c % 17;
+        if (ci > H || cj > W) continue;
+        const float2 v = tp[(size_t)ci * (W + 1) + cj];
+        if (!(v.x < 0 || v.y < 0)) V.set(c, v.x, fmod_2pi(v.y + 0.0f));
+    }
+    __syncthreads();
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     int i = blockIdx.y * blockDim.y + threadIdx.y;
     if (i >= H || j >= W) return;
@@ -443,8 +491,19 @@ __global__ __launch_bounds__(256) void bh_area(const float* thphi, int W, int H,
     bool ok = corners(thphi, W, i * (W + 1) + j, t, p, pc, 0.0f);
     size_t ij = (size_t)i * W + j;
     bh[ij] = ok ? 0 : 1;
-    area[ij] = ok ? calc_area3(t[0], t[1], t[2], p[0], p[1], p[2]) + calc_area3(t[0], t[2], t[3], p[0], p[2], p[3])
-                  : 0.f;
+    float a = 0.f;
+    if (ok && pc) {
+        a = quad_area_cold(t[0], t[1], t[2], t[3], p[0], p[1], p[2], p[3]);
+    } else if (ok) {
+        const int o = threadIdx.y * 17 + threadIdx.x;
+        const int c0[3] = {o + 17, o, o + 1}, c1[3] = {o + 17, o + 1, o + 18};
+        float x[3], y[3], z[3];
+        V.get(c0, x, y, z, 3);
+        a = area3_of(x, y, z);
+        V.get(c1, x, y, z, 3);
+        a = a + area3_of(x, y, z);
+    }
+    area[ij] = a;
 }
 
 __device__ __forceinline__ int filter_size(const int* gap, int W, int i, int j) {
@@ -471,7 +530,9 @@ __global__ __launch_bounds__(256) void smooth_h(const float* area, const uint8_t
     float sum = 0.f;
     int count = 0;
     for (int h = -fs; h <= fs; h++) {
-        int jj = ((j + h) % W + W) % W;
+        int jj = j + h;
+        while (jj < 0) jj += W;   // at most one step unless the filter is wider than the frame
+        while (jj >= W) jj -= W;
         if (bh[(size_t)i * W + jj] == 0) {
             sum += area[(size_t)i * W + jj];
             count++;
@@ -523,15 +584,24 @@ __device__ void lensing_redshift(const float* t, const float* p, int W, int ind,
 // The camera-sky solid angle of every pixel's view quad (the pixArea of
 // kernel.cuh:679-680): it depends on the view alone, so a view makes it once.
 __global__ __launch_bounds__(256) void view_pixel_areas(const float* view, int W, int H, float* out) {
+    __shared__ TileVec V;
+    const int M1 = W + 1;
+    const float2* v = reinterpret_cast<const float2*>(view);
+    for (int c = threadIdx.y * 16 + threadIdx.x; c < 17 * 17; c += 256) {
+        const int ci = blockIdx.y * 16 + c / 17, cj = blockIdx.x * 16 + c % 17;
+        if (ci > H || cj > W) continue;
+        const float2 d = v[(size_t)ci * M1 + cj];
+        V.set(c, d.x, d.y);
+    }
+    __syncthreads();
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     const int i = blockIdx.y * blockDim.y + threadIdx.y;
     if (i >= H || j >= W) return;
-    const int M1 = W + 1, ind = i * M1 + j;
-    const float2* v = reinterpret_cast<const float2*>(view);
-    float2 v0 = v[ind], v1 = v[ind + 1], v2 = v[ind + M1 + 1], v3 = v[ind + M1];
-    float ver4[4] = {v0.x, v1.x, v2.x, v3.x};
-    float hor4[4] = {v0.y, v1.y, v2.y, v3.y};
-    out[(size_t)i * W + j] = calc_area4(ver4, hor4);
+    const int o = threadIdx.y * 17 + threadIdx.x;
+    const int c4[4] = {o, o + 1, o + 18, o + 17};
+    float x[4], y[4], z[4];
+    V.get(c4, x, y, z, 4);
+    out[(size_t)i * W + j] = area4_of(x, y, z);
 }
 
 // ---- star pass ---------------------------------------------------------
@@ -1743,7 +1813,10 @@ __global__ __launch_bounds__(256) void star_sum(const float* taps, const uint8_t
     const float factor = 20.f;
     for (int u = start; u <= stop; u++)
         for (int v = 0; v <= 2 * STEP; v++) {
-            size_t src = (size_t)(i + u - STEP) * W + ((j + v - STEP + W) % W);
+            int jj = j + v - STEP;
+            while (jj < 0) jj += W;   // one step unless the frame is narrower than the splat
+            while (jj >= W) jj -= W;
+            size_t src = (size_t)(i + u - STEP) * W + jj;
             if (lit[src] == kDark) continue;   // its taps are zero (and not stored)
             int tap = FW * FW - (FW * u + v + 1);
             br += factor * taps[(size_t)(tap * 3 + 0) * NP + src];
@@ -2349,6 +2422,12 @@ __global__ __launch_bounds__(256) void env_map(const float* thphi, const uint8_t
     reinterpret_cast<uchar4*>(img)[ij] = o;
 }
 
+// The block's place in an order in which the blocks of one XCD (blocks go to
+// the eight XCDs in turn) are neighbours: neighbouring pixels of a queue read
+// the same sky rows, and then find them in their XCD's L2.  The grid is a
+// multiple of 8 blocks.
+__device__ __forceinline__ unsigned xcd_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
+
 // Sixteen lanes per queued pixel: a lane takes every sixteenth column
 // boundary, the running span (an exact min/max) is scanned over the lanes,
 // the sixteen columns' loads are in flight together, and their terms, staged
@@ -2382,7 +2461,7 @@ __global__ __launch_bounds__(256) void env_map_group(const float* thphi, SkyK K,
     const unsigned rounds = min(64u / kGroupPix, max(1u, n / (kGroupPix * nwaves)));
     const unsigned per = rounds * kGroupPix;   // pixels a wave takes at a time
     const int cols = K.cols;
-    for (unsigned e0 = (blockIdx.x * 4 + wslot) * per; e0 < n; e0 += nwaves * per) {
+    for (unsigned e0 = (xcd_block() * 4 + wslot) * per; e0 < n; e0 += nwaves * per) {
         for (unsigned r = 0; r < rounds; r++) {
             const unsigned e = e0 + r * kGroupPix + grp;
             int num = -1;   // last boundary; -1: nothing to do here
@@ -2469,8 +2548,8 @@ __global__ __launch_bounds__(128) void env_map_heavy(const float* thphi, SkyK K,
     __shared__ float4 s_c[2][64];
     __shared__ float4 s_d[2][kHeavyWindow];
     const unsigned lane = threadIdx.x & 63, wslot = threadIdx.x >> 6;
-    const unsigned wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const unsigned nwaves = (gridDim.x * blockDim.x) >> 6;
+    const unsigned wave = xcd_block() * 2 + wslot;
+    const unsigned nwaves = gridDim.x * 2;
     const unsigned n = *nheavy;
     const int rows = K.rows, cols = K.cols;
     // pixel wave + k nwaves is the wave's k-th
@@ -2490,10 +2569,11 @@ __global__ __launch_bounds__(128) void env_map_heavy(const float* thphi, SkyK K,
                 float cmn = cols + 1, cmx = -100;      // the span after the boundaries so far
                 int col = (E.pixMin + (int)lane) % cols;
                 for (int w0 = 0; w0 < nb; w0 += kHeavyWindow) {
-#pragma unroll 4
-                    for (int b0 = 0; b0 < kHeavyWindow; b0 += 64) {
-                        if (w0 + b0 >= nb) break;
-                        const int b = w0 + b0 + (int)lane;
+                    for (int b4 = 0; b4 < kHeavyWindow && w0 + b4 < nb; b4 += 256) {
+                      int ihi[4], ilo[4];
+#pragma unroll
+                      for (int u = 0; u < 4; u++) {
+                        const int b = w0 + b4 + 64 * u + (int)lane;
                         float mn = cols + 1, mx = -100;
                         if (b < nb) env_boundary(E, (E.pixMin + b) * K.pixSize, mn, mx);
                         // inclusive scan over the rows of 16, then over the rows
@@ -2512,11 +2592,20 @@ __global__ __launch_bounds__(128) void env_map_heavy(const float* thphi, SkyK K,
                         mx = fmaxf(fmaxf(mx, cmx), row == 0 ? mx : row == 1 ? x0 : row == 2 ? x01 : x02);
                         cmn = fminf(cmn, fminf(n02, n3));
                         cmx = fmaxf(cmx, fmaxf(x02, x3));
-                        float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
-                        if (b > 0 && b < nb) d = env_column(K, col, mn, mx);
+                        ihi[u] = ilo[u] = -1;
+                        if (b > 0 && b < nb) env_ends(K, col, mn, mx, ihi[u], ilo[u]);
                         col += 64;
                         while (col >= cols) col -= cols;
-                        s_d[wslot][b0 + lane] = d;
+                      }
+                      float4 x[4], y[4];
+#pragma unroll
+                      for (int u = 0; u < 4; u++) {
+                        x[u] = y[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                        if (ihi[u] >= 0) x[u] = K.table[ihi[u]];
+                        if (ilo[u] >= 0) y[u] = K.table[ilo[u]];
+                      }
+#pragma unroll
+                      for (int u = 0; u < 4; u++) s_d[wslot][b4 + 64 * u + lane] = env_diff(x[u], y[u]);
                     }
                     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -2650,10 +2739,6 @@ __global__ void grid_to_f32(const double* cel, int GN, int GM, int sym, int GN1,
     }
 }
 
-__global__ void zero_u32_r(unsigned* p, int n) {
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
-}
-
 // The pixels that one lane each traces: those of few candidates, then the
 // odd ones among them.
 int few_span(size_t NP) {
@@ -2759,6 +2844,10 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
     if ((rc = c->buffer("r_img_map", 4 * NP, &p))) return rc;
     uint8_t* img_map = (uint8_t*)p;
 
+    // the counters of the star and the sky queues, cleared by bh_area
+    if ((rc = c->buffer("r_queue_ctr", sizeof(unsigned) * (kStarCtrWords + kEnvCtrWords), &p))) return rc;
+    unsigned* ctr = (unsigned*)p;
+
     Cam7 cam;
     for (int q = 0; q < 7; q++) cam.v[q] = cam7[q];
     {
@@ -2804,7 +2893,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
     }
     {
         KTimer t(c, "bh_area");
-        bh_area<<<grid2d(W, H), blk, 0, c->stream>>>(thphi, W, H, bh, area);
+        bh_area<<<grid2d(W, H), blk, 0, c->stream>>>(thphi, W, H, bh, area, ctr, kStarCtrWords + kEnvCtrWords);
     }
     {
         KTimer t(c, "smooth");
@@ -2825,13 +2914,11 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         if ((rc = c->buffer("r_env_q", sizeof(uint32_t) * 2 * (NP + 64), &p))) return rc;
         qgroup = (uint32_t*)p;
         qwave = (uint32_t*)p + NP + 64;
-        if ((rc = c->buffer("r_env_qn", sizeof(unsigned) * kEnvCtrWords, &p))) return rc;
-        nq = (unsigned*)p;
+        nq = ctr + kStarCtrWords;
     }
     // distortEnvironmentMap: pixels with few sky columns inline, those with
     // more eight lanes each; then the wide ones, one wave each
     auto sky_light = [&](hipStream_t es) {
-        zero_u32_r<<<1, 64, 0, es>>>(nq, kEnvCtrWords);
         KTimer t(c, "env_map", es);
         env_map<<<grid2d(W, H), blk, 0, es>>>(thphi, bh, sky, cam, W, H, f.offset, f.lr, area, v.view, img_map, qgroup,
                                               qwave, nq);
@@ -2876,8 +2963,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         Q.rcap = (unsigned)(NP / 4 + 65536);
         if ((rc = c->buffer("r_star_ranges", sizeof(int2) * (size_t)Q.rcap, &p))) return rc;
         Q.ranges = (int2*)p;
-        if ((rc = c->buffer("r_star_qn", sizeof(unsigned) * kStarCtrWords, &p))) return rc;
-        Q.ctr = (unsigned*)p;
+        Q.ctr = ctr;
         if ((rc = c->buffer("r_star_lit", NP, &p))) return rc;
         Q.lit = (uint8_t*)p;
         const int NT = fw * fw * 3;
@@ -2886,15 +2972,13 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         Q.cap = (unsigned)(NP + 64);
         if ((rc = c->buffer("r_star_part", sizeof(float) * NT * (size_t)Q.cap, &p))) return rc;
         Q.partial = (float*)p;
-        zero_u32_r<<<1, 256, 0, c->stream>>>(Q.ctr, kStarCtrWords);
         const unsigned nwave = (unsigned)c->num_cus * 16, nred = (unsigned)c->num_cus * 4;
         const unsigned ntree = (unsigned)c->num_cus * 4;
         const int tiles = NP >= (size_t(1) << 20) ? kScanTiles : 1;
         const dim3 gscan((unsigned)((W + 16 * tiles - 1) / (16 * tiles)), (unsigned)((H + 15) / 16));
         if (tf) {
-            // with both passes on, the trails go first on the auxiliary stream:
-            // the main stream waits there (after the odd chunks) before the
-            // chunk reduction, and so before star_sum reads the trails
+            // with both passes on, the trails go first on the auxiliary stream;
+            // the main stream waits for them before star_sum reads them
             const hipStream_t ts = overlap ? c->aux : c->stream;
             KTimer t(c, "trails", ts);
             const TrailK& T = tf->k;
@@ -2904,6 +2988,11 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             trail_cache<<<(unsigned)((T.S + 255) / 256), 256, 0, ts>>>(T, W);
             trail_lines<<<(unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(T, cam, T.grad, W, H);
             BT_HIP(hipGetLastError());
+            if (overlap) BT_HIP(hipEventRecord(c->ev_back, ts));
+        }
+        if (overlap) {
+            sky_light(c->aux);
+            sky_heavy(c->aux);
         }
 #define BT_STAR_LAUNCH(S)                                                                                    \
     {                                                                                                       \
@@ -2918,29 +3007,14 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             star_assign<<<nred, 256, 0, c->stream>>>(thphi, s, cam, W, H, f.offset, f.lr, area, v.view, Q); \
             star_heads<(2 * S + 1) * (2 * S + 1) * 3><<<nred, 256, 0, c->stream>>>(thphi, cam, W, f.offset, Q); \
         }                                                                                                   \
-        if (overlap) {                                                                                      \
-            /* the odd pixels' chunks (few, long, latency-bound) on the auxiliary stream, between */       \
-            /* the sky pass's light and heavy kernels, beside the other chunks */                           \
-            BT_HIP(hipEventRecord(c->ev_hand, c->stream));                                                  \
-            sky_light(c->aux);                                                                              \
-            BT_HIP(hipStreamWaitEvent(c->aux, c->ev_hand, 0));                                              \
-            star_rest<S>(c, c->aux, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);               \
-            star_map_chunk<S, true><<<nred, 256, 0, c->aux>>>(thphi, bh, s, cam, W, H, f.offset, f.lr,      \
-                                                              area, v.view, taps, Q);                       \
-            BT_HIP(hipEventRecord(c->ev_back, c->aux));                                                     \
-            sky_heavy(c->aux);                                                                              \
-        }                                                                                                   \
         {                                                                                                   \
             KTimer t2(c, "star_chunk");                                                                     \
-            star_map_chunk<S, false><<<nwave, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr,  \
+            star_map_chunk<S, false><<<nwave, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, \
                                                                    area, v.view, taps, Q);                  \
-            if (!overlap) {                                                                                 \
-                star_rest<S>(c, c->stream, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);        \
-                star_map_chunk<S, true><<<nred, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset,     \
-                                                                     f.lr, area, v.view, taps, Q);          \
-            }                                                                                               \
+            star_map_chunk<S, true><<<nred, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr,   \
+                                                                 area, v.view, taps, Q);                    \
         }                                                                                                   \
-        if (overlap) BT_HIP(hipStreamWaitEvent(c->stream, c->ev_back, 0));                                  \
+        star_rest<S>(c, c->stream, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);                      \
         KTimer t3(c, "star_reduce");                                                                        \
         star_chunk_reduce<S><<<nwave, 256, 0, c->stream>>>(W, H, taps, Q);                                  \
     }
@@ -2958,6 +3032,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             if ((rc = c->buffer("r_diff_light", sizeof(float) * 3 * NP * 2, &p))) return rc;
             light = (float*)p;
         }
+        if (tf && overlap) BT_HIP(hipStreamWaitEvent(c->stream, c->ev_back, 0));
         {
             KTimer t(c, "star_sum");
             float* ostar = diffract ? light : (dbg ? dbg->star : nullptr);

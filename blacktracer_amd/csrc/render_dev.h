@@ -50,16 +50,8 @@ __device__ __forceinline__ float f_exp(float x) { return (float)exp((double)x); 
 __device__ __forceinline__ float f_log10(float x) { return (float)log10((double)x); }
 __device__ __forceinline__ float f_exp10(float x) { return (float)pow(10.0, (double)x); }
 
-// kernel.cuh:586-610
-__device__ inline float calc_area4(const float* t, const float* p) {
-    float x[4], y[4], z[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        float sint = f_sin(t[q]);
-        x[q] = sint * f_cos(p[q]);
-        y[q] = sint * f_sin(p[q]);
-        z[q] = f_cos(t[q]);
-    }
+// kernel.cuh:586-610 from the corners' unit vectors
+__device__ __forceinline__ float area4_of(const float* x, const float* y, const float* z) {
     float dotpr1 = 1.f;
     dotpr1 += x[0] * x[2] + y[0] * y[2] + z[0] * z[2];
     float dotpr2 = dotpr1;
@@ -72,6 +64,19 @@ __device__ inline float calc_area4(const float* t, const float* p) {
     float triprod2 = fabsf(x[0] * (y[2] * z[3] - y[3] * z[2]) - y[0] * (x[2] * z[3] - x[3] * z[2]) +
                            z[0] * (x[2] * y[3] - x[3] * y[2]));
     return 2.f * (f_atan(triprod1 / dotpr1) + f_atan(triprod2 / dotpr2));
+}
+
+// kernel.cuh:586-610
+__device__ inline float calc_area4(const float* t, const float* p) {
+    float x[4], y[4], z[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        float sint = f_sin(t[q]);
+        x[q] = sint * f_cos(p[q]);
+        y[q] = sint * f_sin(p[q]);
+        z[q] = f_cos(t[q]);
+    }
+    return area4_of(x, y, z);
 }
 
 // kernel.cuh:612-649 from the corners' unit vectors
