@@ -599,7 +599,7 @@ __device__ void lensing_redshift(const float* t, const float* p, int W, int ind,
     float2 v0 = v[ind], v1 = v[ind + 1], v2 = v[ind + M1 + 1], v3 = v[ind + M1];
     float ver4[4] = {v0.x, v1.x, v2.x, v3.x};
     float hor4[4] = {v0.y, v1.y, v2.y, v3.y};
-    // calc_area4 of these corners, made once per view (view_pixel_areas)
+    // area4_of these corners, made once per view (view_pixel_areas)
     const int pi = ind / M1, pj = ind - pi * M1;
     const float pixArea = cam.pix_area[(size_t)pi * W + pj];
     frac = pixArea / solidAngle;
@@ -749,8 +749,10 @@ __device__ __forceinline__ void node_range(const int32_t* tree, int node, int& b
 // called for every listed node in the reference's list order.  The node's
 // rectangle is held in scalars (0: theta, 1: phi), not in arrays indexed by
 // the level's axis, which would live in scratch memory.
-template <class F>
-__device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn, const float* mx, F&& visit) {
+// The walk ends early once done() holds.
+template <class F, class D>
+__device__ void search_tree_until(const int32_t* tree, int treeLevel, const float* mn, const float* mx, F&& visit,
+                                  D&& done) {
     float start0 = 0.f, start1 = 0.f, size0 = BT_FPI, size1 = BT_FPI2;
     int node = 0;
     unsigned bitMask = 1u << treeLevel;
@@ -782,6 +784,7 @@ __device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn,
             if (list) {
                 if (rd) visit(node * 2 + 2);
                 if (lu) visit(node * 2 + 1);
+                if (done()) return;
                 node = node * 2 + 1;
                 break;
             } else {
@@ -808,6 +811,11 @@ __device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn,
             else start0 += size0;
         }
     }
+}
+
+template <class F>
+__device__ void search_tree(const int32_t* tree, int treeLevel, const float* mn, const float* mx, F&& visit) {
+    search_tree_until(tree, treeLevel, mn, mx, visit, [] { return false; });
 }
 
 __device__ __forceinline__ int bin_of(float v, float d, int n) { return min(max(cvt_i32(v / d), 0), n - 1); }
@@ -1961,50 +1969,127 @@ __global__ __launch_bounds__(256) void trail_grad(const float* thphi, int W, int
     grad[2 * ((size_t)i * M1 + j) + 1] = gy;
 }
 
-// The images of this frame: per pixel with starsToCheck < S/100
-// (MakeImageKernel.cu:273-282,301), every star inside its quad, with the
-// quantities addTrails uses (part, frac, blackbody index).
-__global__ __launch_bounds__(256) void trail_hits(const float* thphi, const uint8_t* bh, SceneK s, Cam7 cam,
-                                                  int W, int H, float offset, int lr, const float* area,
-                                                  const float* view, TrailK T) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = blockIdx.y * blockDim.y + threadIdx.y;
-    if (i >= H || j >= W) return;
-    StarPix P;
-    if (!star_pixel(thphi, bh, W, i, j, offset, lr, area, view, cam, P)) return;
+// One image: star q of the scene, the slot-th one of its images.
+__device__ __forceinline__ void trail_record(const TrailK& T, const StarPix& P, int q, unsigned slot, float2 mg,
+                                             uint32_t pix) {
+    if (slot >= (unsigned)kTrailHits) {
+        atomicAdd(&T.stats[1], 1u);
+        return;
+    }
+    float temp = 46.f / P.redshft * ((1.f / ((0.92f * mg.y) + 1.7f)) + (1.f / ((0.92f * mg.y) + 0.62f))) - 10.f;
+    const int index = max(0, min(cvt_i32(floorf(temp)), 390));
+    const size_t h = (size_t)q * kTrailHits + slot;
+    T.hit_pix[h] = pix;
+    T.hit_data[3 * h] = mg.x + P.red;
+    T.hit_data[3 * h + 1] = P.frac;
+    T.hit_data[3 * h + 2] = (float)index;
+}
+
+// Largest star tree (level 10), held in LDS for the walks.
+constexpr int kTreeWords = (1 << 11) - 1;
+
+// Whether the pixel's starsToCheck (MakeImageKernel.cu:273-282) stays below
+// S/100: the walk of the star tree ends once it does not.
+__device__ bool trail_pixel(const SceneK& s, const StarPix& P) {
     int starsToCheck = 0;
-    search_tree(s.tree, s.tree_level, P.mn, P.mx, [&](int node) {
-        int b, e;
-        node_range(s.tree, node, b, e);
-        starsToCheck += e - b;
-    });
-    if (!(starsToCheck < s.S / 100)) return;
-    const uint32_t pix = (uint32_t)i * (uint32_t)W + (uint32_t)j;
-    // candidates as in the star pass: the binned stars of the quad's rows
-    // (tree order for quads across phi = 2 pi); the same stars test inside
+    search_tree_until(
+        s.tree, s.tree_level, P.mn, P.mx,
+        [&](int node) {
+            int b, e;
+            node_range(s.tree, node, b, e);
+            starsToCheck += e - b;
+        },
+        [&] { return starsToCheck >= s.S / 100; });
+    return starsToCheck < s.S / 100;
+}
+
+// The images among candidates b + first, b + first + step, .. below e: as in
+// the star pass, binned stars, or tree order for quads across phi = 2 pi.
+__device__ __forceinline__ void trail_range(const TrailK& T, const SceneK& s, const StarPix& P, uint32_t ij, int b,
+                                            int e, int first, int step) {
     const float* pos = P.picheck ? s.star_pos : s.bin_pos;
     const float* magv = P.picheck ? s.star_mag : s.bin_mag;
-    for_ranges(P, s, [&](int b, int e) {
-        for (int k = b; k < e; k++) {
-            float st, sp;
-            if (!star_test(P, pos, k, st, sp)) continue;
-            const int q = P.picheck ? k : s.bin_idx[k];
-            const float2 mg = reinterpret_cast<const float2*>(magv)[k];
-            const float part = mg.x + P.red;
-            float temp = 46.f / P.redshft * ((1.f / ((0.92f * mg.y) + 1.7f)) + (1.f / ((0.92f * mg.y) + 0.62f))) - 10.f;
-            const int index = max(0, min(cvt_i32(floorf(temp)), 390));
-            const unsigned slot = atomicAdd(&T.nhits[q], 1u);
-            if (slot < (unsigned)kTrailHits) {
-                const size_t h = (size_t)q * kTrailHits + slot;
-                T.hit_pix[h] = pix;
-                T.hit_data[3 * h] = part;
-                T.hit_data[3 * h + 1] = P.frac;
-                T.hit_data[3 * h + 2] = (float)index;
-            } else {
-                atomicAdd(&T.stats[1], 1u);
-            }
+    for (int k = b + first; k < e; k += step) {
+        float st, sp;
+        if (!star_test(P, pos, k, st, sp)) continue;
+        const int q = P.picheck ? k : s.bin_idx[k];
+        trail_record(T, P, q, atomicAdd(&T.nhits[q], 1u), reinterpret_cast<const float2*>(magv)[k], ij);
+    }
+}
+
+// The images of this frame: per pixel with starsToCheck < S/100
+// (MakeImageKernel.cu:273-282,301), every star inside its quad, with the
+// quantities addTrails uses (part, frac, blackbody index).  Runs after the
+// star pass has sorted the pixels: one that is kDark has no star inside.
+// trail_hits does the kFew pixels, gathered in LDS from a span of the frame so
+// that full waves walk the star tree (from LDS) and lens; trail_queued the
+// queued ones, whose lensing star_assign has stored, sixteen lanes to a
+// pixel's candidates.  Most pixels hold no star: a lane per pixel of the
+// frame, walking the tree for each, took 980 us at 1366 x 768 with 100000
+// stars.
+__global__ __launch_bounds__(256) void trail_hits(const float* thphi, SceneK s, Cam7 cam, int W, int H, float offset,
+                                                  int lr, const float* area, const float* view, TrailK T,
+                                                  const uint8_t* lit, int span) {
+    __shared__ int32_t s_tree[kTreeWords];
+    __shared__ uint16_t s_list[kFewSpan];
+    __shared__ unsigned s_n;
+    const size_t NP = (size_t)W * H;
+    const size_t p0 = (size_t)blockIdx.x * span;
+    const int words = (2 << s.tree_level) - 1;
+    if (threadIdx.x == 0) s_n = 0;
+    for (int k = threadIdx.x; k < words; k += 256) s_tree[k] = s.tree[k];
+    __syncthreads();
+    for (int k = 0; k < span; k += 256) {
+        const size_t p = p0 + k + threadIdx.x;
+        if (p < NP && lit[p] == kFew) s_list[atomicAdd(&s_n, 1u)] = (uint16_t)(k + threadIdx.x);
+    }
+    __syncthreads();
+    s.tree = s_tree;
+    for (unsigned t = threadIdx.x; t < s_n; t += 256) {
+        const size_t ij = p0 + s_list[t];
+        const int i = (int)(ij / (size_t)W), j = (int)(ij % (size_t)W);
+        StarPix P;
+        star_pixel_geom(thphi, W, i, j, offset, cam, P);
+        if (!trail_pixel(s, P)) continue;
+        star_lens(W, ij, i * (W + 1) + j, lr, area, view, cam, P);
+        for_ranges(P, s, [&](int b, int e) { trail_range(T, s, P, (uint32_t)ij, b, e, 0, 1); });
+    }
+}
+
+__global__ __launch_bounds__(256) void trail_queued(const float* thphi, SceneK s, Cam7 cam, int W, float offset,
+                                                    TrailK T, StarQueue Q) {
+    __shared__ int32_t s_tree[kTreeWords];
+    const int words = (2 << s.tree_level) - 1;
+    for (int k = threadIdx.x; k < words; k += 256) s_tree[k] = s.tree[k];
+    __syncthreads();
+    s.tree = s_tree;
+    const unsigned n = Q.ctr[kCtrQueued];
+    const unsigned lane = __lane_id(), wave = blockIdx.x * 4 + threadIdx.x / 64;
+    StarPix P;
+    for (unsigned e0 = wave * 16; e0 < n; e0 += gridDim.x * 4 * 16) {
+        bool pass = false;
+        if (lane < 16 && e0 + lane < n && Q.cnt[e0 + lane]) {
+            const uint32_t ij = Q.pix[e0 + lane];
+            star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
+            pass = trail_pixel(s, P);
         }
-    });
+        unsigned todo = (unsigned)__ballot(pass);
+        // four of the pixels at a time, sixteen lanes each
+        while (todo) {
+            unsigned m = todo;
+            for (unsigned g = 0; g < lane / 16; g++) m &= m - 1;
+            if (m) {
+                const unsigned k = e0 + (unsigned)__ffs((int)m) - 1;
+                const uint32_t ij = Q.pix[k];
+                star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
+                P.frac = Q.lens[3 * k];
+                P.redshft = Q.lens[3 * k + 1];
+                P.red = Q.lens[3 * k + 2];
+                for_ranges(P, s, [&](int b, int e) { trail_range(T, s, P, ij, b, e, (int)(lane & 15), 16); });
+            }
+            for (int g = 0; g < 4; g++) todo &= todo - 1;
+        }
+    }
 }
 
 // Per star: its images in pixel order; the first kTrailNum become this
@@ -2129,14 +2214,34 @@ __global__ __launch_bounds__(256) void trail_lines(TrailK T, Cam7 cam, const flo
 // whose sprite window covers it, in ascending pixel order, so the sums do
 // not depend on scheduling (the reference adds with float atomics).
 
-// Per frame row, the columns of its bright pixels in ascending order and
-// their light over the reference's divisor 10000 * max^0.6 (one wavefront
-// per row).
+// Columns per entry of the bright pixels' index (a tile's width).
+constexpr int kDiffCols = 16;
+// Black texels around the sprite: a wave's 8 x 8 pixels reach at most seven
+// beyond a window that covers one of them.
+constexpr int kDiffPad = 8;
+
+// Per frame row, the columns of its bright pixels in ascending order, their
+// light over the reference's divisor 10000 * max^0.6, and how many of them lie
+// left of every kDiffCols-th column (`left`, one entry more than the row has
+// such groups); one wavefront per row.  Also the sprite with four bytes a
+// texel, which one load reads, inside a black margin of kDiffPad texels.
 __global__ __launch_bounds__(256) void diff_rows(const float* light, int W, int H, uint32_t* cols, float* scaled,
-                                                 int* nrow) {
+                                                 int* left, const uint8_t* sprite, int fs, uint32_t* sprite4) {
+    const int pitch = fs + 2 * kDiffPad;
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < pitch * pitch; t += (int)gridDim.x * 256) {
+        const int y = t / pitch - kDiffPad, x = t % pitch - kDiffPad;
+        uint32_t v = 0;
+        if (x >= 0 && x < fs && y >= 0 && y < fs) {
+            const uint8_t* p = sprite + 3 * (y * fs + x);
+            v = (uint32_t)p[0] | (uint32_t)p[1] << 8 | (uint32_t)p[2] << 16;
+        }
+        sprite4[t] = v;
+    }
     const int row = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
     if (row >= H) return;
     const unsigned lane = threadIdx.x & 63;
+    const int groups = (W + kDiffCols - 1) / kDiffCols;
+    int* lrow = left + (size_t)row * (groups + 1);
     int n = 0;
     for (int j0 = 0; j0 < W; j0 += 64) {
         const int j = j0 + (int)lane;
@@ -2151,8 +2256,10 @@ __global__ __launch_bounds__(256) void diff_rows(const float* light, int W, int 
             hot = mx > 65025.f;
         }
         const unsigned long long m = __ballot(hot);
+        const int at = n + __popcll(m & ((1ull << lane) - 1));
+        if (lane % kDiffCols == 0 && j < W) lrow[j / kDiffCols] = at;
         if (hot) {
-            const size_t o = (size_t)row * W + n + __popcll(m & ((1ull << lane) - 1));
+            const size_t o = (size_t)row * W + at;
             const float div = 10000 * f_pow(mx, 0.6f);
             cols[o] = (uint32_t)j;
             scaled[3 * o] = l0 / div;
@@ -2161,123 +2268,168 @@ __global__ __launch_bounds__(256) void diff_rows(const float* light, int W, int 
         }
         n += __popcll(m);
     }
-    if (lane == 0) nrow[row] = n;
+    if (lane == 0) lrow[groups] = n;
 }
 
 constexpr int kDiffCand = 512;   // bright pixels staged in LDS per round
+constexpr int kDiffFly = 8;      // candidates whose sprite texels load together
 
-// One 16 x 16 tile of output pixels per workgroup: lane 0 lists, in pixel
-// order, the bright pixels whose window can reach the tile; every thread
-// then adds the ones whose window covers its pixel.
-__global__ __launch_bounds__(256) void diff_gather(const float* light, float* acc, const uint32_t* cols,
-                                                   const float* scaled, const int* nrow, const uint8_t* sprite, int fs,
-                                                   int W, int H) {
-    __shared__ int c_r[kDiffCand], c_c[kDiffCand], c_x0[kDiffCand], c_x1[kDiffCand];
-    __shared__ float c_l[kDiffCand][3];
-    __shared__ int s_n, s_row, s_k, s_done;
+// One 16 x 16 tile of output pixels per workgroup.  The bright pixels whose
+// window can reach the tile are, in each row, one or (across the frame's
+// edge) two runs of its list, which `left` bounds: a thread per row takes the
+// runs, their lengths are summed over the rows, and the threads then fetch the
+// candidates by their number, which is their pixel order.  A wave has 8 x 8
+// pixels, keeps the candidates whose window reaches those, and every lane adds
+// them all, kDiffFly sprite loads in flight: where the window does not cover
+// its pixel it reads the sprite's black margin and adds zero (with a light
+// that is no finite number, which times zero is NaN, it tests instead).  The
+// window's rows outside the frame are those of no pixel.  What bounds it is
+// the arithmetic of the tiles among the brightest pixels (up to 2800
+// candidates a tile at 1366 x 768, 340 on average).  (One wave listing row after row, and two integer remainders per
+// candidate and pixel, took 1180 us there.)
+__global__ __launch_bounds__(256) void diff_gather(const float* light, const uint32_t* cols, const float* scaled,
+                                                   const int* left, const uint32_t* sprite4, int fs, int W, int H,
+                                                   uint8_t* img, float* o_star) {
+    __shared__ float4 c_light[kDiffCand + 1];   // light, and the tile's first pixel's texel
+    __shared__ short2 c_win[kDiffCand];         // that pixel's row and column of the window
+    __shared__ __align__(16) uint16_t s_list[4][kDiffCand + kDiffFly];
+    __shared__ int s_pre[257], s_first[256], s_len0[256], s_second[256], s_wave[4];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid / 64;
+    const int wx = 8 * (wave & 1), wy = 8 * (wave / 2);
+    const int tx = wx + (lane & 7), ty = wy + lane / 8;
     const int oj0 = blockIdx.x * 16, oi0 = blockIdx.y * 16;
-    const int oj = oj0 + (int)threadIdx.x, oi = oi0 + (int)threadIdx.y;
-    const int tid = threadIdx.y * 16 + threadIdx.x;
+    const int oj = oj0 + tx, oi = oi0 + ty;
+    const int pitch = fs + 2 * kDiffPad;
+    const unsigned texel = (unsigned)(ty * pitch + tx);
     const int fh = fs / 2;
+    uint16_t* list = s_list[wave];
+    if (tid == 0) c_light[kDiffCand] = make_float4(0.f, 0.f, 0.f, 0.f);   // adds nothing
+    const int groups = (W + kDiffCols - 1) / kDiffCols;
     const bool mine = oi < H && oj < W;
+    const size_t ij = (size_t)oi * W + oj;
     float a0 = 0.f, a1 = 0.f, a2 = 0.f;
     if (mine) {
-        const float* l = light + 3 * ((size_t)oi * W + oj);
-        a0 = l[0];
-        a1 = l[1];
-        a2 = l[2];
+        a0 = light[3 * ij];
+        a1 = light[3 * ij + 1];
+        a2 = light[3 * ij + 2];
     }
+    // columns whose windows can reach the tile: c0 .. c1, c1 beyond W where they wrap
+    const bool whole = 15 + fs >= W;
+    int c0 = oj0 - (fs - 1 - fh);
+    if (c0 < 0) c0 += W;
+    const int c1 = c0 + 14 + fs;
+    const bool wrap = c1 >= W;
+    const int g0 = c0 / kDiffCols, g1 = (wrap ? c1 - W : c1) / kDiffCols + 1;
     // rows whose windows can reach the tile
     const int r_lo = max(0, oi0 - (fs - 1 - fh)), r_hi = min(H - 1, oi0 + 15 + fh);
-    if (tid == 0) {
-        s_row = r_lo;
-        s_k = 0;
-        s_done = 0;
-    }
-    __syncthreads();
-    while (true) {
-        if (tid < 64) {
-            // wavefront 0 lists the next candidates in pixel order, 64 row
-            // entries at a time (a ballot keeps their order)
-            int n = 0, r = s_row, k = s_k;
-            const unsigned lane = (unsigned)tid;
-            while (r <= r_hi) {
-                const int nr = nrow[r];
-                if (k >= nr) {
-                    r++;
-                    k = 0;
-                    continue;
-                }
-                const int kk = k + (int)lane;
-                bool take = false;
-                int c = 0;
-                if (kk < nr) {
-                    c = (int)cols[(size_t)r * W + kk];
-                    // the window's columns c - fh .. c - fh + fs - 1 (mod W) against the tile's
-                    const int e = ((c - fh - oj0) % W + W) % W;
-                    take = e <= 15 || e >= W - fs + 1;
-                }
-                const unsigned long long m = __ballot(take);
-                if (n + __popcll(m) > kDiffCand) break;   // the rest in the next round
-                if (take) {
-                    const int d = n + __popcll(m & ((1ull << lane) - 1));
-                    int startx = 0, endx = fs;
-                    if (r < fh) startx = fh - r;
-                    if (r > (H - fh)) endx = H - r + fh;
-                    const float* l = scaled + 3 * ((size_t)r * W + kk);
-                    c_r[d] = r;
-                    c_c[d] = c;
-                    c_x0[d] = startx;
-                    c_x1[d] = endx;
-                    c_l[d][0] = l[0];
-                    c_l[d][1] = l[1];
-                    c_l[d][2] = l[2];
-                }
-                n += __popcll(m);
-                k += 64;
-            }
-            if (lane == 0) {
-                s_n = n;
-                s_row = r;
-                s_k = k;
-                s_done = r > r_hi;
+    for (int rb = r_lo; rb <= r_hi; rb += 256) {
+        int first = 0, len0 = 0, second = 0, len = 0;
+        if (rb + tid <= r_hi) {
+            const int* lrow = left + (size_t)(rb + tid) * (groups + 1);
+            if (whole || (wrap && g1 >= g0)) {
+                len0 = len = lrow[groups];
+            } else if (wrap) {
+                len0 = lrow[g1];
+                second = lrow[g0];
+                len = len0 + lrow[groups] - second;
+            } else {
+                first = lrow[g0];
+                len0 = len = lrow[g1] - first;
             }
         }
+        int sum = len;   // inclusive over the wave, then over the workgroup
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int up = __shfl_up(sum, d);
+            if (lane >= d) sum += up;
+        }
+        __syncthreads();   // the last batch's runs are no longer read
+        if (lane == 63) s_wave[wave] = sum;
+        s_first[tid] = first;
+        s_len0[tid] = len0;
+        s_second[tid] = second;
         __syncthreads();
-        const int n = s_n;
-        if (mine) {
-            for (int k = 0; k < n; k++) {
-                const int qq = oi - (c_r[k] - fh);
-                if (qq < c_x0[k] || qq >= c_x1[k]) continue;
-                const int pp = ((oj - c_c[k] + fh) % W + W) % W;
-                if (pp >= fs) continue;
-                const uint8_t* sp = sprite + 3 * ((size_t)qq * fs + pp);
-                const float dx = c_l[k][0] * (float)sp[0], dy = c_l[k][1] * (float)sp[1], dz = c_l[k][2] * (float)sp[2];
+        for (int w = 0; w < wave; w++) sum += s_wave[w];
+        s_pre[tid + 1] = sum;
+        if (tid == 0) s_pre[0] = 0;
+        __syncthreads();
+        const int total = s_pre[256];
+        for (int x0 = 0; x0 < total; x0 += kDiffCand) {
+            const int n = min(kDiffCand, total - x0);
+            bool tame = true;
+            for (int k = tid; k < n; k += 256) {
+                const int x = x0 + k;
+                int row = 0;   // the last one with s_pre[row] <= x
+#pragma unroll
+                for (int d = 128; d > 0; d /= 2)
+                    if (s_pre[row + d] <= x) row += d;
+                const int at = x - s_pre[row];
+                const int r = rb + row;
+                const size_t o = (size_t)r * W + (at < s_len0[row] ? s_first[row] + at : s_second[row] + at - s_len0[row]);
+                const int qq = oi0 - r + fh;
+                int pp = oj0 - (int)cols[o] + fh;
+                if (pp < 0) pp += W;
+                if (pp >= W) pp -= W;
+                if (pp >= W - 15) pp -= W;   // reaches the tile from its left only
+                pp = min(pp, fs);
+                const float* l = scaled + 3 * o;
+                c_win[k] = make_short2((short)qq, (short)pp);
+                c_light[k] = make_float4(l[0], l[1], l[2], __int_as_float((qq + kDiffPad) * pitch + pp + kDiffPad));
+                tame = tame && fabsf(l[0]) <= 3.4e38f && fabsf(l[1]) <= 3.4e38f && fabsf(l[2]) <= 3.4e38f;
+            }
+            tame = __syncthreads_and(tame);
+            int m = 0;
+            for (int k0 = 0; k0 < n; k0 += 64) {
+                const int k = k0 + lane;
+                bool reach = false;
+                if (k < n) {
+                    const short2 w = c_win[k];
+                    reach = w.x + wy + 7 >= 0 && w.x + wy < fs && w.y + wx + 7 >= 0 && w.y + wx < fs;
+                }
+                const unsigned long long b = __ballot(reach);
+                if (reach) list[m + __popcll(b & ((1ull << lane) - 1))] = (uint16_t)k;
+                m += __popcll(b);
+            }
+            if (lane < kDiffFly) list[m + lane] = kDiffCand;
+            __builtin_amdgcn_wave_barrier();
+            const auto add = [&](const float4& l, uint32_t px) {
+                const float dx = l.x * (float)(px & 255u), dy = l.y * (float)(px >> 8 & 255u),
+                            dz = l.z * (float)(px >> 16 & 255u);
                 a0 += fminf(65025.f, dx * dx);
                 a1 += fminf(65025.f, dy * dy);
                 a2 += fminf(65025.f, dz * dz);
+            };
+            if (tame) {
+                for (int k = 0; k < m; k += kDiffFly) {
+                    uint32_t px[kDiffFly];
+                    float4 l[kDiffFly];
+#pragma unroll
+                    for (int u = 0; u < kDiffFly; u++) {
+                        l[u] = c_light[list[k + u]];
+                        px[u] = sprite4[(unsigned)__float_as_int(l[u].w) + texel];
+                    }
+#pragma unroll
+                    for (int u = 0; u < kDiffFly; u++) add(l[u], px[u]);
+                }
+            } else {
+                for (int k = 0; k < m; k++) {
+                    const short2 w = c_win[list[k]];
+                    const float4 l = c_light[list[k]];
+                    if ((unsigned)(w.x + ty) < (unsigned)fs && (unsigned)(w.y + tx) < (unsigned)fs)
+                        add(l, sprite4[(unsigned)__float_as_int(l.w) + texel]);
+                }
             }
+            __syncthreads();
         }
-        const int done = s_done;
-        __syncthreads();
-        if (done) break;
     }
-    if (mine) {
-        float* o = acc + 3 * ((size_t)oi * W + oj);
-        o[0] = a0;
-        o[1] = a1;
-        o[2] = a2;
+    if (!mine) return;
+    make_pix(a0, a1, a2, img, ij);
+    if (o_star) {
+        o_star[3 * ij] = a0;
+        o_star[3 * ij + 1] = a1;
+        o_star[3 * ij + 2] = a2;
     }
-}
-
-__global__ __launch_bounds__(256) void copy_f32(const float* src, float* dst, int64_t n) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[t] = src[t];
-}
-
-__global__ __launch_bounds__(256) void make_pix_all(const float* light, int64_t NP, uint8_t* img) {
-    const int64_t ij = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ij < NP) make_pix(light[3 * ij], light[3 * ij + 1], light[3 * ij + 2], img, (size_t)ij);
 }
 
 // ---- distortEnvironmentMap (MakeImageKernel.cu:631-751) ----
@@ -3116,27 +3268,37 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         // through; from four million pixels on, where the sky pass is the
         // longer one, the one-lane pixels stay on the main stream (3840x2160:
         // 1322 against 1401 us; 1920x1080 the other way round, 883 against 855).
-        const bool few_on_main = !overlap || NP >= (size_t(1) << 22);
+        // Trails fill the auxiliary stream: the odd chunks stay on the main one
+        // too then.
+        const bool few_on_main = !overlap || tf || NP >= (size_t(1) << 22);
         const unsigned ntree = (unsigned)c->num_cus * 4;
         const int tiles = NP >= (size_t(1) << 20) ? kScanTiles : 1;
         const dim3 gscan((unsigned)((W + 16 * tiles - 1) / (16 * tiles)), (unsigned)((H + 15) / 16));
         if (tf) {
-            // with both passes on, the trails go first on the auxiliary stream;
-            // the main stream waits for that one before star_sum reads them
+            // with both passes on, the trails are made on the auxiliary
+            // stream, their images once the pixels are sorted; the main stream
+            // waits for that one before star_sum reads them
             const hipStream_t ts = overlap ? c->aux : c->stream;
             KTimer t(c, "trails", ts);
             const TrailK& T = tf->k;
             trail_clear<<<(unsigned)c->num_cus * 4, 256, 0, ts>>>(T, tf->first ? 1 : 0, 3 * NP);
             trail_grad<<<grid2d(W + 1, H + 1), blk, 0, ts>>>(thphi, W, H, T.grad);
-            trail_hits<<<grid2d(W, H), blk, 0, ts>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, area, v.view, T);
-            trail_cache<<<(unsigned)((T.S + 255) / 256), 256, 0, ts>>>(T, W);
-            trail_lines<<<(unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(T, cam, T.grad, W, H);
             BT_HIP(hipGetLastError());
         }
         if (overlap) {
             sky_light(c->aux);
             sky_heavy(c->aux);
         }
+        const auto trail_images = [&](hipStream_t ts) {
+            KTimer t(c, "trail_images", ts);
+            const TrailK& T = tf->k;
+            const int span = std::max(256, few_span(NP) / 4);
+            trail_hits<<<(unsigned)((NP + span - 1) / span), 256, 0, ts>>>(thphi, s, cam, W, H, f.offset, f.lr, area,
+                                                                           v.view, T, Q.lit, span);
+            trail_queued<<<(unsigned)c->num_cus * 4, 256, 0, ts>>>(thphi, s, cam, W, f.offset, T, Q);
+            trail_cache<<<(unsigned)((T.S + 255) / 256), 256, 0, ts>>>(T, W);
+            trail_lines<<<(unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(T, cam, T.grad, W, H);
+        };
 #define BT_STAR_LAUNCH(S)                                                                                    \
     {                                                                                                       \
         {                                                                                                   \
@@ -3160,8 +3322,9 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             star_map_chunk<S, false><<<nwave, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, \
                                                                    area, v.view, taps, Q);                  \
         }                                                                                                   \
-        star_map_chunk<S, true><<<nred, 256, 0, rs>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, area, v.view,\
-                                                      taps, Q);                                             \
+        if (tf) trail_images(rs);                                                                           \
+        star_map_chunk<S, true><<<nred, 256, 0, tf ? c->stream : rs>>>(thphi, bh, s, cam, W, H, f.offset,   \
+                                                                       f.lr, area, v.view, taps, Q);        \
         star_rest<S>(c, few_on_main ? c->stream : rs, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);   \
         if (overlap) {                                                                                      \
             BT_HIP(hipEventRecord(c->ev_back, rs));                                                         \
@@ -3181,7 +3344,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         const bool diffract = tf && tf->sprite;
         float* light = nullptr;
         if (diffract) {
-            if ((rc = c->buffer("r_diff_light", sizeof(float) * 3 * NP * 2, &p))) return rc;
+            if ((rc = c->buffer("r_diff_light", sizeof(float) * 3 * NP, &p))) return rc;
             light = (float*)p;
         }
         {
@@ -3198,17 +3361,16 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         BT_HIP(hipGetLastError());
         if (diffract) {
             KTimer t(c, "diffraction");
-            float* acc = light + 3 * NP;
-            if ((rc = c->buffer("r_diff_rows", sizeof(uint32_t) * 4 * NP + sizeof(int) * (size_t)H, &p))) return rc;
+            const size_t nleft = (size_t)H * ((W + kDiffCols - 1) / kDiffCols + 1), npad = (size_t)tf->fs + 2 * kDiffPad;
+            if ((rc = c->buffer("r_diff_rows", sizeof(uint32_t) * (4 * NP + nleft + npad * npad), &p))) return rc;
             uint32_t* cols = (uint32_t*)p;
             float* scaled = reinterpret_cast<float*>(cols + NP);
-            int* nrow = reinterpret_cast<int*>(cols + 4 * NP);
-            const unsigned b3 = (unsigned)((3 * NP + 255) / 256), b1 = (unsigned)((NP + 255) / 256);
-            diff_rows<<<(unsigned)((H + 3) / 4), 256, 0, c->stream>>>(light, W, H, cols, scaled, nrow);
-            diff_gather<<<grid2d(W, H), blk, 0, c->stream>>>(light, acc, cols, scaled, nrow, tf->sprite, tf->fs, W,
-                                                             H);
-            make_pix_all<<<b1, 256, 0, c->stream>>>(acc, (int64_t)NP, img_star);
-            if (dbg && dbg->star) copy_f32<<<b3, 256, 0, c->stream>>>(acc, dbg->star, (int64_t)(3 * NP));
+            int* left = reinterpret_cast<int*>(cols + 4 * NP);
+            uint32_t* sprite4 = cols + 4 * NP + nleft;
+            diff_rows<<<(unsigned)((H + 3) / 4), 256, 0, c->stream>>>(light, W, H, cols, scaled, left, tf->sprite,
+                                                                      tf->fs, sprite4);
+            diff_gather<<<grid2d(W, H), 256, 0, c->stream>>>(light, cols, scaled, left, sprite4, tf->fs, W, H,
+                                                             img_star, dbg ? dbg->star : nullptr);
             BT_HIP(hipGetLastError());
         }
         return BT_OK;

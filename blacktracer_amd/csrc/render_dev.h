@@ -66,19 +66,6 @@ __device__ __forceinline__ float area4_of(const float* x, const float* y, const 
     return 2.f * (f_atan(triprod1 / dotpr1) + f_atan(triprod2 / dotpr2));
 }
 
-// kernel.cuh:586-610
-__device__ inline float calc_area4(const float* t, const float* p) {
-    float x[4], y[4], z[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        float sint = f_sin(t[q]);
-        x[q] = sint * f_cos(p[q]);
-        y[q] = sint * f_sin(p[q]);
-        z[q] = f_cos(t[q]);
-    }
-    return area4_of(x, y, z);
-}
-
 // kernel.cuh:612-649 from the corners' unit vectors
 __device__ __forceinline__ float area3_of(const float* xi, const float* yi, const float* zi) {
     float dot01 = xi[0] * xi[1] + yi[0] * yi[1] + zi[0] * zi[1];
