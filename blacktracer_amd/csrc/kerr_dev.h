@@ -54,6 +54,13 @@ struct SharedDiv {
         e = fma(-den, r, 1.0);
         y = fma(r, e, r);
     }
+    // For a product of factors whose reciprocals are at hand: est, the product
+    // of those, is 1 / den to a relative error of at most 2^-40 or so, and one
+    // refinement squares that, far below the rounding it ends with, as the
+    // two refinements of the hardware's estimate (2^-24 or better) do.
+    __device__ __forceinline__ SharedDiv(double den, double est) : d(den) {
+        y = fma(est, fma(-den, est, 1.0), est);
+    }
     // d > 0.  The remainder is taken as d q - x (the negated x - d q, exact),
     // which gives a zero x's quotient the sign x / d has.
     __device__ __forceinline__ double pos(double x) const {
@@ -68,6 +75,13 @@ struct SharedDiv {
         return copysign(fma(fma(-d, q, x), y, q), q);
     }
 };
+
+// 1 / x to about twice the bits of the hardware's estimate: a factor of the
+// estimates that SharedDiv(den, est) refines.
+__device__ __forceinline__ double rcp_once(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    return fma(r, fma(-x, r, 1.0), r);
+}
 
 // R(r) of Metric.h:96-98 with P and Delta of Metric.h:64-66,92-94.
 __device__ __forceinline__ double Rfun(double a, double asq, double r, double b, double q) {
@@ -220,46 +234,52 @@ __device__ __forceinline__ bool check_celest(const PoseK& P, double pR, double b
     return check2 || check3;
 }
 
-// Metric.h:198-226.  v = (r, theta, phi, pR, pTheta).  Every operation is
-// the reference's, in its order; the sixteen divisions run through
-// SharedDiv, fourteen of them sharing five reciprocals (rosq, sinsq,
-// rosq 2 delta, rosqsq and sqrosqdel; the denominators rosq * 2 * delta and
-// rosq * (2 * delta) are the same double, and x / (2 rosq) is half of
-// x / rosq exactly).
+// Metric.h:198-226.  v = (r, theta, phi, pR, pTheta).  Every rounding is the
+// reference's, in its order.  Its factors 2 and 4 are powers of two, which no
+// rounding sees: where numerator and denominator of a quotient hold the same
+// one it is left out of both (2a P - (2a - 2b) delta + 2b cos^2 delta / sin^2
+// over 2 rho^2 delta, 4 p^2 r over (2 rho^2)^2, (4r - 4) x over
+// rho^2 (2 delta)^2), which saves a dozen of about 215 operations; so does
+// partR, the bracket of R.  The sixteen divisions run through SharedDiv.  Its
+// denominators are products of rho^2, delta and sin theta: three hardware
+// reciprocals (each worth four FMAs of issue) and a refinement per product
+// serve the seven of them.
 __device__ __forceinline__ void derivs(double a, double asq, const double* v, double* o,
                                        double b, double q) {
     const double r = v[0], pr = v[3], pt = v[4];
     double sinv, cosv;
     sincos(v[1], &sinv, &cosv);
-    double cossq = sq(cosv);
-    double sinsq = sq(sinv);
-    double bsq = sq(b);
-    double delta = sq(r) - 2. * r + asq;
-    double rosq = sq(r) + asq * cossq;
-    double P = sq(r) + asq - a * b;
-    double prsq = sq(pr);
-    double pthetasq = sq(pt);
-    double R = sq(P) - delta * (sq((b - a)) + q);
-    double partR = (q + sq(a - b));
-    const SharedDiv by_rosq(rosq), by_sinsq(sinsq);
+    const double cossq = sq(cosv);
+    const double sinsq = sq(sinv);
+    const double bsq = sq(b);
+    const double rsq = sq(r), twor = 2. * r;
+    const double delta = rsq - twor + asq;
+    const double rosq = rsq + asq * cossq;
+    const double P = rsq + asq - a * b;
+    const double prsq = sq(pr);
+    const double pthetasq = sq(pt);
+    const double partR = q + sq(a - b);
+    const double R = sq(P) - delta * partR;
+    const double idelta = rcp_once(delta), isin = rcp_once(sinv);
+    const SharedDiv by_rosq(rosq), by_sinsq(sinsq, isin * isin);
     const double bsq_sinsq = by_sinsq.pos(bsq);   // bsq / sinsq
-    double btheta = q - cossq * (bsq_sinsq - asq);
-    double rosqsq = sq(2 * rosq);
-    double sqrosqdel = (sq(rosq) * delta);
-    double asqcossin = asq * cosv * sinv;
-    double rtwo = 2 * r - 2;
-    const SharedDiv by_rd2(rosq * 2 * delta), by_rosqsq(rosqsq), by_srd(sqrosqdel);
+    const double btheta = q - cossq * (bsq_sinsq - asq);
+    const double asqcossin = asq * cosv * sinv;
+    const double rm1 = r - 1.;
+    const double rosq2 = sq(rosq);
+    const SharedDiv by_rd(rosq * delta, by_rosq.y * idelta), by_rosq2(rosq2, by_rosq.y * by_rosq.y);
+    const SharedDiv by_srd(rosq2 * delta, by_rosq2.y * idelta), by_rdd(rosq * sq(delta), by_rd.y * idelta);
     const double bdr = btheta * delta + R;
 
     o[0] = by_rosq.pos(delta) * pr;
     o[1] = by_rosq.pos(1.) * pt;
-    o[2] = by_rd2.any(2 * a * P - (2 * a - 2 * b) * delta + by_sinsq.pos(2 * b * cossq * delta));
-    o[3] = by_rd2.any(rtwo * btheta - rtwo * partR + 4 * r * P) - by_rosq.pos(prsq * rtwo) * 0.5
-        + by_rosqsq.pos(4 * pthetasq * r) - SharedDiv(rosq * sq(2 * delta)).pos((4 * r - 4) * bdr)
-        + by_rosqsq.pos(4 * prsq * r * (delta)) - by_srd.any(r * bdr);
-    o[4] = by_rd2.any((2 * cosv * sinv * (bsq_sinsq - asq) + SharedDiv(sq3(sinv)).any(2 * bsq * sq3(cosv))) *
-                      delta)
-        - by_rosqsq.pos(4 * asqcossin * pthetasq) - by_rosqsq.pos(4 * asqcossin * prsq * delta)
+    o[2] = by_rd.any(a * P - (a - b) * delta + by_sinsq.pos(b * cossq * delta));
+    o[3] = by_rd.any(rm1 * btheta - rm1 * partR + twor * P) - by_rosq.pos(prsq * rm1)
+        + by_rosq2.pos(pthetasq * r) - by_rdd.pos(rm1 * bdr)
+        + by_rosq2.pos(prsq * r * delta) - by_srd.any(r * bdr);
+    o[4] = by_rd.any((cosv * sinv * (bsq_sinsq - asq) + SharedDiv(sq3(sinv), by_sinsq.y * isin).any(bsq * sq3(cosv))) *
+                     delta)
+        - by_rosq2.pos(asqcossin * pthetasq) - by_rosq2.pos(asqcossin * prsq * delta)
         + by_srd.any(asqcossin * bdr);
 }
 

@@ -261,6 +261,10 @@ __global__ void selfcheck_div(int64_t n, unsigned long long seed, unsigned long 
         miss = __double_as_longlong(by.any(x)) != __double_as_longlong(ref);
         const SharedDiv byp(fabs(d));
         miss = miss || __double_as_longlong(byp.pos(x)) != __double_as_longlong(x / fabs(d));
+        // a product's reciprocal from its factors'
+        const double f = operand(h3, h1), df = d * f;
+        const SharedDiv by2(df, by.y * rcp_once(f));
+        miss = miss || __double_as_longlong(by2.any(x)) != __double_as_longlong(x / df);
     }
     const unsigned long long m = __ballot(miss);
     if (lane_id() == 0 && m) atomicAdd(bad, (unsigned long long)__popcll(m));
