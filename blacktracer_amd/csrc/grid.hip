@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "grid_dev.h"
+#include "kerr_dev.h"
 
 namespace bt {
 namespace {
@@ -313,6 +314,134 @@ __device__ __forceinline__ void refine_block_wave(const GridK& G, bool live, uin
 __global__ void final_level(GridK G, const uint32_t* blocks, unsigned nb, int level) {
     unsigned q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q < nb) G.level[blocks[q]] = (int8_t)level;
+}
+
+// ------------------------------------------------- levels traced ahead
+// The first levels of an adaptive build are a few thousand rays each, and
+// every one waits for its longest ray (some 200 attempts of 4 us, one after
+// the other).  On the FP64 path the whole lattice of a level S (Ahead: as fine
+// as kAheadRays rays allow) is therefore traced at once, straight into the
+// grid; the levels below S then refine without tracing, on device counts.
+// Afterwards the lattice points that no block asked for go back to their
+// untraced values, and the rays that were asked for are counted: the grid, its
+// ray count and its statistics are those of the level-by-level build.
+//
+// A level-10 grid built level by level took ten launches of about 1 ms.
+struct AheadJob {
+    GridK G;
+    PoseK P;
+    uint32_t* keys;       // every point of the lattice of level S
+    uint32_t* lists[2];   // blocks of level start_level + 0, 2, .. / 1, 3, ..
+    unsigned* ctr;        // per level, kCtrStride words apart: points claimed, children
+    int64_t item0;        // first lattice item (a multiple of 64)
+    uint32_t npts, ncols;
+    unsigned nb0;         // blocks of the start level
+    int S, gap0;
+};
+constexpr int kAheadLevels = 16;   // levels of a grid, at most 12
+
+// Lattice points traced ahead in one launch, at most (one grid's, or a batch's
+// together): a few rays for every lane the chip holds.
+constexpr int64_t kAheadRays = int64_t(3) << 18;
+
+__device__ __forceinline__ const AheadJob& ahead_job(const AheadJob* jobs, int njobs, int64_t t) {
+    int lo = 0, hi = njobs - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (jobs[mid].item0 <= t) lo = mid;
+        else hi = mid - 1;
+    }
+    return jobs[lo];
+}
+
+__device__ __forceinline__ uint32_t ahead_key(const AheadJob& J, uint32_t t) {
+    const int shift = J.G.max_level - J.S;
+    return ((t / J.ncols) << shift) * (uint32_t)J.G.M + ((t % J.ncols) << shift);
+}
+
+__global__ __launch_bounds__(256) void ahead_keys(const AheadJob* jobs, int njobs, int64_t items) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= items) return;
+    const AheadJob& J = ahead_job(jobs, njobs, t);
+    const int64_t lt = t - J.item0;
+    if (lt < (int64_t)J.npts) J.keys[lt] = ahead_key(J, (uint32_t)lt);
+}
+
+// What the trace of key's ray adds to the statistics: the a-priori test again
+// (its iterations are not kept), and the attempts from the step index.
+struct RayCount {
+    unsigned long long rays = 0, integrated = 0, attempts = 0, newton = 0, golden = 0;
+    __device__ __forceinline__ void add(const AheadJob& J, const ParamsK& prm, uint32_t key) {
+        RayIO io;
+        io.keys = &key;
+        io.N = J.G.N;
+        io.M = J.G.M;
+        io.eq = J.G.eq;
+        double th, ph, pR, pT, b, q;
+        kerr::ray_direction(io, 0, th, ph);
+        kerr::initial_conditions(J.P, th, ph, pR, pT, b, q);
+        unsigned nw = 0, gd = 0;
+        const bool escapes = prm.apriori ? kerr::check_celest(J.P, pR, b, q, prm.newton_cap, nw, gd) : true;
+        rays++;
+        newton += nw;
+        golden += gd;
+        if (escapes) {
+            integrated++;
+            attempts += (unsigned long long)J.G.steps[key] + 1;
+        }
+    }
+    __device__ __forceinline__ void store(StatsK* st) const {
+        const unsigned long long c[6] = {rays, integrated, attempts, attempts, newton, golden};
+        unsigned long long* const d[6] = {&st->rays,          &st->integrated, &st->attempts,
+                                          &st->attempts_fp64, &st->newton,     &st->golden};
+        kerr::block_add_stats<6>(c, d);
+    }
+};
+
+// The pole rays of job blockIdx.x, before the pole rows take their counts.
+__global__ __launch_bounds__(64) void ahead_poles(const AheadJob* jobs, ParamsK prm, StatsK* st) {
+    const AheadJob& J = jobs[blockIdx.x];
+    RayCount C;
+    if ((int)threadIdx.x <= J.G.eq) C.add(J, prm, threadIdx.x * (uint32_t)(J.G.N - 1) * (uint32_t)J.G.M);
+    C.store(st);
+}
+
+// One level below S of job blockIdx.y (adaptiveBlockIntegration's loop, the
+// points it claims being traced already).
+__global__ __launch_bounds__(256) void ahead_refine(const AheadJob* jobs, int level, double thresh) {
+    const AheadJob& J = jobs[blockIdx.y];
+    const int step = level - J.G.start_level;
+    if (step < 0 || level >= J.S) return;
+    const unsigned nb = step == 0 ? J.nb0 : J.ctr[(level - 1) * kCtrStride + 1];
+    for (unsigned q0 = blockIdx.x * 256; q0 < nb; q0 += gridDim.x * 256) {
+        const unsigned q = q0 + threadIdx.x;
+        const bool live = q < nb;
+        refine_block_wave(J.G, live, live ? J.lists[step & 1][q] : 0u, level, thresh, J.lists[(step & 1) ^ 1], J.keys,
+                          J.ctr + level * kCtrStride, true);
+    }
+}
+
+// Every lattice point once the levels below S are refined: back to untraced,
+// or counted (the pole rows' points at the start spacing are copies).
+__global__ __launch_bounds__(256) void ahead_settle(const AheadJob* jobs, int njobs, int64_t items, ParamsK prm,
+                                                    StatsK* st) {
+    RayCount C;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < items; t += (int64_t)gridDim.x * 256) {
+        const AheadJob& J = ahead_job(jobs, njobs, t);
+        const int64_t lt = t - J.item0;
+        if (lt >= (int64_t)J.npts) continue;
+        const uint32_t idx = ahead_key(J, (uint32_t)lt);
+        if (!((J.G.present[idx >> 5] >> (idx & 31)) & 1u)) {
+            J.G.cel[2 * (size_t)idx] = -2.0;
+            J.G.cel[2 * (size_t)idx + 1] = -2.0;
+            J.G.steps[idx] = 0;
+            continue;
+        }
+        const uint32_t i = idx / (uint32_t)J.G.M, j = idx % (uint32_t)J.G.M;
+        const bool pole = i == 0 || (J.G.eq && i == (uint32_t)(J.G.N - 1));
+        if (!(pole && j % (uint32_t)J.gap0 == 0)) C.add(J, prm, idx);
+    }
+    C.store(st);
 }
 
 // ---------------------------------------------------------------- T-vertices
@@ -616,6 +745,120 @@ int grid_fix_tvertices_multi(Context* c, const std::vector<bt_grid*>& gs) {
     return BT_OK;
 }
 
+namespace {
+
+// The key list of a grid build's first rays, its block lists, and what
+// grid_ahead leaves: the level reached and its blocks.
+struct AheadGrid {
+    bt_grid* g;
+    uint32_t *keys, *blocks, *next;
+    unsigned nb0;
+    int gap0;
+    // out
+    int level;
+    unsigned nb;
+};
+
+int64_t lattice_points(const bt_grid* g, int level) {
+    const int shift = g->max_level - level;
+    return ((int64_t)((g->N - 1) >> shift) + 1) * (g->M >> shift);
+}
+
+// The levels of `gs` below the one traced ahead (see above), FP64 path.  The
+// grids are initialised and their start lattices marked; `trace_keys(counts)`
+// traces the first counts[k] keys of grid k, outside the build's statistics.
+template <class Trace, class PoleRows>
+int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, double thresh, StatsK* d_stats,
+               Trace&& trace_keys, PoleRows&& fill_pole_rows) {
+    const int n = (int)gs.size();
+    const auto level_of = [&](const bt_grid* g, int s) { return std::min(std::max(s, g->start_level), g->max_level); };
+    const auto total = [&](int s) {
+        int64_t t = 0;
+        for (const AheadGrid& a : gs) t += lattice_points(a.g, level_of(a.g, s));
+        return t;
+    };
+    int s = 1;
+    while (s < 12 && total(s + 1) <= kAheadRays) s++;
+    std::vector<AheadJob> jobs(n);
+    std::vector<int64_t> counts(n);
+    const size_t ctr_words = (size_t)kCtrStride * kAheadLevels;
+    int rc;
+    void* p;
+    if ((rc = c->buffer("ahead_ctr", sizeof(unsigned) * ctr_words * n, &p))) return rc;
+    unsigned* ctr = (unsigned*)p;
+    int64_t items = 0;
+    int lmin = 99, lmax = 0;
+    unsigned most = 1;
+    for (int k = 0; k < n; k++) {
+        AheadGrid& a = gs[k];
+        AheadJob& J = jobs[k];
+        J.G = a.g->k;
+        J.P = a.g->pose;
+        J.keys = a.keys;
+        J.lists[0] = a.blocks;
+        J.lists[1] = a.next;
+        J.ctr = ctr + ctr_words * k;
+        J.item0 = items;
+        J.S = level_of(a.g, s);
+        counts[k] = lattice_points(a.g, J.S);
+        J.npts = (uint32_t)counts[k];
+        J.ncols = (uint32_t)a.g->M >> (a.g->max_level - J.S);
+        J.nb0 = a.nb0;
+        J.gap0 = a.gap0;
+        items += (counts[k] + 63) / 64 * 64;
+        lmin = std::min(lmin, a.g->start_level);
+        lmax = std::max(lmax, J.S);
+        // the blocks of level S - 1, at most
+        if (J.S > a.g->start_level) most = std::max(most, (J.npts + 3) / 4);
+    }
+    void* hs;
+    if ((rc = c->stage(sizeof(AheadJob) * n, &hs))) return rc;
+    std::memcpy(hs, jobs.data(), sizeof(AheadJob) * n);
+    if ((rc = c->buffer("ahead_jobs", sizeof(AheadJob) * n, &p))) return rc;
+    const AheadJob* d_jobs = (const AheadJob*)p;
+    BT_HIP(hipMemcpyAsync(p, hs, sizeof(AheadJob) * n, hipMemcpyHostToDevice, c->stream));
+    if ((rc = c->stage_done())) return rc;
+    ahead_keys<<<blocks_for(items, 256), 256, 0, c->stream>>>(d_jobs, n, items);
+    zero_span<<<blocks_for((int64_t)ctr_words * n, 256), 256, 0, c->stream>>>(ctr, (int)(ctr_words * n));
+    BT_HIP(hipGetLastError());
+    if ((rc = trace_keys(counts))) return rc;
+    ahead_poles<<<(unsigned)n, 64, 0, c->stream>>>(d_jobs, prm, d_stats);
+    fill_pole_rows();
+    BT_HIP(hipGetLastError());
+    {
+        KTimer t(c, "refine_level");
+        for (int level = lmin; level < lmax; level++)
+            ahead_refine<<<dim3(std::min(blocks_for(most, 256), 256u), (unsigned)n), 256, 0, c->stream>>>(d_jobs, level,
+                                                                                                        thresh);
+        ahead_settle<<<std::min(blocks_for(items, 256), (unsigned)c->num_cus * 8), 256, 0, c->stream>>>(
+            d_jobs, n, items, prm, d_stats);
+    }
+    BT_HIP(hipGetLastError());
+    std::vector<unsigned> h_ctr(ctr_words * n);
+    BT_HIP(hipMemcpyAsync(h_ctr.data(), ctr, sizeof(unsigned) * h_ctr.size(), hipMemcpyDeviceToHost, c->stream));
+    BT_HIP(hipStreamSynchronize(c->stream));
+    for (int k = 0; k < n; k++) {
+        AheadGrid& a = gs[k];
+        const unsigned* h = h_ctr.data() + ctr_words * k;
+        const int eq = a.g->eq;
+        int64_t nrows = (a.g->N - 1) / a.gap0;   // the start lattice's
+        if (eq) nrows--;
+        a.g->rays = 1 + eq + nrows * (a.g->M / a.gap0);
+        a.level = a.g->start_level;
+        a.nb = a.nb0;
+        // a level of no blocks ends the build there (Grid.h:469)
+        while (a.level < jobs[k].S && a.nb > 0) {
+            a.g->rays += h[a.level * kCtrStride];
+            a.nb = h[a.level * kCtrStride + 1];
+            a.level++;
+            std::swap(a.blocks, a.next);
+        }
+    }
+    return BT_OK;
+}
+
+}  // namespace
+
 int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
     const int N = g->N, M = g->M, eq = g->eq;
     const int max_level = g->max_level, start_level = g->start_level;
@@ -669,10 +912,9 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
     start_lattice<<<blocks_for(nlat, 256), 256, 0, c->stream>>>(
         G, gap0, nrows, ncols, trace_keys + 1 + eq, blocks + npole, uniform ? start_level : -1);
     BT_HIP(hipGetLastError());
-    if ((rc = trace(c, g->pose, g->prm, 1 + eq + nlat, io, d_stats))) return rc;
-    g->rays += 1 + eq + nlat;
-    pole_rows<<<blocks_for(npole, 256), 256, 0, c->stream>>>(G, gap0, blocks);
-    BT_HIP(hipGetLastError());
+    const auto fill_pole_rows = [&] {
+        pole_rows<<<blocks_for(npole, 256), 256, 0, c->stream>>>(G, gap0, blocks);
+    };
     unsigned nb = npole;
     if (!uniform) {
         unsigned lat_blocks = nrows * ncols;
@@ -680,8 +922,27 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
         nb += lat_blocks;
     }
 
-    // adaptiveBlockIntegration(startLevel)
     int level = start_level;
+    if (g->prm.precision == BT_PREC_FP64) {
+        if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
+        StatsK* spare = (StatsK*)p;
+        std::vector<AheadGrid> a{{g, trace_keys, blocks, next, nb, gap0, 0, 0}};
+        rc = grid_ahead(
+            c, a, g->prm, thresh, d_stats,
+            [&](const std::vector<int64_t>& n) { return trace(c, g->pose, g->prm, n[0], io, spare); }, fill_pole_rows);
+        if (rc) return rc;
+        level = a[0].level;
+        nb = a[0].nb;
+        blocks = a[0].blocks;
+        next = a[0].next;
+    } else {
+        if ((rc = trace(c, g->pose, g->prm, 1 + eq + nlat, io, d_stats))) return rc;
+        g->rays += 1 + eq + nlat;
+        fill_pole_rows();
+        BT_HIP(hipGetLastError());
+    }
+
+    // adaptiveBlockIntegration(startLevel)
     bool early = false;
     while (level < max_level) {
         if (nb == 0) {
@@ -826,32 +1087,7 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
     BT_HIP(hipGetLastError());
     start_lattice_multi<<<blocks_for(n_lat, 256), 256, 0, c->stream>>>(d_sj, G, n_lat);
     BT_HIP(hipGetLastError());
-    if (prm.precision == BT_PREC_FP64) {
-        // the FP64 path: every level of every grid in one dataflow kernel
-        std::vector<FlowGridHost> fh(G);
-        for (int k = 0; k < G; k++) {
-            FlowGridHost& f = fh[k];
-            f.G = gs[k]->k;
-            f.P = gs[k]->pose;
-            f.keys = per[k].keys;
-            f.list0 = per[k].blocks;
-            f.list1 = per[k].next;
-            f.nkeys = (unsigned)counts[k];
-            f.nb0 = per[k].nb;
-            f.npole = sj[k].npole;
-            f.gap0 = sj[k].gap;
-        }
-        std::vector<int64_t> rays;
-        if ((rc = grid_flow_run(c, fh, prm, thresh, d_stats, &rays))) return rc;
-        for (int k = 0; k < G; k++) gs[k]->rays = rays[k];
-        if (fix && (rc = grid_fix_tvertices_multi(c, gs))) return rc;
-        StatsK s;
-        BT_HIP(hipMemcpyAsync(&s, d_stats, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-        BT_HIP(hipStreamSynchronize(c->stream));
-        if (h_stats) *h_stats = s;
-        return BT_OK;
-    }
-    auto run_batch = [&](const std::vector<int64_t>& counts) -> int {
+    auto run_batch = [&](const std::vector<int64_t>& counts, StatsK* stats) -> int {
         BatchHost b;
         for (int k = 0; k < G; k++) {
             if (counts[k] <= 0) continue;
@@ -860,13 +1096,34 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
             b.counts.push_back(counts[k]);
             gs[k]->rays += counts[k];
         }
-        return trace_batch(c, b, prm, d_stats);
+        return trace_batch(c, b, prm, stats);
     };
-    // the poles and start lattices of all grids in one batch; the pole rows
-    // are filled once the pole rays are done
-    if ((rc = run_batch(counts))) return rc;
-    pole_rows_multi<<<blocks_for(n_pole, 256), 256, 0, c->stream>>>(d_sj, G, n_pole);
-    BT_HIP(hipGetLastError());
+    const auto fill_pole_rows = [&] {
+        pole_rows_multi<<<blocks_for(n_pole, 256), 256, 0, c->stream>>>(d_sj, G, n_pole);
+    };
+    if (prm.precision == BT_PREC_FP64) {
+        if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
+        StatsK* spare = (StatsK*)p;
+        std::vector<AheadGrid> a(G);
+        for (int k = 0; k < G; k++)
+            a[k] = AheadGrid{gs[k], per[k].keys, per[k].blocks, per[k].next, per[k].nb, sj[k].gap, 0, 0};
+        rc = grid_ahead(
+            c, a, prm, thresh, d_stats, [&](const std::vector<int64_t>& n) { return run_batch(n, spare); },
+            fill_pole_rows);
+        if (rc) return rc;
+        for (int k = 0; k < G; k++) {
+            per[k].level = a[k].level;
+            per[k].nb = a[k].nb;
+            per[k].blocks = a[k].blocks;
+            per[k].next = a[k].next;
+        }
+    } else {
+        // the poles and start lattices of all grids in one batch; the pole
+        // rows are filled once the pole rays are done
+        if ((rc = run_batch(counts, d_stats))) return rc;
+        fill_pole_rows();
+        BT_HIP(hipGetLastError());
+    }
     // adaptiveBlockIntegration(startLevel), all grids one level per round
     std::vector<unsigned> h_ctr((size_t)kCtrStride * G);
     std::vector<RefineJob> rjobs;
@@ -920,7 +1177,7 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
         BT_HIP(hipMemcpyAsync(h_ctr.data(), ctr, sizeof(unsigned) * h_ctr.size(), hipMemcpyDeviceToHost, c->stream));
         BT_HIP(hipStreamSynchronize(c->stream));
         for (int k = 0; k < G; k++) counts[k] = per[k].active ? (int64_t)h_ctr[(size_t)kCtrStride * k] : 0;
-        if ((rc = run_batch(counts))) return rc;
+        if ((rc = run_batch(counts, d_stats))) return rc;
         for (int k = 0; k < G; k++) {
             Per& q = per[k];
             if (!q.active) continue;

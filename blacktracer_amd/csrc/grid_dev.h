@@ -1,7 +1,6 @@
-// grid_dev.h -- device helpers of the adaptive grid shared by the level-by-
-// level build (grid.hip) and the dataflow build (grid_flow.hip).
-// Compiled with -ffp-contract=off in both (the refinement test compares
-// squared differences as the reference does).
+// grid_dev.h -- device helpers of the adaptive grid build (grid.hip).
+// Compiled with -ffp-contract=off (the refinement test compares squared
+// differences as the reference does).
 #pragma once
 
 #include "bt_grid.h"
@@ -48,20 +47,6 @@ struct BlockRefine {
     uint32_t kids[4];
 };
 
-// Grid values as COHERENT reads them: agent-scope atomic loads, which see
-// values other waves stored with agent-scope atomic stores (the dataflow
-// build, where the XCDs' L2 caches are not coherent with each other);
-// otherwise plain loads (the level-by-level build, where kernel boundaries
-// order the accesses).
-template <bool COHERENT>
-__device__ __forceinline__ double cel_load(const double* p) {
-    if (COHERENT)
-        return __longlong_as_double((long long)__hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED,
-                                                                 __HIP_MEMORY_SCOPE_AGENT));
-    return *p;
-}
-
-template <bool COHERENT = false>
 __device__ __forceinline__ bool refine_test(const GridK& G, uint32_t key, int level, double thresh,
                                             BlockRefine& R) {
     const uint32_t M = (uint32_t)G.M;
@@ -72,10 +57,10 @@ __device__ __forceinline__ bool refine_test(const GridK& G, uint32_t key, int le
     const uint32_t l = j + gap / 2;
     const uint32_t kk = i + gap, ll = (j + gap) % M;
     const double* c = G.cel;
-    double th1 = cel_load<COHERENT>(&c[2 * (i * M + j)]), th2 = cel_load<COHERENT>(&c[2 * (kk * M + j)]);
-    double th3 = cel_load<COHERENT>(&c[2 * (i * M + ll)]), th4 = cel_load<COHERENT>(&c[2 * (kk * M + ll)]);
-    double ph1 = cel_load<COHERENT>(&c[2 * (i * M + j) + 1]), ph2 = cel_load<COHERENT>(&c[2 * (kk * M + j) + 1]);
-    double ph3 = cel_load<COHERENT>(&c[2 * (i * M + ll) + 1]), ph4 = cel_load<COHERENT>(&c[2 * (kk * M + ll) + 1]);
+    double th1 = c[2 * (i * M + j)], th2 = c[2 * (kk * M + j)];
+    double th3 = c[2 * (i * M + ll)], th4 = c[2 * (kk * M + ll)];
+    double ph1 = c[2 * (i * M + j) + 1], ph2 = c[2 * (kk * M + j) + 1];
+    double ph3 = c[2 * (i * M + ll) + 1], ph4 = c[2 * (kk * M + ll) + 1];
     double diag = (th1 - th4) * (th1 - th4) + (ph1 - ph4) * (ph1 - ph4);
     double diag2 = (th2 - th3) * (th2 - th3) + (ph2 - ph3) * (ph2 - ph3);
     double mx = (diag < diag2) ? diag2 : diag;   // std::max

@@ -1,0 +1,61 @@
+"""Grids whose first levels are traced ahead: the same grid whichever level
+that is, and the statistics of the rays that its blocks asked for alone.
+
+A single grid traces a finer lattice ahead than the same grid in a batch of
+many, so each must equal the other bit for bit; the counts must equal those of
+a ray batch over exactly the traced directions.
+"""
+import math
+
+import numpy as np
+import pytest
+
+import blacktracer_amd as bt
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = ("rays", "integrated", "attempts", "newton", "golden")
+
+
+def traced_directions(g):
+    """Directions of the rays a build traces: every present point but the
+    copies along the pole rows at the start level's spacing."""
+    present = g.cel[..., 0] != -2
+    gap0 = 1 << (g.MAXLEVEL - g.STARTLVL)
+    for row in (0, g.N - 1) if g.equafactor else (0,):
+        present[row, gap0::gap0] = False
+    i, j = np.nonzero(present)
+    return i / (g.N - 1) * math.pi / (2 - g.equafactor), j / g.M * (2 * math.pi)
+
+
+def camera(k):
+    hole = bt.BlackHole(0.0 if k == 3 else 0.999 - 0.07 * k)
+    return bt.Camera(math.pi / 2 - 0.1 * k, 0.0, 4.0 + k, black_hole=hole), hole
+
+
+@pytest.mark.parametrize("level,start,angle,thresh", [
+    (1, 1, True, 0.015), (2, 1, False, 0.015), (5, 5, True, 0.015), (8, 1, True, 0.015), (8, 3, False, 0.015),
+    (9, 6, True, 0.015), (8, 2, True, 1e9), (10, 1, False, 0.1)])
+def test_same_grid_and_counts(ctx, level, start, angle, thresh):
+    n = 3 if level > 9 else 36
+    cams, holes = zip(*[camera(k % 5) for k in range(n)])
+    print(f"batch of {n} Grid({level},{start},angle={angle}) thresh={thresh}", flush=True)
+    batch, stats = bt.Grid.build_batch(cams, holes, [level] * n, [start] * n, angle=angle, refine_thresh=thresh,
+                                       fix_tvertices=False, ctx=ctx)
+    total = dict.fromkeys(COUNTS, 0)
+    for k in range(min(n, 5)):
+        g = bt.Grid(level, start, angle, cams[k], holes[k], refine_thresh=thresh, fix_tvertices=False, ctx=ctx)
+        for h in batch[k::5]:
+            assert g.rays_traced == h.rays_traced
+            assert np.array_equal(g.cel, h.cel) and np.array_equal(g.steps, h.steps)
+            assert np.array_equal(g.levels, h.levels)
+        assert not g.steps[g.cel[..., 0] == -2].any()
+        th, ph = traced_directions(g)
+        assert th.size == g.rays_traced
+        *_, want = bt.trace_rays(cams[k], th, ph, ctx=ctx, return_stats=True)
+        assert {c: g.stats()[c] for c in COUNTS} == {c: want[c] for c in COUNTS}
+        for c in COUNTS:
+            total[c] += want[c] * len(batch[k::5])
+    assert {c: stats[c] for c in COUNTS} == total
+    for h in batch:
+        h.close()
