@@ -143,6 +143,12 @@ struct Buffer {
     size_t bytes = 0;
 };
 
+struct CopySeg {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+
 // Launch-shape knobs of the persistent integrators.
 struct Tune {
     unsigned chunk = 128;   // queue positions a wave reserves per atomic (>= 64)
@@ -197,6 +203,15 @@ struct Context {
     hipEvent_t ev_stage = nullptr;
     int stage(size_t bytes, void** out);
     int stage_done();
+    // Copies between host and device memory on the main stream (copy.cpp).
+    // On return the host memory has been read, or holds the data; copies to
+    // the device are ordered on the stream.
+    static constexpr int kCopySlots = 12;
+    void* copy_stage = nullptr;   // kCopySlots pinned pieces of 2 MiB
+    hipEvent_t ev_copy[kCopySlots] = {};
+    int copy(const std::vector<CopySeg>& segs, bool to_device);
+    int copy_slots();
+    void release_copy_slots();
     int timer_begin(const char* name, int* slot, hipStream_t st = nullptr);
     int timer_end(int slot);
     int flush_timers();

@@ -366,6 +366,7 @@ void bt_context_destroy(bt_context* h) {
     (void)hipEventDestroy(c.ev_back);
     (void)hipEventDestroy(c.ev_stage);
     if (c.host_stage) (void)hipHostFree(c.host_stage);
+    c.release_copy_slots();
     (void)hipStreamDestroy(c.aux);
     (void)hipStreamDestroy(c.stream);
     delete h;

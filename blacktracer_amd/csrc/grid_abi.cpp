@@ -128,14 +128,11 @@ int bt_grid_export(const bt_grid* g, double* cel, int32_t* steps, int8_t* levels
     std::lock_guard<std::recursive_mutex> lk(c.mu);
     BT_HIP(hipSetDevice(c.device));
     const int64_t NM = (int64_t)g->N * g->M;
-    if (cel)
-        BT_HIP(hipMemcpyAsync(cel, g->k.cel, sizeof(double) * 2 * NM, hipMemcpyDeviceToHost, c.stream));
-    if (steps)
-        BT_HIP(hipMemcpyAsync(steps, g->k.steps, sizeof(int32_t) * NM, hipMemcpyDeviceToHost, c.stream));
-    if (levels)
-        BT_HIP(hipMemcpyAsync(levels, g->k.level, NM, hipMemcpyDeviceToHost, c.stream));
-    BT_HIP(hipStreamSynchronize(c.stream));
-    return BT_OK;
+    std::vector<CopySeg> segs;
+    if (cel) segs.push_back({cel, g->k.cel, sizeof(double) * 2 * NM});
+    if (steps) segs.push_back({steps, g->k.steps, sizeof(int32_t) * NM});
+    if (levels) segs.push_back({levels, g->k.level, (size_t)NM});
+    return c.copy(segs, false);
 }
 
 int bt_grid_export_psh(const bt_grid* g, int* hash_width, int* offset_width, float* hash_table,
@@ -148,10 +145,10 @@ int bt_grid_export_psh(const bt_grid* g, int* hash_width, int* offset_width, flo
     const int64_t nwords = (NM + 31) / 32;
     std::vector<double> cel(2 * NM);
     std::vector<uint32_t> present(nwords);
-    BT_HIP(hipMemcpyAsync(cel.data(), g->k.cel, sizeof(double) * 2 * NM, hipMemcpyDeviceToHost, c.stream));
-    BT_HIP(hipMemcpyAsync(present.data(), g->k.present, sizeof(uint32_t) * nwords,
-                          hipMemcpyDeviceToHost, c.stream));
-    BT_HIP(hipStreamSynchronize(c.stream));
+    if (int crc = c.copy({{cel.data(), g->k.cel, sizeof(double) * 2 * NM},
+                          {present.data(), g->k.present, sizeof(uint32_t) * nwords}},
+                         false))
+        return crc;
     // Grid.h:645-651: every CamToCel entry, as float2
     std::vector<int32_t> keys;
     std::vector<float> vals;

@@ -211,7 +211,7 @@ static int scene_upload(Context& c, bt_scene* s, const int32_t* tree, int tree_l
     void* dsky;
     int rc;
     if ((rc = c.buffer("scene_sky_upload", (size_t)3 * rows * cols, &dsky))) return rc;
-    BT_HIP(hipMemcpyAsync(dsky, sky, (size_t)3 * rows * cols, hipMemcpyHostToDevice, c.stream));
+    if ((rc = c.copy({{dsky, sky, (size_t)3 * rows * cols}}, true))) return rc;
     if ((rc = render_sum_table(&c, (const uint8_t*)dsky, rows, cols, s->table))) return rc;
     BT_HIP(hipStreamSynchronize(c.stream));
     return BT_OK;
@@ -744,10 +744,15 @@ int bt_make_image(bt_context* h, const float* stars, const int32_t* star_tree_in
         scene_release(&scene);
         return rc;
     }
-    BT_HIP(hipMemcpyAsync(dht, hash_tables, sizeof(float) * 2 * (size_t)hw * hw, hipMemcpyHostToDevice, c.stream));
-    BT_HIP(hipMemcpyAsync(dot, offset_tables, sizeof(int32_t) * 2 * (size_t)ow * ow, hipMemcpyHostToDevice, c.stream));
-    BT_HIP(hipMemcpyAsync(dtag, hash_pos_tag, sizeof(int32_t) * 2 * (size_t)hw * hw, hipMemcpyHostToDevice, c.stream));
-    BT_HIP(hipMemcpyAsync(dview, viewthing, sizeof(float) * 2 * NC, hipMemcpyHostToDevice, c.stream));
+    if ((rc = c.copy({{dht, hash_tables, sizeof(float) * 2 * (size_t)hw * hw},
+                      {dot, offset_tables, sizeof(int32_t) * 2 * (size_t)ow * ow},
+                      {dtag, hash_pos_tag, sizeof(int32_t) * 2 * (size_t)hw * hw},
+                      {dview, viewthing, sizeof(float) * 2 * NC}},
+                     true))) {
+        (void)hipStreamSynchronize(c.stream);
+        scene_release(&scene);
+        return rc;
+    }
     int gn1 = 0;
     if ((rc = render_grid_from_psh(&c, (const float*)dht, (const int32_t*)dot, (const int32_t*)dtag, hw, ow, GN, GM,
                                    (float*)dgrid, &gn1)))
@@ -760,11 +765,7 @@ int bt_make_image(bt_context* h, const float* stars, const int32_t* star_tree_in
                           cam_param, f, step, (uint8_t*)dout, nullptr);
         if (rc) goto done;
     }
-    {
-        hipError_t e = hipMemcpyAsync(out_bgra, dout, 4 * NP, hipMemcpyDeviceToHost, c.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-        if (e != hipSuccess) rc = fail(BT_ERR_HIP, std::string("bt_make_image: ") + hipGetErrorString(e));
-    }
+    rc = c.copy({{out_bgra, dout, 4 * NP}}, false);
 done:
     (void)hipStreamSynchronize(c.stream);
     scene_release(&scene);
