@@ -482,11 +482,15 @@ struct Edge {
 // run from an explicit stack.  GROUP issues all loads of a node together
 // (the line walkers, whose nodes are mostly present); without it the node's
 // presence is tested first (the pole walker, which meets many absent nodes).
+// The stack is the wave's own piece of LDS (one lane runs this): in scratch
+// memory every node paid two more round trips (fixing a level-10 grid took
+// 660 us).  A node leaves at most one sibling per level on it.
+constexpr int kFixStack = 16;   // levels of a grid are at most 12
+
 template <bool GROUP>
-__device__ void check_adjacent(const GridK& G, Edge root, int udlr) {
+__device__ void check_adjacent(const GridK& G, Edge root, int udlr, Edge* st) {
     const uint32_t M = (uint32_t)G.M, N = (uint32_t)G.N;
     double* cel = G.cel;
-    Edge st[40];
     int sp = 0;
     st[sp++] = root;
     while (sp > 0) {
@@ -541,7 +545,7 @@ __device__ void check_adjacent(const GridK& G, Edge root, int udlr) {
             cel[2 * mid + 1] = 1. / 2. * (ph[1] + ph[0]);
         }
         if (f.level + 1 == G.max_level) continue;
-        if (sp + 2 > 40) continue;   // unreachable: depth <= max_level
+        if (sp + 2 > kFixStack) continue;   // unreachable: depth <= max_level
         st[sp++] = Edge{i, j, f.ii2, f.jj2, f.level + 1, f.gap / 2};
         st[sp++] = Edge{f.ii, f.jj, i, j, f.level + 1, f.gap / 2};
     }
@@ -562,7 +566,7 @@ __device__ __forceinline__ bool block_fixable(const GridK& G, uint32_t i, uint32
 // The row-0 blocks of level L in key order, with the three edges each
 // repairs that touch the north pole rows (its bottom edge is on row gap and
 // is left to that row's walker).  One wavefront.
-__device__ __forceinline__ void fix_pole(const GridK& G, int L) {
+__device__ __forceinline__ void fix_pole(const GridK& G, int L, Edge* st) {
     const unsigned lane = threadIdx.x & 63;
     const uint32_t M = (uint32_t)G.M;
     const int gap = 1 << (G.max_level - L);
@@ -576,15 +580,16 @@ __device__ __forceinline__ void fix_pole(const GridK& G, int L) {
             m &= m - 1;
             const uint32_t jj = j0 + (uint32_t)src * ug, l = (jj + ug) % M;
             if (lane == 0) {
-                check_adjacent<false>(G, Edge{0, jj, ug, jj, L, gap}, 1);
-                check_adjacent<false>(G, Edge{0, jj, 0, l, L, gap}, 0);
-                check_adjacent<false>(G, Edge{0, l, ug, l, L, gap}, 1);
+                check_adjacent<false>(G, Edge{0, jj, ug, jj, L, gap}, 1, st);
+                check_adjacent<false>(G, Edge{0, jj, 0, l, L, gap}, 0, st);
+                check_adjacent<false>(G, Edge{0, l, ug, l, L, gap}, 1, st);
             }
         }
     }
 }
 
-__device__ __forceinline__ void fix_line(const GridK& G, int L, unsigned nrows, unsigned npairs, unsigned t) {
+__device__ __forceinline__ void fix_line(const GridK& G, int L, unsigned nrows, unsigned npairs, unsigned t,
+                                         Edge* st) {
     const unsigned lane = threadIdx.x & 63;
     const uint32_t M = (uint32_t)G.M, N = (uint32_t)G.N;
     const int gap = 1 << (G.max_level - L);
@@ -606,7 +611,7 @@ __device__ __forceinline__ void fix_line(const GridK& G, int L, unsigned nrows, 
                     const int src = __ffsll((long long)m) - 1;
                     m &= m - 1;
                     const uint32_t jj = j0 + (uint32_t)src * ug;
-                    if (lane == 0) check_adjacent<true>(G, Edge{y, jj, y, (jj + ug) % M, L, gap}, 0);
+                    if (lane == 0) check_adjacent<true>(G, Edge{y, jj, y, (jj + ug) % M, L, gap}, 0, st);
                 }
             }
         }
@@ -639,17 +644,21 @@ __device__ __forceinline__ void fix_line(const GridK& G, int L, unsigned nrows, 
                 m &= m - 1;
                 const uint32_t ii = i0 + (uint32_t)(src >> 2) * ug;
                 const uint32_t cc = __shfl(col, src);
-                if (lane == 0) check_adjacent<true>(G, Edge{ii, cc, ii + ug, cc, L, gap}, 1);
+                if (lane == 0) check_adjacent<true>(G, Edge{ii, cc, ii + ug, cc, L, gap}, 1, st);
             }
         }
     }
 }
 
 __global__ __launch_bounds__(256) void fix_level(GridK G, int L, unsigned nrows, unsigned npairs) {
-    fix_line(G, L, nrows, npairs, (blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    __shared__ Edge s_stack[4][kFixStack];
+    fix_line(G, L, nrows, npairs, (blockIdx.x * blockDim.x + threadIdx.x) >> 6, s_stack[threadIdx.x >> 6]);
 }
 
-__global__ __launch_bounds__(64) void fix_level_pole(GridK G, int L) { fix_pole(G, L); }
+__global__ __launch_bounds__(64) void fix_level_pole(GridK G, int L) {
+    __shared__ Edge s_stack[kFixStack];
+    fix_pole(G, L, s_stack);
+}
 
 // The same for several grids in one launch: grid g owns line items
 // [item0[g], item0[g+1]) (rows first, then meridian pairs, as above).
@@ -661,11 +670,13 @@ struct FixJob {
 
 // fix_pole for job blockIdx.x (one wavefront each)
 __global__ __launch_bounds__(64) void fix_pole_multi(const FixJob* jobs) {
+    __shared__ Edge s_stack[kFixStack];
     const FixJob& J = jobs[blockIdx.x];
-    fix_pole(J.G, J.L);
+    fix_pole(J.G, J.L, s_stack);
 }
 
 __global__ __launch_bounds__(256) void fix_level_multi(const FixJob* jobs, int njobs) {
+    __shared__ Edge s_stack[4][kFixStack];
     const unsigned t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
@@ -675,7 +686,7 @@ __global__ __launch_bounds__(256) void fix_level_multi(const FixJob* jobs, int n
     }
     const FixJob& J = jobs[lo];
     if (t < J.item0) return;
-    fix_line(J.G, J.L, J.nrows, J.npairs, t - J.item0);
+    fix_line(J.G, J.L, J.nrows, J.npairs, t - J.item0, s_stack[threadIdx.x >> 6]);
 }
 
 unsigned blocks_for(int64_t n, int tpb) { return (unsigned)((n + tpb - 1) / tpb); }
