@@ -88,7 +88,22 @@ struct RayIO {
     double* out_ph;
     int ostride;
     int32_t* out_step;
+    // Nullable: per ray, what its trace added to the statistics (RayTally).
+    struct RayTally* tally;
 };
+
+// A ray's attempts, those of them in FP64, and how often it went to the exact
+// FP64 path (the statistics of a launch, ray by ray).
+struct RayTally {
+    uint32_t attempts, fp64, fallback;
+};
+
+// Below this tolerance FP32 cannot carry the step control: the rounding of
+// the FP32 stage sums (unit roundoff 6e-8, relative to |y| + |h y'|) is no
+// longer small against eps, so the error estimate turns into noise, steps
+// collapse and the FP32 right-hand side's rounding accumulates into the
+// angles.  The mixed mode then traces every ray in FP64.
+constexpr double kMixedEpsMin = 1e-6;
 
 // Where the rays of one launch come from.  SingleSrc: one pose, one RayIO
 // (kernel arguments).  MultiSrc: a batch of segments, each with its own

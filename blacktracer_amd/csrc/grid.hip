@@ -67,13 +67,6 @@ __global__ void zero_span(unsigned* p, int n) {
 // batch refine in one launch.
 constexpr int kCtrStride = 32;
 
-__global__ void pole_keys(uint32_t* keys, uint32_t south) {
-    if (threadIdx.x == 0) {
-        keys[0] = 0u;
-        keys[1] = south;
-    }
-}
-
 __global__ void pole_rows(GridK G, int gap, uint32_t* blocks) {
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (uint32_t)G.M / (uint32_t)gap) return;
@@ -87,14 +80,12 @@ __global__ void pole_rows(GridK G, int gap, uint32_t* blocks) {
 // otherwise put 32 atomics on every word).  Every lane of the wave calls
 // this (the OR is a wave collective); lanes with live false touch no memory.
 __device__ __forceinline__ void lattice_point(const GridK& G, int gap, uint32_t nrows, uint32_t ncols,
-                                              uint32_t* trace, uint32_t* blocks, int mark_level, uint32_t t,
-                                              bool live) {
+                                              uint32_t* blocks, int mark_level, uint32_t t, bool live) {
     uint32_t word = 0xFFFFFFFFu, bits = 0u;
     if (live) {
         uint32_t i = (uint32_t)gap * (t / ncols + 1);
         uint32_t j = (uint32_t)gap * (t % ncols);
         uint32_t idx = i * (uint32_t)G.M + j;
-        trace[t] = idx;
         word = idx >> 5;
         bits = 1u << (idx & 31);
         if (i != (uint32_t)(G.N - 1)) {
@@ -114,19 +105,17 @@ __device__ __forceinline__ void lattice_point(const GridK& G, int gap, uint32_t 
     if (live && (lane == 0 || pw != word)) atomicOr(&G.present[word], bits);
 }
 
-__global__ void start_lattice(GridK G, int gap, uint32_t nrows, uint32_t ncols, uint32_t* trace,
-                              uint32_t* blocks, int mark_level) {
+__global__ void start_lattice(GridK G, int gap, uint32_t nrows, uint32_t ncols, uint32_t* blocks, int mark_level) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    lattice_point(G, gap, nrows, ncols, trace, blocks, mark_level, t, t < nrows * ncols);
+    lattice_point(G, gap, nrows, ncols, blocks, mark_level, t, t < nrows * ncols);
 }
 
-// The set-up of every grid of a batch (init_grid + pole_keys, start_lattice,
+// The set-up of every grid of a batch (init_grid, start_lattice,
 // pole_rows), one launch per step for all grids.  Job g owns the items
 // [first_g, first_{g+1}) of each launch; its lattice items start on a
 // multiple of 64, so that no wavefront spans two grids.
 struct SetupJob {
     GridK G;
-    uint32_t* keys;     // [north | south | lattice] ray keys
     uint32_t* blocks;   // [pole-row blocks | lattice blocks]
     int64_t init0, lat0, pole0;
     int64_t nm, nwords;
@@ -163,10 +152,6 @@ __global__ __launch_bounds__(256) void init_grid_multi(const SetupJob* jobs, int
         G.steps[i] = 0;
         G.level[i] = -1;
         if (i < J.nwords) G.present[i] = 0u;
-        if (i == 0) {
-            J.keys[0] = 0u;
-            J.keys[1] = (uint32_t)(G.N - 1) * (uint32_t)G.M;
-        }
     }
 }
 
@@ -178,8 +163,7 @@ __global__ void start_lattice_multi(const SetupJob* jobs, int njobs, int64_t ite
     const SetupJob& J = setup_job<1>(jobs, njobs, in ? t : items - 1);
     const int64_t lt = t - J.lat0;
     const bool live = in && lt < (int64_t)J.nrows * J.ncols;
-    lattice_point(J.G, J.gap, J.nrows, J.ncols, J.keys + 1 + J.G.eq, J.blocks + J.npole, J.mark_level,
-                  live ? (uint32_t)lt : 0u, live);
+    lattice_point(J.G, J.gap, J.nrows, J.ncols, J.blocks + J.npole, J.mark_level, live ? (uint32_t)lt : 0u, live);
 }
 
 __global__ void pole_rows_multi(const SetupJob* jobs, int njobs, int64_t items) {
@@ -319,9 +303,9 @@ __global__ void final_level(GridK G, const uint32_t* blocks, unsigned nb, int le
 // ------------------------------------------------- levels traced ahead
 // The first levels of an adaptive build are a few thousand rays each, and
 // every one waits for its longest ray (some 200 attempts of 4 us, one after
-// the other).  On the FP64 path the whole lattice of a level S (Ahead: as fine
-// as kAheadRays rays allow) is therefore traced at once, straight into the
-// grid; the levels below S then refine without tracing, on device counts.
+// the other).  The whole lattice of a level S (as fine as kAheadRays rays
+// allow) is therefore traced at once, straight into the grid; the levels below
+// S then refine without tracing, on device counts.
 // Afterwards the lattice points that no block asked for go back to their
 // untraced values, and the rays that were asked for are counted: the grid, its
 // ray count and its statistics are those of the level-by-level build.
@@ -331,6 +315,7 @@ struct AheadJob {
     GridK G;
     PoseK P;
     uint32_t* keys;       // every point of the lattice of level S
+    RayTally* tally;      // per point (mixed precision only, else null)
     uint32_t* lists[2];   // blocks of level start_level + 0, 2, .. / 1, 3, ..
     unsigned* ctr;        // per level, kCtrStride words apart: points claimed, children
     int64_t item0;        // first lattice item (a multiple of 64)
@@ -364,14 +349,19 @@ __global__ __launch_bounds__(256) void ahead_keys(const AheadJob* jobs, int njob
     if (t >= items) return;
     const AheadJob& J = ahead_job(jobs, njobs, t);
     const int64_t lt = t - J.item0;
-    if (lt < (int64_t)J.npts) J.keys[lt] = ahead_key(J, (uint32_t)lt);
+    if (lt >= (int64_t)J.npts) return;
+    J.keys[lt] = ahead_key(J, (uint32_t)lt);
+    if (J.tally) J.tally[lt] = RayTally{0, 0, 0};
 }
 
-// What the trace of key's ray adds to the statistics: the a-priori test again
-// (its iterations are not kept), and the attempts from the step index.
+// What the trace of lattice point lt adds to the statistics: the a-priori test
+// again (its iterations are not kept), and the attempts from the step index or
+// the ray's tally.
 struct RayCount {
-    unsigned long long rays = 0, integrated = 0, attempts = 0, newton = 0, golden = 0;
-    __device__ __forceinline__ void add(const AheadJob& J, const ParamsK& prm, uint32_t key) {
+    unsigned long long rays = 0, integrated = 0, attempts = 0, fp64 = 0, newton = 0, golden = 0, fallback = 0;
+    __device__ __forceinline__ void add(const AheadJob& J, const ParamsK& prm, uint32_t lt) {
+        const uint32_t key = ahead_key(J, lt);
+        const bool split = prm.precision == BT_PREC_MIXED && !(prm.eps < kMixedEpsMin);
         RayIO io;
         io.keys = &key;
         io.N = J.G.N;
@@ -382,19 +372,29 @@ struct RayCount {
         kerr::initial_conditions(J.P, th, ph, pR, pT, b, q);
         unsigned nw = 0, gd = 0;
         const bool escapes = prm.apriori ? kerr::check_celest(J.P, pR, b, q, prm.newton_cap, nw, gd) : true;
+        double r0;
+        if (split && escapes && !prm.apriori && !J.P.a_zero) kerr::check_bq(J.P, b, q, prm.newton_cap, nw, &r0);
         rays++;
         newton += nw;
         golden += gd;
-        if (escapes) {
-            integrated++;
+        if (!escapes) return;
+        integrated++;
+        if (split) {
+            const RayTally t = J.tally[lt];
+            attempts += t.attempts;
+            fp64 += t.fp64;
+            fallback += t.fallback;
+        } else {
             attempts += (unsigned long long)J.G.steps[key] + 1;
+            fp64 += (unsigned long long)J.G.steps[key] + 1;
+            fallback += prm.precision == BT_PREC_MIXED;   // every ray, at a tolerance too fine for FP32
         }
     }
     __device__ __forceinline__ void store(StatsK* st) const {
-        const unsigned long long c[6] = {rays, integrated, attempts, attempts, newton, golden};
-        unsigned long long* const d[6] = {&st->rays,          &st->integrated, &st->attempts,
-                                          &st->attempts_fp64, &st->newton,     &st->golden};
-        kerr::block_add_stats<6>(c, d);
+        const unsigned long long c[7] = {rays, integrated, attempts, fp64, newton, golden, fallback};
+        unsigned long long* const d[7] = {&st->rays,   &st->integrated, &st->attempts, &st->attempts_fp64,
+                                          &st->newton, &st->golden,     &st->fallback};
+        kerr::block_add_stats<7>(c, d);
     }
 };
 
@@ -402,7 +402,7 @@ struct RayCount {
 __global__ __launch_bounds__(64) void ahead_poles(const AheadJob* jobs, ParamsK prm, StatsK* st) {
     const AheadJob& J = jobs[blockIdx.x];
     RayCount C;
-    if ((int)threadIdx.x <= J.G.eq) C.add(J, prm, threadIdx.x * (uint32_t)(J.G.N - 1) * (uint32_t)J.G.M);
+    if ((int)threadIdx.x <= J.G.eq) C.add(J, prm, threadIdx.x * (J.npts - J.ncols));
     C.store(st);
 }
 
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(256) void ahead_settle(const AheadJob* jobs, int nj
         }
         const uint32_t i = idx / (uint32_t)J.G.M, j = idx % (uint32_t)J.G.M;
         const bool pole = i == 0 || (J.G.eq && i == (uint32_t)(J.G.N - 1));
-        if (!(pole && j % (uint32_t)J.gap0 == 0)) C.add(J, prm, idx);
+        if (!(pole && j % (uint32_t)J.gap0 == 0)) C.add(J, prm, (uint32_t)lt);
     }
     C.store(st);
 }
@@ -758,8 +758,8 @@ int grid_fix_tvertices_multi(Context* c, const std::vector<bt_grid*>& gs) {
 
 namespace {
 
-// The key list of a grid build's first rays, its block lists, and what
-// grid_ahead leaves: the level reached and its blocks.
+// The key list of a grid build's rays, its block lists, and what grid_ahead
+// leaves: the level reached and its blocks.
 struct AheadGrid {
     bt_grid* g;
     uint32_t *keys, *blocks, *next;
@@ -775,8 +775,8 @@ int64_t lattice_points(const bt_grid* g, int level) {
     return ((int64_t)((g->N - 1) >> shift) + 1) * (g->M >> shift);
 }
 
-// The levels of `gs` below the one traced ahead (see above), FP64 path.  The
-// grids are initialised and their start lattices marked; `trace_keys(counts)`
+// The levels of `gs` below the one traced ahead (see above).  The grids are
+// initialised and their start lattices marked; `trace_keys(counts, tallies)`
 // traces the first counts[k] keys of grid k, outside the build's statistics.
 template <class Trace, class PoleRows>
 int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, double thresh, StatsK* d_stats,
@@ -792,6 +792,7 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
     while (s < 12 && total(s + 1) <= kAheadRays) s++;
     std::vector<AheadJob> jobs(n);
     std::vector<int64_t> counts(n);
+    std::vector<RayTally*> tallies(n, nullptr);
     const size_t ctr_words = (size_t)kCtrStride * kAheadLevels;
     int rc;
     void* p;
@@ -806,6 +807,7 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
         J.G = a.g->k;
         J.P = a.g->pose;
         J.keys = a.keys;
+        J.tally = nullptr;
         J.lists[0] = a.blocks;
         J.lists[1] = a.next;
         J.ctr = ctr + ctr_words * k;
@@ -822,6 +824,10 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
         // the blocks of level S - 1, at most
         if (J.S > a.g->start_level) most = std::max(most, (J.npts + 3) / 4);
     }
+    if (prm.precision == BT_PREC_MIXED) {
+        if ((rc = c->buffer("ahead_tally", sizeof(RayTally) * items, &p))) return rc;
+        for (int k = 0; k < n; k++) tallies[k] = jobs[k].tally = (RayTally*)p + jobs[k].item0;
+    }
     void* hs;
     if ((rc = c->stage(sizeof(AheadJob) * n, &hs))) return rc;
     std::memcpy(hs, jobs.data(), sizeof(AheadJob) * n);
@@ -832,7 +838,7 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
     ahead_keys<<<blocks_for(items, 256), 256, 0, c->stream>>>(d_jobs, n, items);
     zero_span<<<blocks_for((int64_t)ctr_words * n, 256), 256, 0, c->stream>>>(ctr, (int)(ctr_words * n));
     BT_HIP(hipGetLastError());
-    if ((rc = trace_keys(counts))) return rc;
+    if ((rc = trace_keys(counts, tallies))) return rc;
     ahead_poles<<<(unsigned)n, 64, 0, c->stream>>>(d_jobs, prm, d_stats);
     fill_pole_rows();
     BT_HIP(hipGetLastError());
@@ -908,10 +914,7 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
     g->rays = 0;
 
     // raytrace(): the pole rays (Grid.h:295-301) and integrateFirst(gap)
-    // (Grid.h:325-338) are independent, so they are traced in one batch:
-    // keys [poles | start lattice]; the pole rows are filled afterwards.
-    pole_keys<<<1, 64, 0, c->stream>>>(trace_keys, (uint32_t)(N - 1) * (uint32_t)M);
-    BT_HIP(hipGetLastError());
+    // (Grid.h:325-338); the pole rows are filled once the rays are traced.
     io.keys = trace_keys;
     const int gap0 = 1 << (max_level - start_level);
     const unsigned npole = (unsigned)(M / gap0);
@@ -921,7 +924,7 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
     const int64_t nlat = (int64_t)nrows * ncols;
     const bool uniform = (max_level == start_level);
     start_lattice<<<blocks_for(nlat, 256), 256, 0, c->stream>>>(
-        G, gap0, nrows, ncols, trace_keys + 1 + eq, blocks + npole, uniform ? start_level : -1);
+        G, gap0, nrows, ncols, blocks + npole, uniform ? start_level : -1);
     BT_HIP(hipGetLastError());
     const auto fill_pole_rows = [&] {
         pole_rows<<<blocks_for(npole, 256), 256, 0, c->stream>>>(G, gap0, blocks);
@@ -934,23 +937,20 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
     }
 
     int level = start_level;
-    if (g->prm.precision == BT_PREC_FP64) {
+    {
         if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
         StatsK* spare = (StatsK*)p;
         std::vector<AheadGrid> a{{g, trace_keys, blocks, next, nb, gap0, 0, 0}};
-        rc = grid_ahead(
-            c, a, g->prm, thresh, d_stats,
-            [&](const std::vector<int64_t>& n) { return trace(c, g->pose, g->prm, n[0], io, spare); }, fill_pole_rows);
-        if (rc) return rc;
+        const auto trace_ahead = [&](const std::vector<int64_t>& n, const std::vector<RayTally*>& tallies) {
+            RayIO t = io;
+            t.tally = tallies[0];
+            return trace(c, g->pose, g->prm, n[0], t, spare);
+        };
+        if ((rc = grid_ahead(c, a, g->prm, thresh, d_stats, trace_ahead, fill_pole_rows))) return rc;
         level = a[0].level;
         nb = a[0].nb;
         blocks = a[0].blocks;
         next = a[0].next;
-    } else {
-        if ((rc = trace(c, g->pose, g->prm, 1 + eq + nlat, io, d_stats))) return rc;
-        g->rays += 1 + eq + nlat;
-        fill_pole_rows();
-        BT_HIP(hipGetLastError());
     }
 
     // adaptiveBlockIntegration(startLevel)
@@ -1049,7 +1049,6 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
         const bool uniform = (g->max_level == g->start_level);
         SetupJob& J = sj[k];
         J.G = Gk;
-        J.keys = per[k].keys;
         J.blocks = per[k].blocks;
         J.nm = NM;
         J.nwords = (NM + 31) / 32;
@@ -1064,7 +1063,6 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
         n_init += (NM + kInitSpan - 1) / kInitSpan * kInitSpan;
         n_lat += (nlat + 63) / 64 * 64;
         n_pole += npole;
-        counts[k] = 1 + eq + nlat;
         per[k].nb = npole;
         if (!uniform) {
             unsigned lat_blocks = nrows * ncols;
@@ -1098,12 +1096,14 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
     BT_HIP(hipGetLastError());
     start_lattice_multi<<<blocks_for(n_lat, 256), 256, 0, c->stream>>>(d_sj, G, n_lat);
     BT_HIP(hipGetLastError());
-    auto run_batch = [&](const std::vector<int64_t>& counts, StatsK* stats) -> int {
+    auto run_batch = [&](const std::vector<int64_t>& counts, StatsK* stats,
+                         const std::vector<RayTally*>* tallies = nullptr) -> int {
         BatchHost b;
         for (int k = 0; k < G; k++) {
             if (counts[k] <= 0) continue;
             b.poses.push_back(gs[k]->pose);
             b.ios.push_back(per[k].io);
+            if (tallies) b.ios.back().tally = (*tallies)[k];
             b.counts.push_back(counts[k]);
             gs[k]->rays += counts[k];
         }
@@ -1112,28 +1112,22 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
     const auto fill_pole_rows = [&] {
         pole_rows_multi<<<blocks_for(n_pole, 256), 256, 0, c->stream>>>(d_sj, G, n_pole);
     };
-    if (prm.precision == BT_PREC_FP64) {
+    {
         if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
         StatsK* spare = (StatsK*)p;
         std::vector<AheadGrid> a(G);
         for (int k = 0; k < G; k++)
             a[k] = AheadGrid{gs[k], per[k].keys, per[k].blocks, per[k].next, per[k].nb, sj[k].gap, 0, 0};
-        rc = grid_ahead(
-            c, a, prm, thresh, d_stats, [&](const std::vector<int64_t>& n) { return run_batch(n, spare); },
-            fill_pole_rows);
-        if (rc) return rc;
+        const auto trace_ahead = [&](const std::vector<int64_t>& n, const std::vector<RayTally*>& tallies) {
+            return run_batch(n, spare, &tallies);
+        };
+        if ((rc = grid_ahead(c, a, prm, thresh, d_stats, trace_ahead, fill_pole_rows))) return rc;
         for (int k = 0; k < G; k++) {
             per[k].level = a[k].level;
             per[k].nb = a[k].nb;
             per[k].blocks = a[k].blocks;
             per[k].next = a[k].next;
         }
-    } else {
-        // the poles and start lattices of all grids in one batch; the pole
-        // rows are filled once the pole rays are done
-        if ((rc = run_batch(counts, d_stats))) return rc;
-        fill_pole_rows();
-        BT_HIP(hipGetLastError());
     }
     // adaptiveBlockIntegration(startLevel), all grids one level per round
     std::vector<unsigned> h_ctr((size_t)kCtrStride * G);

@@ -98,6 +98,7 @@ __global__ __launch_bounds__(256) void ic_capture(Src S, ParamsK prm, int64_t n,
                 if (!prm.apriori && !P.a_zero) check_bq(P, b, q, prm.newton_cap, newton, &r0);
                 crit = !far_from_critical(P, b, q, r0, prm.crit_eps) &&
                        critical_distance(P, b, q, r0) < prm.crit_eps;
+                if (crit && io.tally) io.tally[kl].fallback++;
             }
         }
         if (escapes) {
@@ -118,6 +119,14 @@ __global__ __launch_bounds__(256) void ic_capture(Src S, ParamsK prm, int64_t n,
     const unsigned long long cnt[5] = {c_rays, c_int, c_nw, c_gd, c_cr};
     unsigned long long* const dst[5] = {&st->rays, &st->integrated, &st->newton, &st->golden, &st->fallback};
     block_add_stats<5>(cnt, dst);
+}
+
+template <class Src>
+__device__ __forceinline__ void tally_fp64(const Src& S, int sg, int64_t slot, int attempts) {
+    if (!S.rio(sg).tally) return;
+    RayTally& t = S.rio(sg).tally[S.local(sg, slot)];
+    t.attempts += (uint32_t)attempts;
+    t.fp64 += (uint32_t)attempts;
 }
 
 // WARM = false: every ray runs to its end (the plain FP64 path).  WARM =
@@ -211,6 +220,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == kWa
                 }
                 ray_store(S.rio(sg), S.local(sg, slot), th, ph, step);
                 if (WARM) cont.nstp[slot] = -1;
+                tally_fp64(S, sg, slot, nstp);
                 slot = -1;
             } else if (WARM && em > ERRCON) {
 #pragma unroll
@@ -218,6 +228,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == kWa
                 cont.y[5 * cont.stride + slot] = z;
                 cont.h[slot] = h;
                 cont.nstp[slot] = nstp;
+                tally_fp64(S, sg, slot, nstp);
                 slot = -1;
             }
         }

@@ -347,6 +347,11 @@ __global__ __launch_bounds__(256, 5) void rk_mixed(Src S, ParamsK prm, QueueK Q,
         }
         queue_push(Q64, restart || flagged, (uint32_t)slot, lane);
         if (restart || flagged) restarts++;
+        if (done && S.rio(sg).tally) {
+            RayTally& t = S.rio(sg).tally[S.local(sg, slot)];
+            t.attempts += (uint32_t)(nstp - cont.nstp[slot]);
+            t.fallback += restart || flagged;
+        }
         if (done) slot = -1;
     }
     const unsigned long long cnt[2] = {attempts, restarts};
@@ -355,13 +360,6 @@ __global__ __launch_bounds__(256, 5) void rk_mixed(Src S, ParamsK prm, QueueK Q,
 }
 
 }  // namespace
-
-// Below this tolerance FP32 cannot carry the step control: the rounding of
-// the FP32 stage sums (unit roundoff 6e-8, relative to |y| + |h y'|) is no
-// longer small against eps, so the error estimate turns into noise, steps
-// collapse and the FP32 right-hand side's rounding accumulates into the
-// angles.  The mixed mode then traces every ray in FP64.
-constexpr double kMixedEpsMin = 1e-6;
 
 namespace {
 // phase 0: snapshot the integrated-ray count; phase 1: add the rays

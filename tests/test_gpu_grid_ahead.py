@@ -14,7 +14,7 @@ import blacktracer_amd as bt
 
 pytestmark = pytest.mark.gpu
 
-COUNTS = ("rays", "integrated", "attempts", "newton", "golden")
+COUNTS = ("rays", "integrated", "attempts", "attempts_fp64", "newton", "golden", "fallback_rays")
 
 
 def traced_directions(g):
@@ -33,18 +33,26 @@ def camera(k):
     return bt.Camera(math.pi / 2 - 0.1 * k, 0.0, 4.0 + k, black_hole=hole), hole
 
 
-@pytest.mark.parametrize("level,start,angle,thresh", [
-    (1, 1, True, 0.015), (2, 1, False, 0.015), (5, 5, True, 0.015), (8, 1, True, 0.015), (8, 3, False, 0.015),
-    (9, 6, True, 0.015), (8, 2, True, 1e9), (10, 1, False, 0.1)])
-def test_same_grid_and_counts(ctx, level, start, angle, thresh):
+FP64, MIXED = {}, {"precision": bt.BT_PREC_MIXED}
+
+
+@pytest.mark.parametrize("level,start,angle,thresh,prm", [
+    (1, 1, True, 0.015, FP64), (2, 1, False, 0.015, FP64), (5, 5, True, 0.015, FP64), (8, 1, True, 0.015, FP64),
+    (8, 3, False, 0.015, FP64), (9, 6, True, 0.015, FP64), (8, 2, True, 1e9, FP64), (10, 1, False, 0.1, FP64),
+    (1, 1, False, 0.015, MIXED), (8, 1, True, 0.015, MIXED), (8, 4, False, 0.015, MIXED), (9, 1, True, 0.1, MIXED),
+    (6, 2, True, 0.015, {**MIXED, "eps": 1e-8}), (7, 1, True, 0.015, {**MIXED, "apriori_capture": 0, "r_capture_factor": 1.01}),
+    (7, 1, True, 0.015, {**FP64, "max_steps": 60})])
+def test_same_grid_and_counts(ctx, level, start, angle, thresh, prm):
     n = 3 if level > 9 else 36
     cams, holes = zip(*[camera(k % 5) for k in range(n)])
-    print(f"batch of {n} Grid({level},{start},angle={angle}) thresh={thresh}", flush=True)
-    batch, stats = bt.Grid.build_batch(cams, holes, [level] * n, [start] * n, angle=angle, refine_thresh=thresh,
-                                       fix_tvertices=False, ctx=ctx)
+    prm = bt.IntegParams(**prm)
+    print(f"batch of {n} Grid({level},{start},angle={angle}) thresh={thresh} precision={prm.precision}", flush=True)
+    batch, stats = bt.Grid.build_batch(cams, holes, [level] * n, [start] * n, angle=angle, params=prm,
+                                       refine_thresh=thresh, fix_tvertices=False, ctx=ctx)
     total = dict.fromkeys(COUNTS, 0)
     for k in range(min(n, 5)):
-        g = bt.Grid(level, start, angle, cams[k], holes[k], refine_thresh=thresh, fix_tvertices=False, ctx=ctx)
+        g = bt.Grid(level, start, angle, cams[k], holes[k], params=prm, refine_thresh=thresh, fix_tvertices=False,
+                    ctx=ctx)
         for h in batch[k::5]:
             assert g.rays_traced == h.rays_traced
             assert np.array_equal(g.cel, h.cel) and np.array_equal(g.steps, h.steps)
@@ -52,7 +60,7 @@ def test_same_grid_and_counts(ctx, level, start, angle, thresh):
         assert not g.steps[g.cel[..., 0] == -2].any()
         th, ph = traced_directions(g)
         assert th.size == g.rays_traced
-        *_, want = bt.trace_rays(cams[k], th, ph, ctx=ctx, return_stats=True)
+        *_, want = bt.trace_rays(cams[k], th, ph, params=prm, ctx=ctx, return_stats=True)
         assert {c: g.stats()[c] for c in COUNTS} == {c: want[c] for c in COUNTS}
         for c in COUNTS:
             total[c] += want[c] * len(batch[k::5])
