@@ -308,7 +308,10 @@ __global__ void final_level(GridK G, const uint32_t* blocks, unsigned nb, int le
 // S then refine without tracing, on device counts.
 // Afterwards the lattice points that no block asked for go back to their
 // untraced values, and the rays that were asked for are counted: the grid, its
-// ray count and its statistics are those of the level-by-level build.
+// ray count and its statistics are those of the level-by-level build.  Where
+// the start level is as fine as that already (a uniform grid), its rays alone
+// are traced and counted as they are: counting the 8.4 million of a 2049 x 4096
+// sky afterwards would cost 0.7 ms.
 //
 // A level-10 grid built level by level took ten launches of about 1 ms.
 struct AheadJob {
@@ -322,6 +325,7 @@ struct AheadJob {
     uint32_t npts, ncols;
     unsigned nb0;         // blocks of the start level
     int S, gap0;
+    int plain;            // no level ahead: keys are the poles, then the start lattice
 };
 constexpr int kAheadLevels = 16;   // levels of a grid, at most 12
 
@@ -340,6 +344,10 @@ __device__ __forceinline__ const AheadJob& ahead_job(const AheadJob* jobs, int n
 }
 
 __device__ __forceinline__ uint32_t ahead_key(const AheadJob& J, uint32_t t) {
+    if (J.plain) {
+        if (t < 1u + J.G.eq) return t * (uint32_t)(J.G.N - 1) * (uint32_t)J.G.M;
+        t += J.ncols - 1u - J.G.eq;   // the lattice from its second row on
+    }
     const int shift = J.G.max_level - J.S;
     return ((t / J.ncols) << shift) * (uint32_t)J.G.M + ((t % J.ncols) << shift);
 }
@@ -776,8 +784,8 @@ int64_t lattice_points(const bt_grid* g, int level) {
 }
 
 // The levels of `gs` below the one traced ahead (see above).  The grids are
-// initialised and their start lattices marked; `trace_keys(counts, tallies)`
-// traces the first counts[k] keys of grid k, outside the build's statistics.
+// initialised and their start lattices marked; `trace_keys(counts, tallies,
+// stats)` traces the first counts[k] keys of grid k.
 template <class Trace, class PoleRows>
 int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, double thresh, StatsK* d_stats,
                Trace&& trace_keys, PoleRows&& fill_pole_rows) {
@@ -798,6 +806,10 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
     void* p;
     if ((rc = c->buffer("ahead_ctr", sizeof(unsigned) * ctr_words * n, &p))) return rc;
     unsigned* ctr = (unsigned*)p;
+    if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
+    StatsK* spare = (StatsK*)p;   // takes what the trace counts beside the build's rays
+    bool ahead = false;
+    for (const AheadGrid& a : gs) ahead = ahead || level_of(a.g, s) > a.g->start_level;
     int64_t items = 0;
     int lmin = 99, lmax = 0;
     unsigned most = 1;
@@ -813,7 +825,10 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
         J.ctr = ctr + ctr_words * k;
         J.item0 = items;
         J.S = level_of(a.g, s);
+        J.plain = !ahead;
+        // without the pole rows, whose points at the start spacing are copies
         counts[k] = lattice_points(a.g, J.S);
+        if (!ahead) counts[k] -= (int64_t)(1 + a.g->eq) * (a.g->M / a.gap0 - 1);
         J.npts = (uint32_t)counts[k];
         J.ncols = (uint32_t)a.g->M >> (a.g->max_level - J.S);
         J.nb0 = a.nb0;
@@ -824,7 +839,7 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
         // the blocks of level S - 1, at most
         if (J.S > a.g->start_level) most = std::max(most, (J.npts + 3) / 4);
     }
-    if (prm.precision == BT_PREC_MIXED) {
+    if (ahead && prm.precision == BT_PREC_MIXED) {
         if ((rc = c->buffer("ahead_tally", sizeof(RayTally) * items, &p))) return rc;
         for (int k = 0; k < n; k++) tallies[k] = jobs[k].tally = (RayTally*)p + jobs[k].item0;
     }
@@ -838,11 +853,11 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
     ahead_keys<<<blocks_for(items, 256), 256, 0, c->stream>>>(d_jobs, n, items);
     zero_span<<<blocks_for((int64_t)ctr_words * n, 256), 256, 0, c->stream>>>(ctr, (int)(ctr_words * n));
     BT_HIP(hipGetLastError());
-    if ((rc = trace_keys(counts, tallies))) return rc;
-    ahead_poles<<<(unsigned)n, 64, 0, c->stream>>>(d_jobs, prm, d_stats);
+    if ((rc = trace_keys(counts, tallies, ahead ? spare : d_stats))) return rc;
+    if (ahead) ahead_poles<<<(unsigned)n, 64, 0, c->stream>>>(d_jobs, prm, d_stats);
     fill_pole_rows();
     BT_HIP(hipGetLastError());
-    {
+    if (ahead) {
         KTimer t(c, "refine_level");
         for (int level = lmin; level < lmax; level++)
             ahead_refine<<<dim3(std::min(blocks_for(most, 256), 256u), (unsigned)n), 256, 0, c->stream>>>(d_jobs, level,
@@ -938,13 +953,11 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
 
     int level = start_level;
     {
-        if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
-        StatsK* spare = (StatsK*)p;
         std::vector<AheadGrid> a{{g, trace_keys, blocks, next, nb, gap0, 0, 0}};
-        const auto trace_ahead = [&](const std::vector<int64_t>& n, const std::vector<RayTally*>& tallies) {
+        const auto trace_ahead = [&](const std::vector<int64_t>& n, const std::vector<RayTally*>& tallies, StatsK* st) {
             RayIO t = io;
             t.tally = tallies[0];
-            return trace(c, g->pose, g->prm, n[0], t, spare);
+            return trace(c, g->pose, g->prm, n[0], t, st);
         };
         if ((rc = grid_ahead(c, a, g->prm, thresh, d_stats, trace_ahead, fill_pole_rows))) return rc;
         level = a[0].level;
@@ -1113,13 +1126,11 @@ int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_
         pole_rows_multi<<<blocks_for(n_pole, 256), 256, 0, c->stream>>>(d_sj, G, n_pole);
     };
     {
-        if ((rc = c->buffer("ahead_stats", sizeof(StatsK), &p))) return rc;
-        StatsK* spare = (StatsK*)p;
         std::vector<AheadGrid> a(G);
         for (int k = 0; k < G; k++)
             a[k] = AheadGrid{gs[k], per[k].keys, per[k].blocks, per[k].next, per[k].nb, sj[k].gap, 0, 0};
-        const auto trace_ahead = [&](const std::vector<int64_t>& n, const std::vector<RayTally*>& tallies) {
-            return run_batch(n, spare, &tallies);
+        const auto trace_ahead = [&](const std::vector<int64_t>& n, const std::vector<RayTally*>& tallies, StatsK* st) {
+            return run_batch(n, st, &tallies);
         };
         if ((rc = grid_ahead(c, a, prm, thresh, d_stats, trace_ahead, fill_pole_rows))) return rc;
         for (int k = 0; k < G; k++) {

@@ -67,3 +67,20 @@ def test_same_grid_and_counts(ctx, level, start, angle, thresh, prm):
     assert {c: stats[c] for c in COUNTS} == total
     for h in batch:
         h.close()
+
+
+def test_uniform_batch_counts(ctx):
+    """A batch whose grids all start at their last level, and one that mixes
+    such grids with adaptive ones, against the single grids."""
+    for levels, starts in (([7, 6, 7], [7, 6, 7]), ([7, 7, 6], [7, 2, 6])):
+        cams, holes = zip(*[camera(k) for k in range(3)])
+        print(f"batch of levels {levels} from {starts}", flush=True)
+        batch, stats = bt.Grid.build_batch(cams, holes, levels, starts, ctx=ctx)
+        total = dict.fromkeys(COUNTS, 0)
+        for k, h in enumerate(batch):
+            g = bt.Grid(levels[k], starts[k], True, cams[k], holes[k], ctx=ctx)
+            assert g.rays_traced == h.rays_traced and g.rays_traced == g.stats()["rays"]
+            assert np.array_equal(g.cel, h.cel) and np.array_equal(g.steps, h.steps)
+            for c in COUNTS:
+                total[c] += g.stats()[c]
+        assert {c: stats[c] for c in COUNTS} == total
