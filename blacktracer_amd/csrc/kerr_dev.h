@@ -613,16 +613,22 @@ struct LanePose {
 
 // Launch shape of a persistent kernel: one resident set of workgroups
 // (Context::tune: block size, resident waves per SIMD), never more than the
-// rays need.
+// rays need.  Where the rays need less than a wave per SIMD, the waves are
+// workgroups of their own, so that the dispatcher spreads them over the CUs;
+// and where they all fit the launch, a wave reserves no more queue positions
+// than it has lanes (with 128 of them half of the waves stayed empty while the
+// others' freed lanes took a second ray, at the end of which the launch ends):
+// 500 rays took 1070 us, with small workgroups 938, with both 720.
 struct Launch {
-    unsigned blocks, threads;
+    unsigned blocks, threads, chunk;
 };
 
 template <class K>
 int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L) {
-    const int threads = (int)c->tune.block;
+    int threads = (int)c->tune.block;
     if (threads != 64 && threads != 128 && threads != 256)
         return fail(BT_ERR_INVALID, "tune: block size must be 64, 128 or 256");
+    if (n_max < (int64_t)c->num_cus * 4 * 64) threads = 64;
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, threads, 0) != hipSuccess || occ < 1)
         occ = 1;
@@ -637,6 +643,7 @@ int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L) {
     if (blocks < 1) blocks = 1;
     L->blocks = (unsigned)blocks;
     L->threads = (unsigned)threads;
+    L->chunk = n_max <= blocks * threads ? 64u : c->tune.chunk;
     if (blocks * threads > c->launch_lanes) c->launch_lanes = blocks * threads;
     return BT_OK;
 }

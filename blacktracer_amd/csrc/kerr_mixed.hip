@@ -454,7 +454,7 @@ int trace_mixed_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, Sta
             return rc;
         }
         rk_mixed<Src><<<L.blocks, L.threads, 0, c->stream>>>(S, prm, Qw, head32, Qr, cont, d_stats, restart_at,
-                                                             c->tune.chunk);
+                                                             L.chunk);
         if (hipGetLastError() != hipSuccess) {
             (void)join();
             return fail(BT_ERR_HIP, "rk_mixed launch failed");
