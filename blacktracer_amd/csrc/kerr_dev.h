@@ -619,16 +619,18 @@ struct LanePose {
 // than it has lanes (with 128 of them half of the waves stayed empty while the
 // others' freed lanes took a second ray, at the end of which the launch ends):
 // 500 rays took 1070 us, with small workgroups 938, with both 720.
+// Not `spread`: the FP32 bulk keeps its workgroups (of 8 rays it took 108 us in
+// one of one wave, 99 to 105 in one of four).
 struct Launch {
     unsigned blocks, threads, chunk;
 };
 
 template <class K>
-int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L) {
+int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L, bool spread = true) {
     int threads = (int)c->tune.block;
     if (threads != 64 && threads != 128 && threads != 256)
         return fail(BT_ERR_INVALID, "tune: block size must be 64, 128 or 256");
-    if (n_max < (int64_t)c->num_cus * 4 * 64) threads = 64;
+    if (spread && n_max < (int64_t)c->num_cus * 4 * 64) threads = 64;
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, threads, 0) != hipSuccess || occ < 1)
         occ = 1;

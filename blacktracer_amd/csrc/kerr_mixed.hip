@@ -449,7 +449,7 @@ int trace_mixed_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, Sta
     {
         KTimer t(c, "rk_mixed");
         Launch L;
-        if ((rc = persistent_launch(c, rk_mixed<Src>, n, &L))) {
+        if ((rc = persistent_launch(c, rk_mixed<Src>, n, &L, false))) {
             (void)join();
             return rc;
         }
