@@ -287,7 +287,8 @@ int trace_f64(Context* c, const PoseK& pose, const ParamsK& prm, int64_t n, cons
 // its initial state (at most n_max rays); with cont given (warm-up mode) a
 // ray leaves after its first attempt with errmax > ERRCON and its state
 // goes to cont (cont.nstp = -1 for a ray that ended during the warm-up);
-// prio is the waves' base issue priority (0..3).
+// prio is the waves' base issue priority (0..3); tuned_chunk: its waves reserve
+// as tuned also where n_max lanes fit the launch (persistent_launch).
 // Zeroes n (<= 1024) 32-bit words with a kernel (no memset node, so the
 // call can sit in a captured graph).
 int zero_words(unsigned* p, int n, hipStream_t st);
@@ -298,7 +299,7 @@ int trace_setup(Context* c, const Src& S, const ParamsK& prm, int64_t n, const Q
 template <class Src>
 int trace_f64_queue(Context* c, const Src& S, const ParamsK& prm, int64_t n_max, const QueueK& Q,
                     StatsK* d_stats, const char* timer, const ContK* cont,
-                    hipStream_t stream = nullptr, int prio = 0);
+                    hipStream_t stream = nullptr, int prio = 0, bool tuned_chunk = false);
 template <class Src>
 int trace_f64_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, StatsK* d_stats);
 // kerr_mixed.hip: FP32 bulk with FP64 set-up, warm-up, fallback and accumulation.

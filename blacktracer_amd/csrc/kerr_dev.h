@@ -615,7 +615,7 @@ struct LanePose {
 // (Context::tune: block size, resident waves per SIMD), never more than the
 // rays need.  Where the rays need less than a wave per SIMD, the waves are
 // workgroups of their own, so that the dispatcher spreads them over the CUs;
-// and where they all fit the launch, a wave reserves no more queue positions
+// and where n_max lanes fit the launch, a wave reserves no more queue positions
 // than it has lanes (with 128 of them half of the waves stayed empty while the
 // others' freed lanes took a second ray, at the end of which the launch ends):
 // 500 rays took 1070 us, with small workgroups 938, with both 720.

@@ -332,7 +332,8 @@ int trace_setup(Context* c, const Src& S, const ParamsK& prm, int64_t n, const Q
 
 template <class Src>
 int trace_f64_queue(Context* c, const Src& S, const ParamsK& prm, int64_t n_max, const QueueK& Q,
-                    StatsK* d_stats, const char* timer, const ContK* cont, hipStream_t stream, int prio) {
+                    StatsK* d_stats, const char* timer, const ContK* cont, hipStream_t stream, int prio,
+                    bool tuned_chunk) {
     if (!stream) stream = c->stream;
     KTimer t(c, timer, stream);
     Launch L;
@@ -341,6 +342,7 @@ int trace_f64_queue(Context* c, const Src& S, const ParamsK& prm, int64_t n_max,
         rk_f64<kWarm, Src><<<L.blocks, L.threads, 0, stream>>>(S, prm, Q, d_stats, L.chunk, *cont, prio);
     } else {
         if (int rc = persistent_launch(c, rk_f64<kExact, Src>, n_max, &L)) return rc;
+        if (tuned_chunk) L.chunk = c->tune.chunk;
         rk_f64<kExact, Src><<<L.blocks, L.threads, 0, stream>>>(S, prm, Q, d_stats, L.chunk, ContK{},
                                                                 prio);
     }
@@ -353,9 +355,9 @@ template int trace_setup<SingleSrc>(Context*, const SingleSrc&, const ParamsK&, 
 template int trace_setup<MultiSrc>(Context*, const MultiSrc&, const ParamsK&, int64_t, const QueueK&,
                                    const QueueK*, StatsK*);
 template int trace_f64_queue<SingleSrc>(Context*, const SingleSrc&, const ParamsK&, int64_t, const QueueK&,
-                                        StatsK*, const char*, const ContK*, hipStream_t, int);
+                                        StatsK*, const char*, const ContK*, hipStream_t, int, bool);
 template int trace_f64_queue<MultiSrc>(Context*, const MultiSrc&, const ParamsK&, int64_t, const QueueK&,
-                                       StatsK*, const char*, const ContK*, hipStream_t, int);
+                                       StatsK*, const char*, const ContK*, hipStream_t, int, bool);
 
 template <class Src>
 int trace_f64_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, StatsK* d_stats) {

@@ -425,13 +425,26 @@ int trace_mixed_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, Sta
     const int margin = prm.max_steps / 16 > 16 ? prm.max_steps / 16 : 16;
     const int restart_at = prm.max_steps - margin > 1 ? prm.max_steps - margin : 1;
     if ((rc = trace_setup(c, S, prm, n, Qw, &Qc, d_stats))) return rc;
-    // fork: critical rays on the auxiliary stream, at most one workgroup per CU
+    // From three quarters of a wave per SIMD to three of them, the bulk and the
+    // critical rays' launch, which run at a time, reserve as tuned though their
+    // rays fit: the critical rays' waves issue first and hold up the bulk's on
+    // their SIMDs, so fewer of them hold up less, and a bulk wave that has
+    // reserved its 64 rays keeps them while lanes elsewhere run empty.  The call
+    // took, with 64 positions and with 128: 90000 rays 1980 and 1605 us, 120000
+    // 2180 and 1735, 150000 2630 and 2265, 180000 2650 and 2500.  Below and
+    // above, the waves have SIMDs of their own, or every SIMD has its share
+    // (20000 rays: 1105 and 1218 us, 325624: 2196 and 2448; 600000 with the
+    // critical rays' launch alone as tuned: 3915 and 4200).
+    const int64_t simds = (int64_t)c->num_cus * 4;
+    const bool tuned = n > simds * 48 && n <= simds * 64 * 3;
+    // fork: critical rays on the auxiliary stream, on the lanes of one workgroup
+    // per CU at most
     BT_HIP(hipEventRecord(c->ev_fork, c->stream));
     BT_HIP(hipStreamWaitEvent(c->aux, c->ev_fork, 0));
     const int64_t crit_lanes = (int64_t)c->num_cus * c->tune.block;
     // the critical rays' waves issue ahead of the bulk's (base priority 1)
     rc = trace_f64_queue(c, S, prm, n < crit_lanes ? n : crit_lanes, Qc, d_stats, "rk_f64_critical",
-                         nullptr, c->aux, 1);
+                         nullptr, c->aux, 1, tuned);
     // join (also on error, so that nothing is left running on the aux stream)
     auto join = [&]() -> hipError_t {
         const hipError_t e = hipEventRecord(c->ev_join, c->aux);
@@ -453,6 +466,7 @@ int trace_mixed_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, Sta
             (void)join();
             return rc;
         }
+        if (tuned) L.chunk = c->tune.chunk;
         rk_mixed<Src><<<L.blocks, L.threads, 0, c->stream>>>(S, prm, Qw, head32, Qr, cont, d_stats, restart_at,
                                                              L.chunk);
         if (hipGetLastError() != hipSuccess) {
