@@ -333,6 +333,14 @@ constexpr int kAheadLevels = 16;   // levels of a grid, at most 12
 // together): a few rays for every lane the chip holds.
 constexpr int64_t kAheadRays = int64_t(3) << 18;
 
+// No two grid values are this far apart (squared; theta' in [0, pi] and phi' in
+// [0, 2 pi], or -1 each): from this threshold on, as with one that is no
+// number, refine_test refines below level 6 alone, and a finer lattice traced
+// ahead would be thrown away (a level-10 grid from level 6 took 2550 us with
+// it, 1330 level by level; at a threshold of 60, where the shadow's edge still
+// refines down to the last level, 3050 against 3920).
+constexpr double kFarthest = 71.0;
+
 __device__ __forceinline__ const AheadJob& ahead_job(const AheadJob* jobs, int njobs, int64_t t) {
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
@@ -797,7 +805,8 @@ int grid_ahead(Context* c, std::vector<AheadGrid>& gs, const ParamsK& prm, doubl
         return t;
     };
     int s = 1;
-    while (s < 12 && total(s + 1) <= kAheadRays) s++;
+    const int deepest = thresh < kFarthest ? 12 : 6;
+    while (s < deepest && total(s + 1) <= kAheadRays) s++;
     std::vector<AheadJob> jobs(n);
     std::vector<int64_t> counts(n);
     std::vector<RayTally*> tallies(n, nullptr);

@@ -84,3 +84,37 @@ def test_uniform_batch_counts(ctx):
             for c in COUNTS:
                 total[c] += g.stats()[c]
         assert {c: stats[c] for c in COUNTS} == total
+
+
+@pytest.mark.parametrize("prm", [FP64, MIXED])
+def test_threshold_beyond_every_jump(ctx, prm):
+    """Thresholds above the largest distance of two grid values, infinite and
+    no number: the grid of the largest threshold below it, and no finer
+    lattice traced for it than the blocks that always refine ask for."""
+    cam, hole = camera(1)
+    prm = bt.IntegParams(**prm)
+    name = "ic_split" if prm.precision == bt.BT_PREC_MIXED else "ic_capture_f64"
+
+    def build(level, start, thresh):
+        print(f"Grid({level},{start}) thresh={thresh} precision={prm.precision}", flush=True)
+        g = bt.Grid(level, start, True, cam, hole, params=prm, refine_thresh=thresh, ctx=ctx)
+        return g, (g.cel, g.steps, g.levels, g.rays_traced)
+
+    for level, start in ((5, 1), (9, 2), (9, 6), (9, 7), (8, 8)):
+        _, want = build(level, start, 70.5)
+        for thresh in (71.0, 1e300, math.inf, math.nan):
+            _, got = build(level, start, thresh)
+            assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        assert want[2].max() == max(start, min(level, 6))
+    capture = []
+    ctx.timing(True)
+    try:
+        for thresh in (70.5, 71.0):
+            build(12, 6, thresh)   # buffers
+            ctx.reset_timers()
+            build(12, 6, thresh)
+            capture.append(ctx.timer(name)[1])
+    finally:
+        ctx.timing(False)
+    print(f"capture test {capture} ms", flush=True)
+    assert capture[1] < 0.5 * capture[0]
