@@ -78,7 +78,8 @@ int Context::copy(const std::vector<CopySeg>& segs, bool to_device) {
     if (!staged || total < kCopyLarge) {
         for (const CopySeg& s : segs)
             if (s.bytes) BT_HIP(hipMemcpyAsync(s.dst, s.src, s.bytes, kind, stream));
-        if (!to_device) BT_HIP(hipStreamSynchronize(stream));
+        // the runtime has read a pageable source when its call returns, a pinned one it may still read
+        if (!to_device || !staged) BT_HIP(hipStreamSynchronize(stream));
         return BT_OK;
     }
     if (int rc = copy_slots()) return rc;
