@@ -224,8 +224,8 @@ struct Context {
     static constexpr int kCopySlots = 12;
     void* copy_stage = nullptr;   // kCopySlots pinned pieces of 2 MiB
     hipEvent_t ev_copy[kCopySlots] = {};
-    int copy(const std::vector<CopySeg>& segs, bool to_device);
-    int copy_slots();
+    int copy(const CopySeg* segs, int nsegs, bool to_device);
+    bool copy_slots();
     void release_copy_slots();
     int timer_begin(const char* name, int* slot, hipStream_t st = nullptr);
     int timer_end(int slot);

@@ -13,7 +13,6 @@
 #include <cstring>
 #include <system_error>
 #include <thread>
-#include <vector>
 
 #include "bt_internal.h"
 
@@ -49,15 +48,20 @@ struct Piece {
 
 }  // namespace
 
-int Context::copy_slots() {
+// The pinned pieces and their events; false where the runtime has none to give.
+bool Context::copy_slots() {
     for (int k = 0; k < kCopySlots; k++)
-        if (!ev_copy[k] && hipEventCreateWithFlags(&ev_copy[k], hipEventDisableTiming) != hipSuccess)
-            return fail(BT_ERR_HIP, "copy: event creation failed");
+        if (!ev_copy[k] && hipEventCreateWithFlags(&ev_copy[k], hipEventDisableTiming) != hipSuccess) {
+            ev_copy[k] = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
     if (!copy_stage && hipHostMalloc(&copy_stage, kCopySlots * kPiece, 0) != hipSuccess) {
         copy_stage = nullptr;
-        return fail(BT_ERR_NOMEM, "hipHostMalloc failed for the copy pieces");
+        (void)hipGetLastError();
+        return false;
     }
-    return BT_OK;
+    return true;
 }
 
 void Context::release_copy_slots() {
@@ -67,26 +71,30 @@ void Context::release_copy_slots() {
     copy_stage = nullptr;
 }
 
-int Context::copy(const std::vector<CopySeg>& segs, bool to_device) {
+int Context::copy(const CopySeg* segs, int nsegs, bool to_device) {
     const hipMemcpyKind kind = to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
-    size_t total = 0;
-    bool staged = true;
-    for (const CopySeg& s : segs) {
-        total += s.bytes;
-        if (s.bytes && is_pinned(to_device ? s.src : s.dst)) staged = false;
+    size_t total = 0, npieces = 0;
+    bool pageable = true;
+    for (int s = 0; s < nsegs; s++) {
+        total += segs[s].bytes;
+        npieces += (segs[s].bytes + kPiece - 1) / kPiece;
+        if (segs[s].bytes && is_pinned(to_device ? segs[s].src : segs[s].dst)) pageable = false;
     }
-    if (!staged || total < kCopyLarge) {
-        for (const CopySeg& s : segs)
-            if (s.bytes) BT_HIP(hipMemcpyAsync(s.dst, s.src, s.bytes, kind, stream));
+    // also where there is no pinned memory for the pieces
+    if (!pageable || total < kCopyLarge || !copy_slots()) {
+        for (int s = 0; s < nsegs; s++)
+            if (segs[s].bytes) BT_HIP(hipMemcpyAsync(segs[s].dst, segs[s].src, segs[s].bytes, kind, stream));
         // the runtime has read a pageable source when its call returns, a pinned one it may still read
-        if (!to_device || !staged) BT_HIP(hipStreamSynchronize(stream));
+        if (!to_device || !pageable) BT_HIP(hipStreamSynchronize(stream));
         return BT_OK;
     }
-    if (int rc = copy_slots()) return rc;
-    std::vector<Piece> pieces;
-    for (const CopySeg& s : segs)
-        for (size_t o = 0; o < s.bytes; o += kPiece)
-            pieces.push_back(Piece{(char*)s.dst + o, (const char*)s.src + o, std::min(kPiece, s.bytes - o)});
+    const auto piece = [&](size_t n) {
+        for (int s = 0;; s++) {
+            const size_t m = (segs[s].bytes + kPiece - 1) / kPiece, o = n * kPiece;
+            if (n < m) return Piece{(char*)segs[s].dst + o, (const char*)segs[s].src + o, std::min(kPiece, segs[s].bytes - o)};
+            n -= m;
+        }
+    };
     std::atomic<size_t> next{0};
     std::atomic<int> error{(int)hipSuccess};
     const auto worker = [&](int w) {
@@ -97,39 +105,39 @@ int Context::copy(const std::vector<CopySeg>& segs, bool to_device) {
         if (!ok(hipSetDevice(device))) return;
         char* slot[2] = {(char*)copy_stage + (2 * w) * kPiece, (char*)copy_stage + (2 * w + 1) * kPiece};
         hipEvent_t ev[2] = {ev_copy[2 * w], ev_copy[2 * w + 1]};
-        const Piece* open[2] = {nullptr, nullptr};   // device to host: on its way into the slot
+        Piece open[2] = {};   // device to host: on its way into the slot
         for (int k = 0;; k ^= 1) {
             // the slot's last copy is done (an event never recorded is)
-            if (!to_device || next.load() < pieces.size())
+            if (!to_device || next.load() < npieces)
                 if (!ok(hipEventSynchronize(ev[k]))) return;
-            if (open[k]) std::memcpy(open[k]->dst, slot[k], open[k]->bytes);
-            open[k] = nullptr;
-            const size_t n = error.load() == (int)hipSuccess ? next.fetch_add(1) : pieces.size();
-            if (n < pieces.size()) {
-                const Piece& p = pieces[n];
+            if (open[k].bytes) std::memcpy(open[k].dst, slot[k], open[k].bytes);
+            open[k].bytes = 0;
+            const size_t n = error.load() == (int)hipSuccess ? next.fetch_add(1) : npieces;
+            if (n < npieces) {
+                const Piece p = piece(n);
                 if (to_device) {
                     std::memcpy(slot[k], p.src, p.bytes);
                     if (!ok(hipMemcpyAsync(p.dst, slot[k], p.bytes, kind, stream))) return;
                 } else {
                     if (!ok(hipMemcpyAsync(slot[k], p.src, p.bytes, kind, stream))) return;
-                    open[k] = &p;
+                    open[k] = p;
                 }
                 if (!ok(hipEventRecord(ev[k], stream))) return;
-            } else if (!open[k ^ 1]) {
+            } else if (!open[k ^ 1].bytes) {
                 return;
             }
         }
     };
-    std::vector<std::thread> threads;
+    std::thread threads[kCopyThreads];
     const int want = (int)std::min<size_t>(kCopyThreads, total / kCopyPerThread);
     try {
-        threads.reserve(want);
-        for (int w = 1; w < want; w++) threads.emplace_back(worker, w);
+        for (int w = 1; w < want; w++) threads[w] = std::thread(worker, w);
     } catch (const std::exception&) {
         // fewer threads share the pieces then
     }
     worker(0);
-    for (std::thread& t : threads) t.join();
+    for (std::thread& t : threads)
+        if (t.joinable()) t.join();
     if (error.load() != (int)hipSuccess) {
         (void)hipStreamSynchronize(stream);
         return fail(BT_ERR_HIP, std::string("copy: ") + hipGetErrorString((hipError_t)error.load()));

@@ -128,11 +128,10 @@ int bt_grid_export(const bt_grid* g, double* cel, int32_t* steps, int8_t* levels
     std::lock_guard<std::recursive_mutex> lk(c.mu);
     BT_HIP(hipSetDevice(c.device));
     const int64_t NM = (int64_t)g->N * g->M;
-    std::vector<CopySeg> segs;
-    if (cel) segs.push_back({cel, g->k.cel, sizeof(double) * 2 * NM});
-    if (steps) segs.push_back({steps, g->k.steps, sizeof(int32_t) * NM});
-    if (levels) segs.push_back({levels, g->k.level, (size_t)NM});
-    return c.copy(segs, false);
+    const CopySeg segs[] = {{cel, g->k.cel, cel ? sizeof(double) * 2 * NM : 0},
+                            {steps, g->k.steps, steps ? sizeof(int32_t) * NM : 0},
+                            {levels, g->k.level, levels ? (size_t)NM : 0}};
+    return c.copy(segs, 3, false);
 }
 
 int bt_grid_export_psh(const bt_grid* g, int* hash_width, int* offset_width, float* hash_table,
@@ -145,10 +144,9 @@ int bt_grid_export_psh(const bt_grid* g, int* hash_width, int* offset_width, flo
     const int64_t nwords = (NM + 31) / 32;
     std::vector<double> cel(2 * NM);
     std::vector<uint32_t> present(nwords);
-    if (int crc = c.copy({{cel.data(), g->k.cel, sizeof(double) * 2 * NM},
-                          {present.data(), g->k.present, sizeof(uint32_t) * nwords}},
-                         false))
-        return crc;
+    const CopySeg segs[] = {{cel.data(), g->k.cel, sizeof(double) * 2 * NM},
+                            {present.data(), g->k.present, sizeof(uint32_t) * nwords}};
+    if (int crc = c.copy(segs, 2, false)) return crc;
     // Grid.h:645-651: every CamToCel entry, as float2
     std::vector<int32_t> keys;
     std::vector<float> vals;

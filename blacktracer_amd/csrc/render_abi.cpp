@@ -211,7 +211,8 @@ static int scene_upload(Context& c, bt_scene* s, const int32_t* tree, int tree_l
     void* dsky;
     int rc;
     if ((rc = c.buffer("scene_sky_upload", (size_t)3 * rows * cols, &dsky))) return rc;
-    if ((rc = c.copy({{dsky, sky, (size_t)3 * rows * cols}}, true))) return rc;
+    const CopySeg seg{dsky, sky, (size_t)3 * rows * cols};
+    if ((rc = c.copy(&seg, 1, true))) return rc;
     if ((rc = render_sum_table(&c, (const uint8_t*)dsky, rows, cols, s->table))) return rc;
     BT_HIP(hipStreamSynchronize(c.stream));
     return BT_OK;
@@ -744,11 +745,12 @@ int bt_make_image(bt_context* h, const float* stars, const int32_t* star_tree_in
         scene_release(&scene);
         return rc;
     }
-    if ((rc = c.copy({{dht, hash_tables, sizeof(float) * 2 * (size_t)hw * hw},
-                      {dot, offset_tables, sizeof(int32_t) * 2 * (size_t)ow * ow},
-                      {dtag, hash_pos_tag, sizeof(int32_t) * 2 * (size_t)hw * hw},
-                      {dview, viewthing, sizeof(float) * 2 * NC}},
-                     true))) {
+    const CopySeg in[] = {{dht, hash_tables, sizeof(float) * 2 * (size_t)hw * hw},
+                          {dot, offset_tables, sizeof(int32_t) * 2 * (size_t)ow * ow},
+                          {dtag, hash_pos_tag, sizeof(int32_t) * 2 * (size_t)hw * hw},
+                          {dview, viewthing, sizeof(float) * 2 * NC}};
+    const CopySeg out{out_bgra, dout, 4 * NP};
+    if ((rc = c.copy(in, 4, true))) {
         (void)hipStreamSynchronize(c.stream);
         scene_release(&scene);
         return rc;
@@ -765,7 +767,7 @@ int bt_make_image(bt_context* h, const float* stars, const int32_t* star_tree_in
                           cam_param, f, step, (uint8_t*)dout, nullptr);
         if (rc) goto done;
     }
-    rc = c.copy({{out_bgra, dout, 4 * NP}}, false);
+    rc = c.copy(&out, 1, false);
 done:
     (void)hipStreamSynchronize(c.stream);
     scene_release(&scene);

@@ -17,6 +17,7 @@ std::map<const char*, size_t> pinned;         // allocations the runtime knows
 std::deque<std::function<void()>> work;       // the stream's copies, not yet carried out
 size_t done = 0;                              // copies carried out so far
 std::map<void*, size_t> events;               // copies that an event waits for
+bool no_pinned = false;
 
 bool is_known(const void* p) {
     for (auto& a : pinned)
@@ -65,6 +66,7 @@ hipError_t hipStreamSynchronize(hipStream_t) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (no_pinned) return hipErrorOutOfMemory;
     std::lock_guard<std::recursive_mutex> lk(mu);
     *p = std::malloc(n);
     pinned[(const char*)*p] = n;
@@ -96,8 +98,9 @@ int main() {
     const size_t mib = size_t(1) << 20;
     const size_t sets[][3] = {{1, 0, 0}, {4 * mib - 1, 0, 0}, {4 * mib, 0, 0}, {2 * mib, 2 * mib + 1, 0},
                               {4 * mib + 1, 7, 2 * mib - 1}, {0, 9 * mib + 5, 3}, {30 * mib + 11, 1, 14 * mib}};
-    for (int mode = 0; mode < 2; mode++) {   // pageable, the caller's memory pinned
+    for (int mode = 0; mode < 3; mode++) {   // pageable, no pinned memory to have, the caller's memory pinned
         bt::Context c;
+        no_pinned = mode == 1;
         for (const auto& set : sets)
             for (int to_device = 0; to_device < 2; to_device++) {
                 bt::CopySeg segs[3];
@@ -106,10 +109,10 @@ int main() {
                     src[s] = (unsigned char*)std::malloc(set[s] + 1);
                     dst[s] = (unsigned char*)std::calloc(set[s] + 1, 1);
                     for (size_t k = 0; k < set[s]; k++) src[s][k] = (unsigned char)(1 + (k * 2654435761u >> 13) % 255);
-                    if (mode == 1) pinned[(const char*)(to_device ? src[s] : dst[s])] = set[s] + 1;
+                    if (mode == 2) pinned[(const char*)(to_device ? src[s] : dst[s])] = set[s] + 1;
                     segs[s] = {dst[s], src[s], set[s]};
                 }
-                const int rc = c.copy(std::vector<bt::CopySeg>(segs, segs + 3), to_device != 0);
+                const int rc = c.copy(segs, 3, to_device != 0);
                 bool ok = rc == 0;
                 for (int s = 0; s < 3 && ok; s++) {
                     // the caller's memory is its own again; what it gave is on the stream, or there

@@ -1,6 +1,6 @@
 """Context::copy on the host, over a stand-in for the runtime (copy_host.cpp):
-sizes around the pieces and the rule's limit, and from and to memory that the
-caller has pinned itself."""
+sizes around the pieces and the rule's limit, without pinned memory to have,
+and from and to memory that the caller has pinned itself."""
 import os
 import subprocess
 
