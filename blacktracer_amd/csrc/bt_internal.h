@@ -175,6 +175,7 @@ struct Context {
     int device = 0;
     Tune tune;
     int64_t launch_lanes = 0;   // widest persistent launch since last reset (lanes)
+    uint64_t launch_shapes = 0;   // hash of the persistent launches' shapes since last reset
     int num_cus = 256;
     hipStream_t stream = nullptr;
     hipStream_t aux = nullptr;                 // overlapping work, joined before a call returns

@@ -620,13 +620,14 @@ struct LanePose {
 // others' freed lanes took a second ray, at the end of which the launch ends):
 // 500 rays took 1070 us, with small workgroups 938, with both 720.
 // Not `spread`: the FP32 bulk keeps its workgroups (of 8 rays it took 108 us in
-// one of one wave, 99 to 105 in one of four).
+// one of one wave, 99 to 105 in one of four).  tuned_chunk: reserve as tuned
+// also where the lanes fit (trace_mixed_src).
 struct Launch {
     unsigned blocks, threads, chunk;
 };
 
 template <class K>
-int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L, bool spread = true) {
+int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L, bool spread = true, bool tuned_chunk = false) {
     int threads = (int)c->tune.block;
     if (threads != 64 && threads != 128 && threads != 256)
         return fail(BT_ERR_INVALID, "tune: block size must be 64, 128 or 256");
@@ -645,8 +646,9 @@ int persistent_launch(Context* c, K kernel, int64_t n_max, Launch* L, bool sprea
     if (blocks < 1) blocks = 1;
     L->blocks = (unsigned)blocks;
     L->threads = (unsigned)threads;
-    L->chunk = n_max <= blocks * threads ? 64u : c->tune.chunk;
+    L->chunk = n_max <= blocks * threads && !tuned_chunk ? 64u : c->tune.chunk;
     if (blocks * threads > c->launch_lanes) c->launch_lanes = blocks * threads;
+    for (unsigned v : {L->blocks, L->threads, L->chunk}) c->launch_shapes = (c->launch_shapes ^ v) * 0x100000001b3ull;
     return BT_OK;
 }
 

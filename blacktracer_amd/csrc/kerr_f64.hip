@@ -341,8 +341,7 @@ int trace_f64_queue(Context* c, const Src& S, const ParamsK& prm, int64_t n_max,
         if (int rc = persistent_launch(c, rk_f64<kWarm, Src>, n_max, &L)) return rc;
         rk_f64<kWarm, Src><<<L.blocks, L.threads, 0, stream>>>(S, prm, Q, d_stats, L.chunk, *cont, prio);
     } else {
-        if (int rc = persistent_launch(c, rk_f64<kExact, Src>, n_max, &L)) return rc;
-        if (tuned_chunk) L.chunk = c->tune.chunk;
+        if (int rc = persistent_launch(c, rk_f64<kExact, Src>, n_max, &L, true, tuned_chunk)) return rc;
         rk_f64<kExact, Src><<<L.blocks, L.threads, 0, stream>>>(S, prm, Q, d_stats, L.chunk, ContK{},
                                                                 prio);
     }

@@ -462,11 +462,10 @@ int trace_mixed_src(Context* c, const Src& S, const ParamsK& prm, int64_t n, Sta
     {
         KTimer t(c, "rk_mixed");
         Launch L;
-        if ((rc = persistent_launch(c, rk_mixed<Src>, n, &L, false))) {
+        if ((rc = persistent_launch(c, rk_mixed<Src>, n, &L, false, tuned))) {
             (void)join();
             return rc;
         }
-        if (tuned) L.chunk = c->tune.chunk;
         rk_mixed<Src><<<L.blocks, L.threads, 0, c->stream>>>(S, prm, Qw, head32, Qr, cont, d_stats, restart_at,
                                                              L.chunk);
         if (hipGetLastError() != hipSuccess) {

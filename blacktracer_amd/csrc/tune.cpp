@@ -8,7 +8,9 @@
 // i pi / (N - 1), phi = j 2 pi / M, M = 2 (N - 1)) at about n_rays points,
 // traced with the caller's integrator settings -- for candidate shapes by
 // coordinate descent (chunk, then block, then waves), keeps the fastest in
-// the context and reports it.  The best shape depends on the batch size
+// the context and reports it.  A knob that changes no launch at this size
+// (small batches take workgroups and reservations of their own,
+// persistent_launch) keeps the value it had.  The best shape depends on the batch size
 // (small batches are bound by their slowest rays, large ones by
 // throughput), so callers calibrate at the size they trace.  Results do not
 // depend on the launch shape: every ray's arithmetic is the same whichever
@@ -95,12 +97,19 @@ int bt_autotune(bt_context* h, const bt_pose* pose, const bt_integ_params* prm, 
         return fail(BT_ERR_HIP, "bt_autotune: event creation failed");
     }
     const Tune saved = c.tune;
-    // best of three runs (the first also warms caches and clocks)
-    auto time_of = [&](const Tune& t, float* ms_out, int64_t* lanes) -> int {
+    struct Timed {
+        float ms = 0;
+        int64_t lanes = 0;
+        uint64_t shapes = 0;
+    };
+    // best of three runs (the first also warms caches and clocks); only the
+    // first where its launches are those of `known`
+    auto time_of = [&](const Tune& t, const Timed* known, Timed* out) -> int {
         c.tune = t;
-        c.launch_lanes = 0;
         float best = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
+            c.launch_lanes = 0;
+            c.launch_shapes = 0;
             BT_HIP(hipMemcpyAsync(d_th, d_in, sizeof(double) * n, hipMemcpyDeviceToDevice, c.stream));
             BT_HIP(hipMemcpyAsync(d_ph, (double*)d_in + n, sizeof(double) * n, hipMemcpyDeviceToDevice, c.stream));
             BT_HIP(hipEventRecord(e0, c.stream));
@@ -111,22 +120,22 @@ int bt_autotune(bt_context* h, const bt_pose* pose, const bt_integ_params* prm, 
             BT_HIP(hipEventSynchronize(e1));
             float ms = 0;
             BT_HIP(hipEventElapsedTime(&ms, e0, e1));
+            if (known && c.launch_shapes == known->shapes) break;
             if (rep > 0 && ms < best) best = ms;
         }
-        *ms_out = best;
-        *lanes = c.launch_lanes;
+        *out = Timed{best, c.launch_lanes, c.launch_shapes};
         return BT_OK;
     };
     Tune best = saved;
     best.chunk = 128;
     best.block = 256;
     best.waves = 0;
-    float best_t = 0;
-    int64_t best_lanes = 0;
-    rc = time_of(best, &best_t, &best_lanes);
+    Timed best_t;
+    rc = time_of(best, nullptr, &best_t);
     const unsigned chunks[] = {64, 128, 256, 512, 1024};
     const unsigned blocks[] = {64, 128, 256};
     const int waves[] = {0, 1, 2, 3, 4};
+    bool told[3] = {};   // some value of the knob changes the launches
     for (int pass = 0; pass < 3 && !rc; pass++) {
         const int count = pass == 0 ? 5 : pass == 1 ? 3 : 5;
         for (int k = 0; k < count && !rc; k++) {
@@ -135,15 +144,24 @@ int bt_autotune(bt_context* h, const bt_pose* pose, const bt_integ_params* prm, 
             if (pass == 1) t.block = blocks[k];
             if (pass == 2) t.waves = waves[k];
             if (t.chunk == best.chunk && t.block == best.block && t.waves == best.waves) continue;
-            float ms = 0;
-            int64_t lanes = 0;
-            rc = time_of(t, &ms, &lanes);
-            if (!rc && ms < best_t) {
+            Timed u;
+            rc = time_of(t, &best_t, &u);
+            if (rc || u.shapes == best_t.shapes) continue;
+            told[pass] = true;
+            if (u.ms < best_t.ms) {
                 best = t;
-                best_t = ms;
-                best_lanes = lanes;
+                best_t = u;
             }
         }
+    }
+    if (!rc) {
+        Tune t = best;
+        if (!told[0]) t.chunk = saved.chunk;
+        if (!told[1]) t.block = saved.block;
+        if (!told[2]) t.waves = saved.waves;
+        Timed u;
+        rc = time_of(t, &best_t, &u);
+        if (u.shapes == best_t.shapes) best = t;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -157,9 +175,9 @@ int bt_autotune(bt_context* h, const bt_pose* pose, const bt_integ_params* prm, 
         out->block = (int)best.block;
         out->waves = best.waves;
         // rays per lane of the widest persistent launch at this shape
-        out->rays_per_lane = best_lanes > 0 ? (double)n / (double)best_lanes : 0.0;
+        out->rays_per_lane = best_t.lanes > 0 ? (double)n / (double)best_t.lanes : 0.0;
     }
-    if (best_ms) *best_ms = best_t;
+    if (best_ms) *best_ms = best_t.ms;
     return BT_OK;
 }
 

@@ -158,7 +158,10 @@ int bt_selfcheck_division(bt_context* ctx, int64_t n, uint64_t seed, int64_t* mi
 
 /* ---- launch-shape tuning of the persistent integrators (no reference
  * counterpart: the reference launches one thread per ray with a fixed block,
- * integration_wrapper Grid.h:514-556) ---- */
+ * integration_wrapper Grid.h:514-556).  The shape of launches that fill the
+ * GPU.  Smaller ones may take smaller workgroups (fewer rays than four waves
+ * per compute unit) and smaller reservations (all rays fit the resident lanes)
+ * than these. ---- */
 typedef struct {
     int chunk;             /* queue positions a wave reserves per atomic (>= 64) */
     int block;             /* threads per workgroup: 64, 128 or 256 */
@@ -173,7 +176,8 @@ int bt_tune_set(bt_context* ctx, const bt_tune* t);
 /* Times about n_rays (<= 0: 2^20; at most 2^24) directions of the pose's
  * equal-angle camera sky (the lattice grid builds trace) under prm for
  * candidate shapes (coordinate descent over chunk {64..1024}, block
- * {64,128,256}, waves {0..4}) and keeps the fastest in the context; out and
+ * {64,128,256}, waves {0..4}) and keeps the fastest in the context (of a
+ * knob that changes no launch at this size, the value set before); out and
  * best_ms (nullable) receive it and its time.  The best shape depends on
  * the batch size: calibrate at the size that will be traced. */
 int bt_autotune(bt_context* ctx, const bt_pose* pose, const bt_integ_params* prm, int64_t n_rays,

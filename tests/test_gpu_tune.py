@@ -80,3 +80,46 @@ def test_autotune_keeps_a_valid_fastest_shape():
             assert np.array_equal(a, b)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("precision", [bt.BT_PREC_FP64, bt.BT_PREC_MIXED])
+def test_autotune_keeps_what_it_cannot_tell(precision):
+    """A batch of less than a wave per SIMD launches alike under every chunk
+    (and on the FP64 path under every block and waves): those stay as set."""
+    ctx = bt.Context(0)
+    try:
+        cam = bt.Camera(math.pi / 2, 0.0, 5.0, black_hole=bt.BlackHole(0.999))
+        ctx.set_tune(768, 64, 3)
+        res = ctx.autotune(cam, params=bt.IntegParams(precision), n_rays=1 << 14)
+        print(f"autotune {res}", flush=True)
+        assert res["chunk"] == 768 and res["ms"] > 0
+        if precision == bt.BT_PREC_FP64:
+            assert ctx.tune() == {"chunk": 768, "block": 64, "waves": 3}
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("precision", [bt.BT_PREC_FP64, bt.BT_PREC_MIXED])
+def test_results_independent_of_launch_shape_when_lanes_refill(precision):
+    """More rays than resident lanes under every shape, so that lanes take
+    further rays from reservations of every size, and workgroups of every
+    size run."""
+    ctx = bt.Context(0)
+    try:
+        cam = bt.Camera(1.2, 0.0, 6.0, black_hole=bt.BlackHole(0.9))
+        th, ph = _rays(700001, 9)
+        prm = bt.IntegParams(precision)
+        ref = None
+        for shape in SHAPES:
+            print(f"precision={precision} shape={shape}", flush=True)
+            ctx.set_tune(*shape)
+            out = bt.trace_rays(cam, th, ph, params=prm, ctx=ctx)
+            ref = ref or out
+            assert all(np.array_equal(a, b) for a, b in zip(out, ref))
+        before = ref
+        res = ctx.autotune(cam, params=prm, n_rays=700001)
+        print(f"autotune {res}", flush=True)
+        after = bt.trace_rays(cam, th, ph, params=prm, ctx=ctx)
+        assert all(np.array_equal(a, b) for a, b in zip(after, before))
+    finally:
+        ctx.close()
