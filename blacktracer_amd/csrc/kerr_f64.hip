@@ -276,6 +276,12 @@ __global__ void selfcheck_div(int64_t n, unsigned long long seed, unsigned long 
         const double f = operand(h3, h1), df = d * f;
         const SharedDiv by2(df, by.y * rcp_once(f));
         miss = miss || __double_as_longlong(by2.any(x)) != __double_as_longlong(x / df);
+        // ... and another product's from that one's
+        const double g = operand(mix64(h2 + 4), h2), dfg = df * g;
+        const SharedDiv by3(dfg, by2.y * rcp_once(g));
+        miss = miss || __double_as_longlong(by3.any(x)) != __double_as_longlong(x / dfg);
+        const SharedDiv sqr(d * d, by.y * by.y);
+        miss = miss || __double_as_longlong(sqr.any(x)) != __double_as_longlong(x / (d * d));
     }
     const unsigned long long m = __ballot(miss);
     if (lane_id() == 0 && m) atomicAdd(bad, (unsigned long long)__popcll(m));

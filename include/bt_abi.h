@@ -149,8 +149,9 @@ int bt_trace_rays_device_noalloc(bt_context* ctx, const bt_pose* pose, const bt_
 
 /* Self-check (no reference counterpart): the FP64 integrator divides by a
  * shared reciprocal where several quotients have one denominator (the
- * division sequence's own steps, the reciprocal refined once).  This runs
- * that form against the device's IEEE division on n generated operand pairs
+ * division sequence's own steps, the reciprocal refined once), and takes a
+ * product's reciprocal from its factors'.  This runs those forms (one factor,
+ * a square, products of two and of three) against the device's IEEE division on n generated operand pairs
  * (exponents within 2^+-200, with all-ones significands, zero numerators
  * and power-of-two denominators among them) and stores in *mismatches the
  * pairs whose quotients differ in any bit.  n at most 2^30. */

@@ -165,8 +165,9 @@ def test_trace_rays_radius_stop_variant(ctx):
 
 def test_shared_division_is_ieee_division():
     """The FP64 attempt's divisions through the shared-reciprocal form (the
-    right-hand side's sixteen quotients, five reciprocals among them, and
-    the error ratios) equal the device's IEEE division bit for bit, on 2^24
+    right-hand side's sixteen quotients over seven denominators, which are
+    products of three whose reciprocals the hardware estimates, and the error
+    ratios) equal the device's IEEE division bit for bit, on 2^24
     generated operand pairs with
     exponents within 2^+-200 (the right-hand side's values stay far inside:
     r below 1e8, sin^2 theta above 1e-40) and the hard classes among them:
