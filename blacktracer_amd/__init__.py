@@ -25,14 +25,49 @@ __all__ = ["Context", "BlackHole", "Camera", "Grid", "IntegParams", "trace_rays"
            "BT_PREC_FP64", "BT_PREC_MIXED", "default_context"]
 
 
-class Context:
+class _Native:
+    """A native object, freed by close() or with its Python object, but not
+    before those made from it (its context or scene is each one's parent):
+    Python finalises a set of objects that becomes garbage together, as at the
+    interpreter's exit, in any order."""
+
+    handle = _h = None
+    _live = 0           # objects made from this one and not freed yet
+    _parents = ()
+
+    def _open(self, handle, free, *parents):
+        self.handle = self._h = handle
+        self._free, self._parents = free, parents
+        for p in parents:
+            p._live += 1
+
+    def close(self):
+        self.handle = None
+        self._release()
+
+    def _release(self):
+        if self._h and self.handle is None and not self._live:
+            h, self._h = self._h, None
+            getattr(_lib.load(), self._free)(h)
+            for p in self._parents:
+                p._live -= 1
+                p._release()
+
+    def __del__(self):
+        try:
+            self.close()
+        except Exception:
+            pass
+
+
+class Context(_Native):
     """A bt_context: one HIP device, its stream, work buffers and timers."""
 
     def __init__(self, device=0):
         L = _lib.load()
         h = C.c_void_p()
         check(L.bt_context_create(device, C.byref(h)))
-        self.handle = h
+        self._open(h, "bt_context_destroy")
         self.device = device
 
     def sync(self):
@@ -76,17 +111,6 @@ class Context:
         """A device buffer owned by the caller (DeviceBuffer)."""
         return DeviceBuffer(self, nbytes)
 
-    def close(self):
-        if getattr(self, "handle", None):
-            _lib.load().bt_context_destroy(self.handle)
-            self.handle = None
-
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
-
 
 class DeviceBuffer:
     """Device memory from bt_device_alloc, freed with the object."""
@@ -97,6 +121,7 @@ class DeviceBuffer:
         p = C.c_void_p()
         check(_lib.load().bt_device_alloc(ctx.handle, self.nbytes, C.byref(p)))
         self.ptr = p
+        ctx._live += 1
 
     def to_host(self, out):
         check(_lib.load().bt_memcpy(self.ctx.handle, out.ctypes.data_as(C.c_void_p), self.ptr,
@@ -109,8 +134,10 @@ class DeviceBuffer:
 
     def close(self):
         if getattr(self, "ptr", None):
-            _lib.load().bt_device_free(self.ctx.handle, self.ptr)
+            _lib.load().bt_device_free(self.ctx._h, self.ptr)
             self.ptr = None
+            self.ctx._live -= 1
+            self.ctx._release()
 
     def __del__(self):
         try:
@@ -211,7 +238,7 @@ def trace_rays(camera, theta, phi, params=None, ctx=None, return_stats=False):
     return th, ph, st
 
 
-class Grid:
+class Grid(_Native):
     """Grid(maxLevel, startLevel, angle, camera, blackhole) (Grid.h:605-624),
     built and kept resident on the device.  ``cel``/``steps``/``levels``
     are dense host copies made on first access."""
@@ -233,7 +260,7 @@ class Grid:
 
     def _adopt(self, h):
         L = _lib.load()
-        self.handle = h
+        self._open(h, "bt_grid_free", self.ctx)
         vals = [C.c_int() for _ in range(5)]
         rays = C.c_int64()
         check(L.bt_grid_info(h, *[C.byref(v) for v in vals], C.byref(rays)))
@@ -320,17 +347,6 @@ class Grid:
                                    tag.ctypes.data_as(_lib.I32P)))
         return ht, ot, tag, hw.value, ow.value
 
-    def close(self):
-        if getattr(self, "handle", None):
-            _lib.load().bt_grid_free(self.handle)
-            self.handle = None
-
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
-
 
 # ---------------------------------------------------------------- render
 
@@ -375,7 +391,7 @@ def sky_add_low_stars(sky_bgr, stars4, magnitude_cut):
     return sky
 
 
-class Scene:
+class Scene(_Native):
     """Device-resident stars (star tree, StarProcessor.h) and summed-area sky
     table (MakeImageKernel.cu:1312-1331)."""
 
@@ -389,7 +405,7 @@ class Scene:
         check(_lib.load().bt_scene_create(self.ctx.handle, s4.ctypes.data_as(_lib.FP), s4.shape[0],
                                           tree_level, sky.ctypes.data_as(_lib.U8P), self.rows,
                                           self.cols, C.byref(h)))
-        self.handle = h
+        self._open(h, "bt_scene_free", self.ctx)
 
     def table(self):
         t = np.zeros((self.rows, self.cols, 4), dtype=np.float32)
@@ -411,22 +427,11 @@ class Scene:
                                                pos.ctypes.data_as(_lib.FP), mag.ctypes.data_as(_lib.FP),
                                                pos.size // 2, sky.ctypes.data_as(_lib.U8P), self.rows,
                                                self.cols, C.byref(h)))
-        self.handle = h
+        self._open(h, "bt_scene_free", self.ctx)
         return self
 
-    def close(self):
-        if getattr(self, "handle", None):
-            _lib.load().bt_scene_free(self.handle)
-            self.handle = None
 
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
-
-
-class View:
+class View(_Native):
     """Device-resident Viewer matrix of one resolution."""
 
     def __init__(self, width, height, view_angle=np.pi / 2, off_up=0.0, off_right=0.25 * np.pi / 4,
@@ -436,18 +441,7 @@ class View:
         h = C.c_void_p()
         check(_lib.load().bt_view_create(self.ctx.handle, view_angle, off_up, off_right, width,
                                          height, 1 if sphere else 0, C.byref(h)))
-        self.handle = h
-
-    def close(self):
-        if getattr(self, "handle", None):
-            _lib.load().bt_view_free(self.handle)
-            self.handle = None
-
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
+        self._open(h, "bt_view_free", self.ctx)
 
 
 def frame_bytes(width, height, step=1):
@@ -531,7 +525,7 @@ def render_frame_blend(grid0, grid1, alpha, scene, view, flags=None, cam14=None,
     return out
 
 
-class Trails:
+class Trails(_Native):
     """State of a frame sequence with star trails (and diffraction when a
     sprite of (width // 16, width // 16, 3) uint8 is given): each
     render() is the next frame (MakeImageKernel.cu:98-174,775-800)."""
@@ -549,7 +543,7 @@ class Trails:
             sp = self._sprite.ctypes.data_as(_lib.U8P)
         h = C.c_void_p()
         check(_lib.load().bt_trails_create(self.ctx.handle, scene.handle, width, height, sp, C.byref(h)))
-        self.handle = h
+        self._open(h, "bt_trails_free", self.ctx)
 
     def render(self, grid, scene, view, flags=None, cam7=None, step=1, stages=False, out_buffer=None):
         """The next frame (BGRA uint8, (h, w, 4)); with stages also the summed
@@ -582,17 +576,6 @@ class Trails:
         f, d = C.c_int64(), C.c_int64()
         check(_lib.load().bt_trails_stats(self.handle, C.byref(f), C.byref(d)))
         return dict(frames=f.value, dropped=d.value)
-
-    def close(self):
-        if getattr(self, "handle", None):
-            _lib.load().bt_trails_free(self.handle)
-            self.handle = None
-
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
 
 
 def make_image(stars, star_tree_arr, cam_param, magnitude, tree_level, M, N, step, sky_bgr,
@@ -681,7 +664,7 @@ def read_grid_file(path):
 # ---------------------------------------------------------------- serving
 
 
-class Server:
+class Server(_Native):
     """Continuous-batching render server (bt_server_*): requests of mixed
     resolution and pose, grids cached in HBM, admission by HBM footprint.
 
@@ -704,8 +687,8 @@ class Server:
         cfg.step = step
         h = C.c_void_p()
         check(L.bt_server_create(self.ctx.handle, scene.handle, C.byref(cfg), C.byref(h)))
-        self.handle = h
-        self.scene = scene          # must outlive the server
+        self._open(h, "bt_server_destroy", self.ctx, scene)
+        self.scene = scene
         self._outs = {}
 
     def submit(self, a, r, theta, offset, out, tag, star=True, map=True, lr=True):
@@ -735,14 +718,3 @@ class Server:
         st = _lib.BtServerStats()
         check(_lib.load().bt_server_stats_get(self.handle, C.byref(st)))
         return {n: getattr(st, n) for n, _ in _lib.BtServerStats._fields_}
-
-    def close(self):
-        if getattr(self, "handle", None):
-            _lib.load().bt_server_destroy(self.handle)
-            self.handle = None
-
-    def __del__(self):
-        try:
-            self.close()
-        except Exception:
-            pass
