@@ -1012,10 +1012,10 @@ int grid_build(Context* c, bt_grid* g, const bt_grid_params* gp) {
     return BT_OK;
 }
 
-// The same build for several grids at once.  The grids advance level by
-// level in lockstep; at each step the rays every grid needs (poles, start
-// lattice, then each refinement level) go into one multi-pose batch, traced
-// by one set of persistent launches with a shared work queue.  Refinement,
+// The same build for several grids at once.  The lattices traced ahead of
+// every grid (grid_ahead) go into one multi-pose batch, traced by one set of
+// persistent launches with a shared work queue; from there the grids advance
+// level by level in lockstep, each level's rays in one batch.  Refinement,
 // final levels and T-vertex repair stay per grid (they are cheap and
 // per-grid ordered).  All grids share the integration parameters of gs[0].
 int grid_build_batch(Context* c, const std::vector<bt_grid*>& gs, const bt_grid_params* gp,

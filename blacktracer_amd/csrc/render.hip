@@ -1,20 +1,24 @@
 // render.hip -- the per-pixel render pass (Path B): the drop-in for the
 // G == 1 frame of cudaPrep (MakeImageKernel.cu:1402-1529).
 //
-// Stages (one kernel each, all on the context stream):
+// Stages, on the context stream but for what runs beside the star pass:
 //   pix_interp   per pixel corner: quadtree descent of the dense grid and
 //                bicubic Hermite interpolation of the celestial angle
 //                (pixInterpolation, interpolatePix, kernel.cuh:736-968)
 //   bh_area      shadow flag and celestial solid angle per pixel
 //                (findBlackPixels + findArea)
 //   smooth_h/v   box-filtered solid angle (smoothAreaH/V)
-//   star_map     per pixel: star-tree search, point-in-quad, sub-pixel
-//                position, blackbody colour and the 3x3 Gaussian taps
-//                (distortStarMap); taps are stored tap-major so the gather
-//                of star_sum reads coalesced rows
+//   star pass    per pixel: candidate stars, point-in-quad, sub-pixel
+//                position, blackbody colour and the Gaussian taps
+//                (distortStarMap), a pixel's taps side by side: star_scan and
+//                star_wide sort the pixels by their work, star_assign and
+//                star_heads prepare the chunks of those with many candidates,
+//                star_map_chunk and star_chunk_reduce trace them, star_few
+//                and star_map_odd the others with a star inside
 //   star_sum     gather of the neighbours' taps + makePix
 //   env_map      summed-area sky sampling, lensing and redshift
-//                (distortEnvironmentMap)
+//                (distortEnvironmentMap); env_map_group and env_map_heavy
+//                for footprints of many sky columns
 //   composite    addStarsAndBackground
 // Pixel (i, j) is processed by thread x = j, y = i so that a wavefront
 // (16 x 4 pixels of a 16 x 16 block) reads consecutive row addresses.
@@ -938,9 +942,11 @@ __device__ __forceinline__ float exp10_f32(float x) {
 }
 
 // Whether every tap of every star takes the fast form in this pixel: the
-// tap weight x = frac * gaussian(d) lies in (0, 3.4e38] for frac in
-// [1e-30, 1e30] (gaussian(d) in [9e-4, 1] over the footprint), and
-// E = 10^(-0.4 (m + red)) stays finite for m >= -10, |red| <= 80.
+// tap weight x = frac * gaussian(d) lies in [0, 3.4e38] for frac in
+// [1e-30, 1e30] (over the footprints of steps 1, 2 and 3 gaussian(d) falls
+// from 1 to 8.8e-4, 3.3e-9 and 2.4e-17; an x that underflows to zero is no
+// light in either form), and E = 10^(-0.4 (m + red)) stays finite for
+// m >= -10, |red| <= 80.
 __device__ __forceinline__ bool star_pixel_odd(const StarPix& P, const SceneK& s) {
     return !(s.mag_tame && P.frac >= 1e-30f && P.frac <= 1e30f && P.red >= -80.f && P.red <= 80.f);
 }
@@ -1031,7 +1037,10 @@ __device__ __forceinline__ void star_accumulate(const StarPix& P, const float* p
 // per chunk; their chunk indices are taken by an atomic in star_assign
 // (contiguous per pixel).  A pixel's chunk partials are summed in
 // chunk order, so the result does not depend on which waves ran which
-// chunks.  Every queued star is then
+// chunks.  (Where a frame has more chunks than pixels, one lane adds up the
+// pixels whose chunks found no room, candidate by candidate; which those are
+// depends on the order of the atomics, and with it the last bits of their
+// sums.)  Every queued star is then
 // one of a few candidates of one lane, whatever the pixel it lands in: the
 // long per-star chain (bisection, taps) of a pixel with tens of thousands of
 // candidates is spread over many waves instead of serialised on a few lanes.
@@ -1124,7 +1133,9 @@ __device__ __forceinline__ void store_taps(float* taps, size_t ij,
 constexpr int kScanRows = 4;
 // Tiles of 16 x 16 pixels side by side per workgroup of star_scan, at most.
 // One in small frames (at 320 x 180 four leave three quarters of the SIMDs
-// without a wave: 37 us against 16), kScanTiles from a million pixels on.
+// without a wave: 37 us against 16), kScanTiles from a million pixels on
+// (whole frames of three grids with one and with four, us: 1920x1080 588, 836,
+// 640 and 591, 842, 638).
 constexpr int kScanTiles = 4;
 
 // Sorts the pixels by how much star work they hold: none (most of a frame),
@@ -1617,14 +1628,13 @@ __device__ __forceinline__ unsigned wave_scan(unsigned v) {
 
 // One wavefront per chunk (grid-stride): lane l takes the chunk's
 // candidates l, l + 64, ...; the taps are reduced over the wave in a fixed
-// order into the chunk's partial, summed per pixel by star_chunk_reduce.  For a binned pixel
-// the wave walks the footprint's bin rows 64 at a time: each lane loads one
-// row's range, a wave scan gives the rows' first candidate numbers (kept in
-// LDS), and each lane finds the row of each of its candidates.
+// order into the chunk's partial, summed per pixel by star_chunk_reduce.
+// The wave walks the candidate ranges its head names (bin rows, or stored
+// tree ranges) 64 at a time: each lane loads one range, a wave scan gives the
+// ranges' first candidate numbers (kept in LDS), and each lane finds the
+// range of each of its candidates.
 template <int STEP, bool ODD>
-__global__ __launch_bounds__(256) void star_map_chunk(const float* thphi, const uint8_t* bh, SceneK s, Cam7 cam,
-                                                      int W, int H, float offset, int lr, const float* area,
-                                                      const float* view, float* taps, StarQueue Q) {
+__global__ __launch_bounds__(256) void star_map_chunk(SceneK s, Cam7 cam, float* taps, StarQueue Q) {
     constexpr int FW = 2 * STEP + 1;
     constexpr int NT = FW * FW * 3;
     const unsigned lane = threadIdx.x & 63;
@@ -1820,7 +1830,6 @@ __global__ __launch_bounds__(256) void star_chunk_reduce(float* taps, StarQueue 
     }
 }
 
-// sumStarLight (MakeImageKernel.cu:753-773, bounds-checked) + makePix (:802-835)
 // Column j of a frame that wraps around, for j in [-W, 2 W) at least.
 __device__ __forceinline__ int wrap_frame(int j, int W) {
     while (j < 0) j += W;
@@ -1855,6 +1864,7 @@ __device__ __forceinline__ void make_pix(float br, float bg, float bb, uint8_t* 
 
 // sumStarLight (MakeImageKernel.cu:753-773) + makePix; trail (or null): the
 // frame's star trails, added after the taps (factor 1).
+// sumStarLight (MakeImageKernel.cu:753-773, bounds-checked) + makePix (:802-835)
 template <int STEP>
 __global__ __launch_bounds__(256) void star_sum(const float* taps, const uint8_t* lit, int W, int H, uint8_t* img,
                                                 float* o_star, const float* trail) {
@@ -3022,8 +3032,6 @@ __global__ void grid_to_f32(const double* cel, int GN, int GM, int sym, int GN1,
     }
 }
 
-// The pixels that one lane each traces: those of few candidates, then the
-// odd ones among them.
 GridV grid_view(const GridF& g) {
     return GridV{g.grid, g.GN, g.GM, (g.GM & (g.GM - 1)) == 0 ? 1.f / (float)g.GM : 0.f};
 }
@@ -3034,6 +3042,8 @@ int few_span(size_t NP) {
     return span;
 }
 
+// The pixels that one lane each traces: those of few candidates, then the
+// odd ones among them.
 template <int STEP>
 void star_rest(Context* c, hipStream_t st, const float* thphi, const uint8_t* bh, const SceneK& s,
                const Cam7& cam, int W, int H, const bt_render_flags& f, const float* area, const float* view,
@@ -3207,7 +3217,7 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         nq = ctr + kStarCtrWords;
     }
     // distortEnvironmentMap: pixels with few sky columns inline, those with
-    // more eight lanes each; then the wide ones, one wave each
+    // more sixteen lanes each; then the wide ones, one wave each
     auto sky_light = [&](hipStream_t es) {
         KTimer t(c, "env_map", es);
         env_map<<<grid2d(W, H), blk, 0, es>>>(thphi, bh, sky, cam, W, H, f.offset, f.lr, area, v.view, img_map, qgroup,
@@ -3266,8 +3276,11 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         // The odd pixels' chunks and the one-lane pixels (few, long chains) run
         // beside the chunks, on the auxiliary stream once the sky pass is
         // through; from four million pixels on, where the sky pass is the
-        // longer one, the one-lane pixels stay on the main stream (3840x2160:
-        // 1322 against 1401 us; 1920x1080 the other way round, 883 against 855).
+        // longer one, the one-lane pixels stay on the main stream (frames of
+        // three grids, us, on the main stream and on the auxiliary one:
+        // 3840x2160 1151, 1716, 1311 and 1216, 1671, 1371, 2880x1620 831, 1238,
+        // 965 and 831, 1194, 1050, 2560x1440 786, 1201, 892 and 777, 1169, 962,
+        // 1920x1080 587, 860, 647 and 591, 842, 638).
         // Trails fill the auxiliary stream: the odd chunks stay on the main one
         // too then.
         const bool few_on_main = !overlap || tf || NP >= (size_t(1) << 22);
@@ -3319,12 +3332,10 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
         }                                                                                                   \
         {                                                                                                   \
             KTimer t2(c, "star_chunk");                                                                     \
-            star_map_chunk<S, false><<<nwave, 256, 0, c->stream>>>(thphi, bh, s, cam, W, H, f.offset, f.lr, \
-                                                                   area, v.view, taps, Q);                  \
+            star_map_chunk<S, false><<<nwave, 256, 0, c->stream>>>(s, cam, taps, Q);                        \
         }                                                                                                   \
         if (tf) trail_images(rs);                                                                           \
-        star_map_chunk<S, true><<<nred, 256, 0, tf ? c->stream : rs>>>(thphi, bh, s, cam, W, H, f.offset,   \
-                                                                       f.lr, area, v.view, taps, Q);        \
+        star_map_chunk<S, true><<<nred, 256, 0, tf ? c->stream : rs>>>(s, cam, taps, Q);                    \
         star_rest<S>(c, few_on_main ? c->stream : rs, thphi, bh, s, cam, W, H, f, area, v.view, taps, Q);   \
         if (overlap) {                                                                                      \
             BT_HIP(hipEventRecord(c->ev_back, rs));                                                         \

@@ -199,9 +199,9 @@ int  bt_grid_build(bt_context* ctx, const bt_pose* pose, const bt_integ_params* 
                    bt_grid** out);
 /* Several grids at once (no counterpart in the reference, which builds one
  * Grid at a time, Grid.h:605): n poses with their own max/start levels and
- * shared integration parameters.  The grids advance level by level in
- * lockstep and the rays of each level of every grid are traced together in
- * one set of persistent launches over a shared device work queue.  out
+ * shared integration parameters.  The rays of every grid are traced
+ * together, in sets of persistent launches over a shared device work queue:
+ * one for the first levels of all grids, then one for each level.  out
  * receives n grids (each freed with bt_grid_free); stats (nullable) the
  * batch's counters; bt_grid_stats of a batched grid holds only its ray
  * count.  1 <= n <= 128. */
