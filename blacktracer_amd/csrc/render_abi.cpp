@@ -464,6 +464,8 @@ struct bt_trails {
     bt::Context* ctx = nullptr;
     int S = 0, W = 0, H = 0, fs = 0;
     int64_t frame = 0;
+    bool begun = false;     // a star pass has run: both halves of the cache hold counts
+    bool counted = false;   // the last frame had one
     void* block = nullptr;
     uint8_t* sprite = nullptr;
     bt::TrailK k{};
@@ -544,7 +546,7 @@ int frame_impl(bt_context* h, const bt_grid* g, const bt_grid* g1, float alpha, 
     if (tr) {
         tf.k = tr->k;
         tf.k.cur = (int)(tr->frame % 2);
-        tf.first = tr->frame == 0;
+        tf.first = !tr->begun;
         tf.W = tr->W;
         tf.H = tr->H;
         tf.sprite = tr->sprite;
@@ -556,6 +558,8 @@ int frame_impl(bt_context* h, const bt_grid* g, const bt_grid* g1, float alpha, 
     if (tr) {
         // the reference's frame counter advances with every displayed frame
         tr->frame++;
+        tr->counted = f.star != 0;
+        tr->begun = tr->begun || f.star;
         if (trail_out && f.star)
             BT_HIP(hipMemcpyAsync(trail_out, tr->k.trail, sizeof(float) * 3 * NP, hipMemcpyDeviceToHost, c.stream));
         else if (trail_out)
@@ -663,7 +667,9 @@ int bt_trails_create(bt_context* h, const bt_scene* s, int width, int height, co
 }
 
 void bt_trails_reset(bt_trails* t) {
-    if (t) t->frame = 0;
+    if (!t) return;
+    t->frame = 0;
+    t->begun = t->counted = false;
 }
 
 int bt_trails_stats(bt_trails* t, int64_t* frames, int64_t* dropped) {
@@ -674,7 +680,7 @@ int bt_trails_stats(bt_trails* t, int64_t* frames, int64_t* dropped) {
     BT_HIP(hipMemcpyAsync(st, t->k.stats, sizeof(st), hipMemcpyDeviceToHost, t->ctx->stream));
     BT_HIP(hipStreamSynchronize(t->ctx->stream));
     if (frames) *frames = t->frame;
-    if (dropped) *dropped = t->frame > 0 ? st[1] : 0;
+    if (dropped) *dropped = t->counted ? st[1] : 0;
     return BT_OK;
 }
 

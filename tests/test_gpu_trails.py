@@ -78,6 +78,27 @@ def test_trail_sequence_matches_oracle(ctx, world, diffraction):
     OT.close()
 
 
+def test_frames_without_a_star_pass(ctx, world):
+    """A sequence that begins without the star pass has no images to draw
+    trails from when it starts, and drops none meanwhile."""
+    view = bt.View(W, H, ctx=ctx)
+    T = bt.Trails(world["scene"], W, H, ctx=ctx)
+    none, lit = bt.RenderFlags(star=False), bt.RenderFlags(offset=0.1)
+    plain = bt.render_frame(world["grid"], world["scene"], view, flags=lit)
+    for sequence in ((none, lit), (none, none, lit), (none, none, none, lit, lit, none)):
+        T.reset()
+        lit_before = False
+        for k, f in enumerate(sequence):
+            img, st = T.render(world["grid"], world["scene"], view, flags=f, stages=True)
+            assert T.stats() == dict(frames=k + 1, dropped=0)
+            if not lit_before:
+                assert st["trail"].max() == 0
+                if f is lit:
+                    assert np.array_equal(img, plain)
+            lit_before = lit_before or f is lit
+    T.close()
+
+
 def test_trails_reset_and_bad_state(ctx, world):
     view = bt.View(W, H, ctx=ctx)
     T = bt.Trails(world["scene"], W, H, ctx=ctx)
