@@ -76,12 +76,6 @@ __device__ F2 interpolate_linear(float percDown, float percRight, const F2* c) {
 // (count 0 -> 1) and never deeper; the two levels are written out here.
 __device__ __attribute__((noinline)) F2 interpolate_hermite_l1(GridV g, int i, int j, int gap, F2 c0, F2 c1, F2 c2, F2 c3);
 
-// x % GM of a column index x < 4 GM (a negative x stays, as with %).
-__device__ __forceinline__ int wrap_col(int x, int GM) {
-    while (x >= GM) x -= GM;
-    return x;
-}
-
 // kernel.cuh:817-889 for recursion depth `count`, for a point (i, j) that the
 // grid does not hold.  Out of line: most points are held, and the eight
 // copies of this in every interpolation were larger than the instruction

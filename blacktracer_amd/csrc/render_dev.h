@@ -31,6 +31,13 @@ __device__ __forceinline__ int cvt_i32(float x) {
     return r;
 }
 
+// x % GM (a negative remainder stays, as with %) of a column index, which is
+// seldom beyond [0, 2 GM): no division there.
+__device__ __forceinline__ int wrap_col(int x, int GM) {
+    if (x >= GM) x -= GM;
+    return x < GM && x > -GM ? x : x % GM;
+}
+
 // fmodf(x, 2 pi) without the general reduction where it is one exact
 // subtraction at most (the remainder of x in [2 pi, 4 pi) is x - 2 pi, which
 // is exact).

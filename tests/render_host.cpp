@@ -1,5 +1,6 @@
-// rdr::div_by (csrc/render_dev.h) against the division, for the gaussian's two
-// constants: every significand, at exponents across the range they meet.
+// Forms of csrc/render_dev.h that leave a division out, against the division:
+// div_by for the gaussian's two constants (every significand, at exponents
+// across the range they meet), wrap_col for small and extreme indices.
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -19,5 +20,11 @@ int main() {
                 if (bt::rdr::div_by(x, d, 1.f / d) != x / d || bt::rdr::div_by(-x, d, 1.f / d) != -x / d) bad++;
             }
     std::printf("%lld quotients differ\n", bad);
-    return bad != 0;
+    long long cols = 0;
+    for (int GM = 1; GM <= 260; GM++)
+        for (int x = -7 * GM - 3; x <= 7 * GM + 3; x++) cols += bt::rdr::wrap_col(x, GM) != x % GM;
+    for (int GM : {1, 2, 3, 4096, 65535, 0x7fffffff})
+        for (int x : {-0x7fffffff, -65536, -4096, 0, 4096, 0x7ffffffe, 0x7fffffff}) cols += bt::rdr::wrap_col(x, GM) != x % GM;
+    std::printf("%lld columns differ\n", cols);
+    return bad != 0 || cols != 0;
 }
