@@ -176,6 +176,8 @@ static void scene_release(bt_scene* s) {
 static int scene_upload(Context& c, bt_scene* s, const int32_t* tree, int tree_level, const float* pos,
                         const float* mag, int S, const uint8_t* sky, int rows, int cols) {
     if (rows <= 0 || cols <= 0 || !sky) return fail(BT_ERR_INVALID, "scene: sky image required");
+    if ((int64_t)rows * cols > INT32_MAX)   // the kernels index texels in 32 bits
+        return fail(BT_ERR_INVALID, "scene: the sky image has more than 2^31 - 1 pixels");
     const size_t tsz = (size_t)((1 << (tree_level + 1)) - 1);
     s->tree_level = tree_level;
     s->S = S;

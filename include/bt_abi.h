@@ -276,6 +276,7 @@ int bt_sky_add_low_stars(uint8_t* sky_bgr, int rows, int cols, const float* star
 typedef struct bt_scene bt_scene;   /* star tree + summed-area sky table */
 typedef struct bt_view bt_view;     /* pixel-corner directions of one resolution */
 
+/* A sky of at most 2^31 - 1 pixels (also for bt_make_image). */
 int  bt_scene_create(bt_context* ctx, const float* stars4, int star_count, int tree_level,
                      const uint8_t* sky_bgr, int sky_rows, int sky_cols, bt_scene** out);
 /* Same from a star tree already built (the arrays of a .star file,
