@@ -1940,6 +1940,7 @@ __global__ __launch_bounds__(256) void trail_clear(TrailK T, int frame0, size_t 
         T.count[(size_t)T.cur * T.S + q] = 0;
         if (frame0) T.count[(size_t)(1 - T.cur) * T.S + q] = 0;
     }
+    for (size_t h = t; h < (size_t)T.S * kTrailHits; h += stride) T.hit_pix[h] = kNoPixel;
     for (size_t p = t; p < n3; p += stride) T.trail[p] = 0.f;
     if (t == 0) T.stats[1] = 0;
 }
@@ -1973,20 +1974,22 @@ __global__ __launch_bounds__(256) void trail_grad(const float* thphi, int W, int
     grad[2 * ((size_t)i * M1 + j) + 1] = gy;
 }
 
-// One image: star q of the scene, the slot-th one of its images.
-__device__ __forceinline__ void trail_record(const TrailK& T, const StarPix& P, int q, unsigned slot, float2 mg,
-                                             uint32_t pix) {
-    if (slot >= (unsigned)kTrailHits) {
-        atomicAdd(&T.stats[1], 1u);
-        return;
+// One image: star q of the scene in pixel pix.  The first kTrailHits images of a
+// star that are found take a slot each.  From then on (few stars have so many)
+// an image goes round the slots, leaves the lesser pixel in each and takes the
+// other on: a star keeps its first images in pixel order, whatever the order
+// they are found in.  Slots only ever fall, so one read as less or equal is
+// passed over, and what has been all the way round is no less than any of them.
+__device__ __forceinline__ void trail_record(const TrailK& T, int q, uint32_t pix) {
+    const unsigned slot = atomicAdd(&T.nhits[q], 1u);
+    uint32_t* hp = T.hit_pix + (size_t)q * kTrailHits;
+    for (unsigned n = 0; n < (unsigned)kTrailHits; n++) {
+        const unsigned k = (slot + n) % kTrailHits;
+        if (slot + n >= (unsigned)kTrailHits && hp[k] <= pix) continue;
+        const uint32_t old = atomicMin(&hp[k], pix);
+        if (old == kNoPixel) return;
+        pix = max(old, pix);
     }
-    float temp = 46.f / P.redshft * ((1.f / ((0.92f * mg.y) + 1.7f)) + (1.f / ((0.92f * mg.y) + 0.62f))) - 10.f;
-    const int index = max(0, min(cvt_i32(floorf(temp)), 390));
-    const size_t h = (size_t)q * kTrailHits + slot;
-    T.hit_pix[h] = pix;
-    T.hit_data[3 * h] = mg.x + P.red;
-    T.hit_data[3 * h + 1] = P.frac;
-    T.hit_data[3 * h + 2] = (float)index;
 }
 
 // Largest star tree (level 10), held in LDS for the walks.
@@ -2012,28 +2015,22 @@ __device__ bool trail_pixel(const SceneK& s, const StarPix& P) {
 __device__ __forceinline__ void trail_range(const TrailK& T, const SceneK& s, const StarPix& P, uint32_t ij, int b,
                                             int e, int first, int step) {
     const float* pos = P.picheck ? s.star_pos : s.bin_pos;
-    const float* magv = P.picheck ? s.star_mag : s.bin_mag;
     for (int k = b + first; k < e; k += step) {
         float st, sp;
-        if (!star_test(P, pos, k, st, sp)) continue;
-        const int q = P.picheck ? k : s.bin_idx[k];
-        trail_record(T, P, q, atomicAdd(&T.nhits[q], 1u), reinterpret_cast<const float2*>(magv)[k], ij);
+        if (star_test(P, pos, k, st, sp)) trail_record(T, P.picheck ? k : s.bin_idx[k], ij);
     }
 }
 
 // The images of this frame: per pixel with starsToCheck < S/100
-// (MakeImageKernel.cu:273-282,301), every star inside its quad, with the
-// quantities addTrails uses (part, frac, blackbody index).  Runs after the
+// (MakeImageKernel.cu:273-282,301), every star inside its quad.  Runs after the
 // star pass has sorted the pixels: one that is kDark has no star inside.
 // trail_hits does the kFew pixels, gathered in LDS from a span of the frame so
-// that full waves walk the star tree (from LDS) and lens; trail_queued the
-// queued ones, whose lensing star_assign has stored, sixteen lanes to a
-// pixel's candidates.  Most pixels hold no star: a lane per pixel of the
+// that full waves walk the star tree (from LDS); trail_queued the queued ones,
+// sixteen lanes to a pixel's candidates.  Most pixels hold no star: a lane per pixel of the
 // frame, walking the tree for each, took 980 us at 1366 x 768 with 100000
 // stars.
 __global__ __launch_bounds__(256) void trail_hits(const float* thphi, SceneK s, Cam7 cam, int W, int H, float offset,
-                                                  int lr, const float* area, const float* view, TrailK T,
-                                                  const uint8_t* lit, int span) {
+                                                  TrailK T, const uint8_t* lit, int span) {
     __shared__ int32_t s_tree[kTreeWords];
     __shared__ uint16_t s_list[kFewSpan];
     __shared__ unsigned s_n;
@@ -2055,7 +2052,6 @@ __global__ __launch_bounds__(256) void trail_hits(const float* thphi, SceneK s, 
         StarPix P;
         star_pixel_geom(thphi, W, i, j, offset, cam, P);
         if (!trail_pixel(s, P)) continue;
-        star_lens(W, ij, i * (W + 1) + j, lr, area, view, cam, P);
         for_ranges(P, s, [&](int b, int e) { trail_range(T, s, P, (uint32_t)ij, b, e, 0, 1); });
     }
 }
@@ -2086,9 +2082,6 @@ __global__ __launch_bounds__(256) void trail_queued(const float* thphi, SceneK s
                 const unsigned k = e0 + (unsigned)__ffs((int)m) - 1;
                 const uint32_t ij = Q.pix[k];
                 star_pixel_geom(thphi, W, (int)(ij / (uint32_t)W), (int)(ij % (uint32_t)W), offset, cam, P);
-                P.frac = Q.lens[3 * k];
-                P.redshft = Q.lens[3 * k + 1];
-                P.red = Q.lens[3 * k + 2];
                 for_ranges(P, s, [&](int b, int e) { trail_range(T, s, P, ij, b, e, (int)(lane & 15), 16); });
             }
             for (int g = 0; g < 4; g++) todo &= todo - 1;
@@ -2096,30 +2089,21 @@ __global__ __launch_bounds__(256) void trail_queued(const float* thphi, SceneK s
     }
 }
 
-// Per star: its images in pixel order; the first kTrailNum become this
-// frame's cache (MakeImageKernel.cu:102-104).
+// Per star: its images in pixel order; the first kTrailNum become this frame's
+// cache (MakeImageKernel.cu:102-104), those beyond kTrailHits are counted.
 __global__ __launch_bounds__(256) void trail_cache(TrailK T, int W) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= T.S) return;
-    const int n = (int)min(T.nhits[q], (unsigned)kTrailHits);
-    if (n == 0) return;
+    const unsigned found = T.nhits[q];
+    if (found == 0) return;
+    if (found > (unsigned)kTrailHits) atomicAdd(&T.stats[1], found - (unsigned)kTrailHits);
+    const int n = (int)min(found, (unsigned)kTrailHits);
     uint32_t* hp = T.hit_pix + (size_t)q * kTrailHits;
-    float* hd = T.hit_data + (size_t)q * kTrailHits * 3;
-    for (int a = 1; a < n; a++) {   // insertion sort by pixel (a star has a few images)
+    for (int a = 1; a < n; a++) {   // insertion sort (a star has a few images)
         const uint32_t kp = hp[a];
-        const float d0 = hd[3 * a], d1 = hd[3 * a + 1], d2 = hd[3 * a + 2];
         int b = a - 1;
-        while (b >= 0 && hp[b] > kp) {
-            hp[b + 1] = hp[b];
-            hd[3 * (b + 1)] = hd[3 * b];
-            hd[3 * (b + 1) + 1] = hd[3 * b + 1];
-            hd[3 * (b + 1) + 2] = hd[3 * b + 2];
-            b--;
-        }
+        for (; b >= 0 && hp[b] > kp; b--) hp[b + 1] = hp[b];
         hp[b + 1] = kp;
-        hd[3 * (b + 1)] = d0;
-        hd[3 * (b + 1) + 1] = d1;
-        hd[3 * (b + 1) + 2] = d2;
     }
     const int keep = min(n, kTrailNum);
     int2* c = T.cache + ((size_t)T.cur * T.S + q) * kTrailNum;
@@ -2132,16 +2116,17 @@ __device__ __forceinline__ void trail_put(float* trail, size_t ij, float v, int 
 }
 
 // addTrails (MakeImageKernel.cu:98-174) for one image of one star.
-__global__ __launch_bounds__(256) void trail_lines(TrailK T, Cam7 cam, const float* grad, int W, int H) {
+__global__ __launch_bounds__(256) void trail_lines(const float* thphi, SceneK s, TrailK T, Cam7 cam, int W, int H,
+                                                   float offset, int lr, const float* area, const float* view) {
+    const float* grad = T.grad;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)T.S * kTrailHits) return;
     const int q = (int)(t / kTrailHits), slot = (int)(t % kTrailHits);
     if (slot >= (int)min(T.nhits[q], (unsigned)kTrailHits)) return;
     const size_t h = (size_t)q * kTrailHits + slot;
     const int M = W, M1 = W + 1;
-    const int i = (int)(T.hit_pix[h] / (uint32_t)W), j = (int)(T.hit_pix[h] % (uint32_t)W);
-    const float part = T.hit_data[3 * h], frac = T.hit_data[3 * h + 1];
-    const float* col = cam.colours + 6 * (int)T.hit_data[3 * h + 2];
+    const uint32_t pix = T.hit_pix[h];
+    const int i = (int)(pix / (uint32_t)W), j = (int)(pix % (uint32_t)W);
     const int prev_half = 1 - T.cur;
     const int pc = T.count[(size_t)prev_half * T.S + q];
     const int2* pcache = T.cache + ((size_t)prev_half * T.S + q) * kTrailNum;
@@ -2173,12 +2158,19 @@ __global__ __launch_bounds__(256) void trail_lines(TrailK T, Cam7 cam, const flo
         }
     }
     if (!line) return;
+    StarPix P;
+    star_pixel_geom(thphi, W, i, j, offset, cam, P);
+    star_lens(W, pix, i * M1 + j, lr, area, view, cam, P);
+    const float2 mg = reinterpret_cast<const float2*>(s.star_mag)[q];
+    const float part = mg.x + P.red;
+    const float temp = 46.f / P.redshft * ((1.f / ((0.92f * mg.y) + 1.7f)) + (1.f / ((0.92f * mg.y) + 0.62f))) - 10.f;
+    const float* col = cam.colours + 6 * max(0, min(cvt_i32(floorf(temp)), 390));
     const int deltax = i - prev.x, deltay = j - prev.y;
     const int sgnDeltaX = deltax < 0 ? -1 : 1, sgnDeltaY = deltay < 0 ? -1 : 1;
     const float deltaerr = deltay == 0 ? fabsf((float)deltax) : fabsf(deltax / (1.f * deltay));
     float error = 0.f;
     int y = prev.y, x = prev.x;
-    const float appMag = part - 2.5f * f_log10(frac);
+    const float appMag = part - 2.5f * f_log10(P.frac);
     const float bright0 = 100 * f_exp10(-.4f * appMag);
     // the reference's walk can miss (i, j) (a purely vertical move steps y
     // off the line) and then never ends; here it stops after as many steps
@@ -3300,11 +3292,12 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             KTimer t(c, "trail_images", ts);
             const TrailK& T = tf->k;
             const int span = std::max(256, few_span(NP) / 4);
-            trail_hits<<<(unsigned)((NP + span - 1) / span), 256, 0, ts>>>(thphi, s, cam, W, H, f.offset, f.lr, area,
-                                                                           v.view, T, Q.lit, span);
+            trail_hits<<<(unsigned)((NP + span - 1) / span), 256, 0, ts>>>(thphi, s, cam, W, H, f.offset, T, Q.lit,
+                                                                           span);
             trail_queued<<<(unsigned)c->num_cus * 4, 256, 0, ts>>>(thphi, s, cam, W, f.offset, T, Q);
             trail_cache<<<(unsigned)((T.S + 255) / 256), 256, 0, ts>>>(T, W);
-            trail_lines<<<(unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(T, cam, T.grad, W, H);
+            trail_lines<<<(unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(
+                thphi, s, T, cam, W, H, f.offset, f.lr, area, v.view);
         };
 #define BT_STAR_LAUNCH(S)                                                                                    \
     {                                                                                                       \

@@ -54,6 +54,42 @@ def test_sizes(ctx, world, W, H, stars, level):
     OT.close()
 
 
+def test_more_images_than_a_star_keeps(ctx):
+    """Stars with more than 32 images in a frame keep the first in pixel order,
+    as the oracle's do, in every run."""
+    W, H = 1000, 560
+    hole = bt.BlackHole(0.3296)
+    cam = bt.Camera(1.42613, 0.0, 6.5869, black_hole=hole)
+    grid = bt.Grid(8, 1, True, cam, hole, ctx=ctx)
+    stars = scene.synthetic_stars(20000, 5)
+    sky = np.zeros((16, 32, 3), np.uint8)
+    sc = bt.Scene(stars, sky, tree_level=8, ctx=ctx)
+    tree, pos, mag = O.make_tree(stars, 8)
+    T, OT = bt.Trails(sc, W, H, ctx=ctx), O.Trails(pos.shape[0], W, H, None)
+    view = bt.View(W, H, ctx=ctx)
+    oview = O.camera_view(math.pi / 2, 0.0, 0.25 * math.pi / 4, W, H)
+    gridf, table = grid.cel.astype(np.float32), O.sum_table(sky)
+    dropped, want = 0, []
+    for k in range(3):
+        off = 0.3 + k * 3.0 / W
+        print(f"frame {k}", flush=True)
+        img, st = T.render(grid, sc, view, flags=bt.RenderFlags(offset=off), stages=True)
+        _, olight, otrail = OT.frame(gridf, 8, oview, cam.getParamArray(), tree, 8, pos, mag, table, offset=off)
+        assert np.allclose(st["trail"], otrail, rtol=1e-4, atol=1e-3)
+        assert np.allclose(st["star"], olight, rtol=1e-4, atol=1e-3, equal_nan=True)
+        dropped += T.stats()["dropped"]
+        want.append((img, st["trail"]))
+    print(f"{dropped} images dropped", flush=True)
+    assert dropped > 0
+    for run in range(4):
+        T.reset()
+        for k in range(3):
+            img, st = T.render(grid, sc, view, flags=bt.RenderFlags(offset=0.3 + k * 3.0 / W), stages=True)
+            assert np.array_equal(img, want[k][0]) and np.array_equal(st["trail"], want[k][1])
+    T.close()
+    OT.close()
+
+
 def test_light_without_bound(ctx, world):
     """Stars bright enough for infinite light: what their sprite window does
     not cover keeps its light."""
