@@ -76,14 +76,14 @@ struct Blend {
 // per star, the pixels of its images in the last two frames.
 constexpr int kTrailNum = 30;    // images kept per star and frame (MakeImageKernel.cu:1255)
 constexpr int kTrailHits = 32;   // images recorded per star and frame
-constexpr uint32_t kNoPixel = 0xffffffffu;
 struct TrailK {
     int S;              // stars
     int cur;            // cache half this frame writes (the other is the previous frame's)
     int2* cache;        // [2][S][kTrailNum] (row, column)
     int* count;         // [2][S]
     unsigned* nhits;    // [S] images this frame
-    uint32_t* hit_pix;  // [S][kTrailHits] pixel index row * W + column (kNoPixel: none)
+    uint32_t* hit_pix;  // [S][kTrailHits] pixel index row * W + column
+    int2* over;         // [S * kTrailHits] star and pixel of the images beyond the slots
     float* grad;        // (H+1)(W+1) float2
     float* trail;       // W*H float3
     unsigned* stats;    // [1]: images beyond kTrailHits this frame (dropped)

@@ -1940,7 +1940,6 @@ __global__ __launch_bounds__(256) void trail_clear(TrailK T, int frame0, size_t 
         T.count[(size_t)T.cur * T.S + q] = 0;
         if (frame0) T.count[(size_t)(1 - T.cur) * T.S + q] = 0;
     }
-    for (size_t h = t; h < (size_t)T.S * kTrailHits; h += stride) T.hit_pix[h] = kNoPixel;
     for (size_t p = t; p < n3; p += stride) T.trail[p] = 0.f;
     if (t == 0) T.stats[1] = 0;
 }
@@ -1975,21 +1974,16 @@ __global__ __launch_bounds__(256) void trail_grad(const float* thphi, int W, int
 }
 
 // One image: star q of the scene in pixel pix.  The first kTrailHits images of a
-// star that are found take a slot each.  From then on (few stars have so many)
-// an image goes round the slots, leaves the lesser pixel in each and takes the
-// other on: a star keeps its first images in pixel order, whatever the order
-// they are found in.  Slots only ever fall, so one read as less or equal is
-// passed over, and what has been all the way round is no less than any of them.
+// star that are found take a slot each, the others (few stars have so many) a
+// place in the list that trail_over goes through.
 __device__ __forceinline__ void trail_record(const TrailK& T, int q, uint32_t pix) {
     const unsigned slot = atomicAdd(&T.nhits[q], 1u);
-    uint32_t* hp = T.hit_pix + (size_t)q * kTrailHits;
-    for (unsigned n = 0; n < (unsigned)kTrailHits; n++) {
-        const unsigned k = (slot + n) % kTrailHits;
-        if (slot + n >= (unsigned)kTrailHits && hp[k] <= pix) continue;
-        const uint32_t old = atomicMin(&hp[k], pix);
-        if (old == kNoPixel) return;
-        pix = max(old, pix);
+    if (slot < (unsigned)kTrailHits) {
+        T.hit_pix[(size_t)q * kTrailHits + slot] = pix;
+        return;
     }
+    const unsigned at = atomicAdd(&T.stats[1], 1u);
+    if (at < (unsigned)T.S * kTrailHits) T.over[at] = make_int2(q, (int)pix);
 }
 
 // Largest star tree (level 10), held in LDS for the walks.
@@ -2089,37 +2083,58 @@ __global__ __launch_bounds__(256) void trail_queued(const float* thphi, SceneK s
     }
 }
 
-// Per star: its images in pixel order; the first kTrailNum become this frame's
-// cache (MakeImageKernel.cu:102-104), those beyond kTrailHits are counted.
-__global__ __launch_bounds__(256) void trail_cache(TrailK T, int W) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= T.S) return;
-    const unsigned found = T.nhits[q];
-    if (found == 0) return;
-    if (found > (unsigned)kTrailHits) atomicAdd(&T.stats[1], found - (unsigned)kTrailHits);
-    const int n = (int)min(found, (unsigned)kTrailHits);
-    uint32_t* hp = T.hit_pix + (size_t)q * kTrailHits;
-    for (int a = 1; a < n; a++) {   // insertion sort (a star has a few images)
-        const uint32_t kp = hp[a];
-        int b = a - 1;
-        for (; b >= 0 && hp[b] > kp; b--) hp[b + 1] = hp[b];
-        hp[b + 1] = kp;
+// The images beyond the slots: each goes round its star's slots, leaves the
+// lesser pixel in each and takes the other on, so that a star keeps its first
+// images in pixel order, whatever the order they were found in.  Slots only
+// ever fall: one read as less or equal is passed over, and what has been all the
+// way round is no less than any of them.
+__global__ __launch_bounds__(256) void trail_over(TrailK T) {
+    const unsigned n = min(T.stats[1], (unsigned)T.S * kTrailHits);
+    for (unsigned t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) {
+        const int2 image = T.over[t];
+        uint32_t* hp = T.hit_pix + (size_t)image.x * kTrailHits;
+        uint32_t pix = (uint32_t)image.y, v[kTrailHits];
+#pragma unroll
+        for (int k = 0; k < kTrailHits; k++) v[k] = hp[k];
+#pragma unroll
+        for (int k = 0; k < kTrailHits; k++)
+            if (v[k] > pix) pix = max(pix, atomicMin(&hp[k], pix));
     }
-    const int keep = min(n, kTrailNum);
+}
+
+// Star q: its first kTrailNum images in pixel order become this frame's cache
+// (MakeImageKernel.cu:102-104).
+__device__ __forceinline__ void trail_cache(const TrailK& T, int q, int W) {
+    const int n = (int)min(T.nhits[q], (unsigned)kTrailHits);
+    if (n == 0) return;
+    const uint32_t* hp = T.hit_pix + (size_t)q * kTrailHits;
     int2* c = T.cache + ((size_t)T.cur * T.S + q) * kTrailNum;
-    for (int k = 0; k < keep; k++) c[k] = make_int2((int)(hp[k] / (uint32_t)W), (int)(hp[k] % (uint32_t)W));
-    T.count[(size_t)T.cur * T.S + q] = keep;
+    for (int k = 0; k < n; k++) {   // a star has a few images
+        const uint32_t pix = hp[k];
+        int rank = 0;
+        for (int m = 0; m < n; m++) rank += hp[m] < pix || (hp[m] == pix && m < k);
+        if (rank < kTrailNum) c[rank] = make_int2((int)(pix / (uint32_t)W), (int)(pix % (uint32_t)W));
+    }
+    T.count[(size_t)T.cur * T.S + q] = min(n, kTrailNum);
 }
 
 __device__ __forceinline__ void trail_put(float* trail, size_t ij, float v, int ch) {
     if (v >= 0.f) atomicMax(reinterpret_cast<int*>(trail) + 3 * ij + ch, __float_as_int(v));
 }
 
-// addTrails (MakeImageKernel.cu:98-174) for one image of one star.
+// addTrails (MakeImageKernel.cu:98-174) for one image of one star; the first
+// `ncache` workgroups fill this frame's half of the cache instead, which nothing
+// reads before the next frame.
 __global__ __launch_bounds__(256) void trail_lines(const float* thphi, SceneK s, TrailK T, Cam7 cam, int W, int H,
-                                                   float offset, int lr, const float* area, const float* view) {
+                                                   float offset, int lr, const float* area, const float* view,
+                                                   unsigned ncache) {
+    if (blockIdx.x < ncache) {
+        const int q = (int)(blockIdx.x * 256 + threadIdx.x);
+        if (q < T.S) trail_cache(T, q, W);
+        return;
+    }
     const float* grad = T.grad;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t t = (size_t)(blockIdx.x - ncache) * 256 + threadIdx.x;
     if (t >= (size_t)T.S * kTrailHits) return;
     const int q = (int)(t / kTrailHits), slot = (int)(t % kTrailHits);
     if (slot >= (int)min(T.nhits[q], (unsigned)kTrailHits)) return;
@@ -3295,9 +3310,10 @@ int render_frame(Context* c, const GridF& g, const SceneK& s, const ViewK& v, co
             trail_hits<<<(unsigned)((NP + span - 1) / span), 256, 0, ts>>>(thphi, s, cam, W, H, f.offset, T, Q.lit,
                                                                            span);
             trail_queued<<<(unsigned)c->num_cus * 4, 256, 0, ts>>>(thphi, s, cam, W, f.offset, T, Q);
-            trail_cache<<<(unsigned)((T.S + 255) / 256), 256, 0, ts>>>(T, W);
-            trail_lines<<<(unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(
-                thphi, s, T, cam, W, H, f.offset, f.lr, area, v.view);
+            trail_over<<<(unsigned)c->num_cus, 256, 0, ts>>>(T);
+            const unsigned ncache = (unsigned)((T.S + 255) / 256);
+            trail_lines<<<ncache + (unsigned)(((size_t)T.S * kTrailHits + 255) / 256), 256, 0, ts>>>(
+                thphi, s, T, cam, W, H, f.offset, f.lr, area, v.view, ncache);
         };
 #define BT_STAR_LAUNCH(S)                                                                                    \
     {                                                                                                       \

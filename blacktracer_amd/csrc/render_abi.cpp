@@ -623,10 +623,10 @@ int bt_trails_create(bt_context* h, const bt_scene* s, int width, int height, co
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t b_cache = up(sizeof(int2) * 2 * S * kTrailNum), b_count = up(sizeof(int) * 2 * S),
                  b_nhits = up(sizeof(unsigned) * S), b_pix = up(sizeof(uint32_t) * S * kTrailHits),
-                 b_grad = up(sizeof(float) * 2 * NC),
+                 b_over = up(sizeof(int2) * S * kTrailHits), b_grad = up(sizeof(float) * 2 * NC),
                  b_trail = up(sizeof(float) * 3 * NP), b_stats = 256,
                  b_sprite = diffraction_rgb ? up((size_t)3 * fs * fs) : 0;
-    const size_t total = b_cache + b_count + b_nhits + b_pix + b_grad + b_trail + b_stats + b_sprite;
+    const size_t total = b_cache + b_count + b_nhits + b_pix + b_over + b_grad + b_trail + b_stats + b_sprite;
     char* base = nullptr;
     if (hipMalloc((void**)&base, total) != hipSuccess) return fail(BT_ERR_NOMEM, "bt_trails_create: hipMalloc failed");
     bt_trails* t = new bt_trails;
@@ -646,6 +646,8 @@ int bt_trails_create(bt_context* h, const bt_scene* s, int width, int height, co
     off += b_nhits;
     t->k.hit_pix = (uint32_t*)(base + off);
     off += b_pix;
+    t->k.over = (int2*)(base + off);
+    off += b_over;
     t->k.grad = (float*)(base + off);
     off += b_grad;
     t->k.trail = (float*)(base + off);
