@@ -54,14 +54,16 @@ def test_sizes(ctx, world, W, H, stars, level):
     OT.close()
 
 
-def test_more_images_than_a_star_keeps(ctx):
+@pytest.mark.parametrize("a,theta,r,W,H,count,least", [
+    (0.3296, 1.42613, 6.5869, 1000, 560, 20000, 1),        # a handful beyond the slots
+    (0.3634, 2.82043, 6.8094, 1976, 1111, 54075, 10000)])  # stars with hundreds of images
+def test_more_images_than_a_star_keeps(ctx, a, theta, r, W, H, count, least):
     """Stars with more than 32 images in a frame keep the first in pixel order,
     as the oracle's do, in every run."""
-    W, H = 1000, 560
-    hole = bt.BlackHole(0.3296)
-    cam = bt.Camera(1.42613, 0.0, 6.5869, black_hole=hole)
+    hole = bt.BlackHole(a)
+    cam = bt.Camera(theta, 0.0, r, black_hole=hole)
     grid = bt.Grid(8, 1, True, cam, hole, ctx=ctx)
-    stars = scene.synthetic_stars(20000, 5)
+    stars = scene.synthetic_stars(count, 5)
     sky = np.zeros((16, 32, 3), np.uint8)
     sc = bt.Scene(stars, sky, tree_level=8, ctx=ctx)
     tree, pos, mag = O.make_tree(stars, 8)
@@ -80,7 +82,7 @@ def test_more_images_than_a_star_keeps(ctx):
         dropped += T.stats()["dropped"]
         want.append((img, st["trail"]))
     print(f"{dropped} images dropped", flush=True)
-    assert dropped > 0
+    assert dropped >= least
     for run in range(4):
         T.reset()
         for k in range(3):
