@@ -154,7 +154,7 @@ int bt_autotune(bt_context* h, const bt_pose* pose, const bt_integ_params* prm, 
             }
         }
     }
-    if (!rc) {
+    if (!rc && !(told[0] && told[1] && told[2])) {
         Tune t = best;
         if (!told[0]) t.chunk = saved.chunk;
         if (!told[1]) t.block = saved.block;
